@@ -75,7 +75,7 @@ def build_oracle(jobs: int = 8) -> None:
     oracle/_ref/libkael_ref-v{3,4}.so (test infrastructure only)."""
     make = shutil.which("make") or "make"
     _run([make, "-C", str(ORACLE), "-B", "build/liboracle.so"])
-    if REFERENCE.is_dir():
+    if (REFERENCE / "src").is_dir():
         _run([make, "-C", str(ORACLE), f"-j{jobs}", "ref"])
 
 

@@ -10,8 +10,8 @@ import support
 
 
 @pytest.fixture(scope="module")
-def cpu_kael():
-    return support.load_ref("ref")
+def cpu_kael(refdev):
+    return refdev
 
 
 CONFIGS = {"small": ((11, 16, 2, 2, 8), 31), "c4": ((96, 128, 4, 4, 256), 3), "odd": ((37, 9, 3, 3, 12), 2**40 + 7),

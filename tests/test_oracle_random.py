@@ -28,8 +28,8 @@ DT = {np.float32: kd.F32, np.float64: kd.F64}
 
 
 @pytest.fixture(scope="module")
-def cpu_kael():
-    return support.load_ref("ref")
+def cpu_kael(refdev):
+    return refdev
 
 
 def seeded(oracle, seed):

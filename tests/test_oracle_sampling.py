@@ -25,8 +25,8 @@ P = support.ptr
 
 
 @pytest.fixture(scope="module")
-def cpu_kael():
-    return support.load_ref("ref")
+def cpu_kael(refdev):
+    return refdev
 
 
 def oracle_pick(oracle, logits, temperature, top_k, u):
