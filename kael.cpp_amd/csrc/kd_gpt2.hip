@@ -1443,7 +1443,7 @@ __global__ __launch_bounds__(kThreads) void attention_kernel(const Step* st, con
 // The prompt's T positions pass each layer together: row LayerNorms, the four Linear products
 // as GEMMs on the MFMA matmul path (weights in [in, out] copies made once so that both operands
 // are row-major; prompts of up to 128 positions as split-K partial products on 64x64 tiles, longer
-// ones on the backend's matmul path with rows padded to 128), epilogue kernels for the partial
+// ones on the backend's matmul path), epilogue kernels for the partial
 // sums, the bias, residual, GELU and the K/V rows into the cache, and a causal attention kernel.
 // Same arithmetic as the decode step; only the summation order of the dot products differs.
 
@@ -1722,8 +1722,6 @@ struct Engine {
     float* pf_f = nullptr;    // [pf_rows, ff] GELU output
     float* pf_p = nullptr;    // [pf_rows, max(3d, ff)] product before its epilogue
     float* pf_parts = nullptr;  // split-K partial products of prompts of at most 128 positions
-    float* wt = nullptr;      // per layer: qkv^T [d, 3d], proj^T [d, d], fc1^T [d, ff], fc2^T [ff, d]
-    bool wt_valid = false;    // cleared by every parameter upload
 
     const float* p(const std::string& name) const { return params + offsets.at(name).first; }
 
@@ -1880,12 +1878,6 @@ struct Engine {
 
     bool stepwise_prefill() const { return (cfg.flags & KD_GPT_STEPWISE_PREFILL) != 0; }
 
-    int64_t layer_t_floats() const { return 12 * d * d; }
-    float* wt_qkv(int64_t l) const { return wt + l * layer_t_floats(); }
-    float* wt_proj(int64_t l) const { return wt_qkv(l) + 3 * d * d; }
-    float* wt_fc1(int64_t l) const { return wt_proj(l) + d * d; }
-    float* wt_fc2(int64_t l) const { return wt_fc1(l) + d * ff; }
-
     int ensure_prefill_buffers() {
         if (pf_x != nullptr) return KD_OK;
         pf_rows = (cfg.max_positions + 127) / 128 * 128;
@@ -1896,16 +1888,12 @@ struct Engine {
             *ptr = static_cast<float*>(mem);
         }
         void* mem = nullptr;
-        KD_HIP(hipMalloc(&mem, static_cast<size_t>(cfg.layers * layer_t_floats()) * sizeof(float)));
-        wt = static_cast<float*>(mem);
-        mem = nullptr;
         KD_HIP(hipMalloc(&mem, static_cast<size_t>(parts_floats()) * sizeof(float)));
         pf_parts = static_cast<float*>(mem);
         return KD_OK;
     }
 
-    // Prompts of at most kShortPrompt positions: rows padded to 64 and the products split over K
-    // into pf_parts (at most one 64x64-tile workgroup per CU, or one whole product), which the
+    // Prompts of at most kShortPrompt positions: the products split over K into pf_parts (at most one 64x64-tile workgroup per CU, or one whole product), which the
     // epilogue adds in split order.
     static constexpr int64_t kShortPrompt = 128;
     int64_t parts_floats() const {
@@ -1919,58 +1907,25 @@ struct Engine {
         int64_t stride;
     };
 
-    // dst [K, N] row-major = transpose of src [N, K] row-major (kael's Linear weight).
-    static int transpose_into(float* dst, const float* src, int64_t N, int64_t K) {
-        kd_element_layout l{};
-        l.dims = 2;
-        l.operands = 2;
-        l.count = N * K;
-        l.shape[0] = K;
-        l.shape[1] = N;
-        l.strides[0][0] = N * 4;
-        l.strides[0][1] = 4;
-        l.strides[1][0] = 4;
-        l.strides[1][1] = K * 4;
-        l.base[0] = dst;
-        l.base[1] = const_cast<float*>(src);
-        return kd_convert(KD_F32, KD_F32, &l);
-    }
-
-    int refresh_transposed() {
-        if (wt_valid) return KD_OK;
-        for (int64_t l = 0; l < cfg.layers; ++l) {
-            const std::string b = "blocks." + std::to_string(l) + ".";
-            if (int rc = transpose_into(wt_qkv(l), p(b + "attn.qkv.weight"), 3 * d, d)) return rc;
-            if (int rc = transpose_into(wt_proj(l), p(b + "attn.proj.weight"), d, d)) return rc;
-            if (int rc = transpose_into(wt_fc1(l), p(b + "mlp.fc1.weight"), ff, d)) return rc;
-            if (int rc = transpose_into(wt_fc2(l), p(b + "mlp.fc2.weight"), d, ff)) return rc;
-        }
-        wt_valid = true;
-        return KD_OK;
-    }
-
-    // A[T, K] . Wt[K, N] for the T positions of the prompt. Up to kShortPrompt positions with N a
-    // multiple of 64 and K of 32: rows padded to 64, K split so that the 64x64-tile grid holds up to
+    // A[T, K] . W[N, K]^T for the T positions of the prompt, W a Linear's weight as it is stored. Up to
+    // kShortPrompt positions with K a multiple of 32: K split so that the 64x64-tile grid holds up to
     // one workgroup per CU (GPT-2 small at T = 64: qkv 36 tiles x 6, proj 12 x 12, fc1 48 x 4,
-    // fc2 12 x 16; measured against two and four per CU and against a half and three quarters of
-    // the CUs: 0.79 ms for the 64-token prefill against 0.87, 0.94, 0.89 and 0.80), the partials
-    // left for the epilogue to add; each product reads its weights once. Otherwise the backend's matmul path on rows padded to 128. Padding rows hold leftovers
-    // of earlier rows; their products are ignored.
-    int product(const float* A, const float* Wt, int64_t T, int64_t K, int64_t N, Product* out) const {
-        const auto aligned = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
-        if (T <= kShortPrompt && N % 64 == 0 && K % 32 == 0 && aligned(A) && aligned(Wt)) {
-            const int64_t rows = (T + 63) / 64 * 64;
-            const int64_t tiles = rows / 64 * (N / 64);
+    // fc2 12 x 16), the partials left for the epilogue to add; each product reads its weights once.
+    // Otherwise the backend's matmul path.
+    int product(const float* A, const float* W, int64_t T, int64_t K, int64_t N, Product* out) const {
+        if (T <= kShortPrompt && K % 32 == 0) {
+            const int64_t tiles = (T + 63) / 64 * ((N + 63) / 64);
             const int64_t steps = K / 32;
             int64_t splits = 1;
             for (int64_t c = 1; c <= steps; ++c)
                 if (steps % c == 0 && tiles * c <= compute_units()) splits = c;
-            *out = Product{pf_parts, splits, rows * N};
-            return kd::matmul_split_parts(A, Wt, pf_parts, rows, N, K, K, N, splits);
+            *out = Product{pf_parts, splits, T * N};
+            return kd::matmul_split_parts(A, W, pf_parts, T, N, K, K, K, splits);
         }
-        kd_matmul_sizes sz{1, (T + 127) / 128 * 128, K, N};
+        const kd_matmul_sizes sz{1, T, K, N};
+        const kd_matmul_strides st{{0, K, 1}, {0, 1, K}, {0, N, 1}};
         *out = Product{pf_p, 1, 0};
-        return kd_matmul(KD_F32, A, Wt, pf_p, &sz);
+        return kd_matmul_strided(KD_F32, A, W, pf_p, &sz, &st);
     }
 
     template <int Epi>
@@ -1995,7 +1950,6 @@ struct Engine {
     // head and the greedy pick on position T - 1, which write seq[T] and leave st->pos = T.
     int batched_prefill(int64_t T) {
         if (int rc = ensure_prefill_buffers()) return rc;
-        if (int rc = refresh_transposed()) return rc;
         hipStream_t s = kd::stream();
         Product pr{};
         const float divisor = static_cast<float>(std::sqrt(static_cast<double>(hd)));
@@ -2015,17 +1969,17 @@ struct Engine {
             const bool last = l + 1 == cfg.layers;
             float* kc = kcache + l * cfg.heads * cfg.max_positions * hd;
             float* vc = vcache + l * cfg.heads * cfg.max_positions * hd;
-            if (int rc = product(pf_h, wt_qkv(l), T, d, 3 * d, &pr)) return rc;
+            if (int rc = product(pf_h, p(b + "attn.qkv.weight"), T, d, 3 * d, &pr)) return rc;
             epilogue<kQkv>(pr, p(b + "attn.qkv.bias"), pf_q, T, 3 * d, kc, vc);
             hipLaunchKernelGGL(prefill_attention_kernel, dim3(static_cast<uint32_t>(cfg.heads), static_cast<uint32_t>(T)),
                                dim3(kThreads), static_cast<size_t>(T) * sizeof(float), s, pf_q, kc, vc, pf_a, d, hd,
                                cfg.max_positions, divisor);
-            if (int rc = product(pf_a, wt_proj(l), T, d, d, &pr)) return rc;
+            if (int rc = product(pf_a, p(b + "attn.proj.weight"), T, d, d, &pr)) return rc;
             residual(p(b + "attn.proj.bias"), p(b + "ln2.weight"), p(b + "ln2.bias"));
-            if (int rc = product(pf_h, wt_fc1(l), T, d, ff, &pr)) return rc;
+            if (int rc = product(pf_h, p(b + "mlp.fc1.weight"), T, d, ff, &pr)) return rc;
             if (cfg.tanh_gelu) epilogue<kGeluTanh>(pr, p(b + "mlp.fc1.bias"), pf_f, T, ff, nullptr, nullptr);
             else epilogue<kGeluExact>(pr, p(b + "mlp.fc1.bias"), pf_f, T, ff, nullptr, nullptr);
-            if (int rc = product(pf_f, wt_fc2(l), T, ff, d, &pr)) return rc;
+            if (int rc = product(pf_f, p(b + "mlp.fc2.weight"), T, ff, d, &pr)) return rc;
             residual(p(b + "mlp.fc2.bias"), last ? nullptr : p(next + "ln1.weight"), last ? nullptr : p(next + "ln1.bias"));
             KD_LAUNCH_CHECK();
         }
@@ -2112,8 +2066,7 @@ struct Engine {
     ~Engine() {
         if (graph) (void)hipGraphExecDestroy(graph);
         for (void* ptr : {static_cast<void*>(pf_x), static_cast<void*>(pf_h), static_cast<void*>(pf_q),
-                          static_cast<void*>(pf_a), static_cast<void*>(pf_f), static_cast<void*>(pf_p), static_cast<void*>(pf_parts),
-                          static_cast<void*>(wt)})
+                          static_cast<void*>(pf_a), static_cast<void*>(pf_f), static_cast<void*>(pf_p), static_cast<void*>(pf_parts)})
             if (ptr) (void)hipFree(ptr);
         for (void* ptr : {static_cast<void*>(params), static_cast<void*>(kcache), static_cast<void*>(vcache),
                           static_cast<void*>(x), static_cast<void*>(q), static_cast<void*>(partials.m),
@@ -2234,7 +2187,6 @@ int load_parameter(const char* what, void* handle, const char* name, const float
     }
     for (size_t i = 0; i < e->names.size(); ++i)
         if (e->names[i] == name) e->loaded[i] = true;
-    e->wt_valid = false;
     return KD_OK;
 }
 

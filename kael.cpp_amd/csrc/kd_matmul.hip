@@ -6,18 +6,14 @@
 // (src/ops/linalg.cpp:72). The reference computes a 4x4 register tile per thread straight from
 // global memory (kernels.inl:136-177). Here, per shape:
 //
-//   mfma   f32, M and N large: 128x128 workgroup tiles, four waves of 64x64, each a 2x2 grid of
-//          v_mfma_f32_32x32x2f32 accumulators. K advances 16 at a time through double-buffered
-//          LDS; global loads for step k+1 are in flight while step k multiplies.
-//   small  f32, few 128x128 tiles and K <= 2048 (C1's 512^3, small MLP layers): 32x32 tiles,
-//          one workgroup of 16 waves each, the waves splitting K and reading their operands
-//          straight from global memory, their partial tiles added in LDS in wave order.
-//   skinny f32, M <= 16 (decode-shaped): lanes own 4 columns each, K is split across the
-//          workgroup's waves and, when N alone cannot fill the device, across workgroups whose
-//          partial sums land in a workspace and are added in a fixed order by a second launch.
-//   rowdot f32, N <= 4 (e.g. the GPT head computing W . x^T): one wave per output row, a
-//          coalesced dot product along K.
-//   tiled  f64 and i64: 64x64 LDS tiles, 4x4 outputs per lane (exact wrapping for i64).
+//   pieces f32, the main family: each operand as three bf16 pieces, products on the bf16 matrix
+//          cores accumulated in f32; tiles from 64x64 to 256x128 and a K split chosen by size.
+//   small  f32, few tiles and a short K (C1's 512^3, small MLP layers): 32x32 tiles, one workgroup of 16
+//          waves each, the waves splitting K and reading their operands straight from global memory,
+//          their partial tiles added in LDS in wave order.
+//   general f32 operands whose strides pieces cannot address, on the f32 matrix cores.
+//   f64    64x64 tiles on the FP64 matrix cores.
+//   tiled  i64: 64x64 LDS tiles, 4x4 outputs per lane (exact wrapping).
 //
 // Every kernel takes per-operand element strides (batch, row, column), which is how
 // kd_matmul_strided reads transposed or batch-broadcast operands in place.
@@ -62,224 +58,11 @@ __host__ __device__ __forceinline__ int64_t batch_offset(const MatmulArgs& p, in
     return o * outer + (batch - o * p.heads) * inner;
 }
 
-// Batch addressing of the kernels with 32-bit tile offsets: blockIdx.y = o * heads + h starts
-// o * a + h * ha elements into A (likewise B and the output). heads = 1 is a plain batch stride,
-// also how split K passes each split's offsets.
-struct BatchStrides {
-    int64_t a, b, o;
-    int64_t ha, hb, ho;
-    uint32_t heads;
-    const float* bias;  // the epilogue's bias (null: none; split-K partials never take it)
-};
-
-BatchStrides batch_strides(int64_t a, int64_t b, int64_t o) { return {a, b, o, 0, 0, 0, 1u, nullptr}; }
-BatchStrides batch_strides(const MatmulArgs& p) {
-    return {p.sa.b, p.sb.b, p.so.b, p.ha, p.hb, p.ho, static_cast<uint32_t>(p.heads), static_cast<const float*>(p.bias)};
-}
-
-// Offsets of this workgroup's batch (blockIdx.y) in A, B and the output.
-__device__ __forceinline__ void batch_offsets(const BatchStrides& s, int64_t& oa, int64_t& ob, int64_t& oo) {
-    const uint32_t y = blockIdx.y;
-    if (s.heads == 1) {
-        oa = y * s.a;
-        ob = y * s.b;
-        oo = y * s.o;
-        return;
-    }
-    const uint32_t o = y / s.heads;
-    const uint32_t h = y - o * s.heads;
-    oa = o * s.a + h * s.ha;
-    ob = o * s.b + h * s.hb;
-    oo = o * s.o + h * s.ho;
-}
-
 constexpr int kThreads = 256;
 
-// ---- mfma family (f32) ---------------------------------------------------------------------
-
-constexpr int kBM = 128;
-constexpr int kBN = 128;
-constexpr int kBK = 16;
-constexpr int kAld = kBK + 4;   // A tile [m][k]: row stride 20 floats, conflict-free 16-byte reads
-constexpr int kBld = kBN + 4;   // B tile [k][n]
-constexpr int kAsize = kBM * kAld;
-constexpr int kBsize = kBK * kBld;
+// ---- tile order ---------------------------------------------------------------------------------
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-
-// Operand access modes, chosen on the host.
-//   A: kRowVec = K contiguous (row-major), kColVec = M contiguous (a transposed view)
-//   B: kRowVec = N contiguous (row-major), kColVec = K contiguous (a transposed view)
-enum { kRowVec = 0, kColVec = 1, kGeneric = 2 };
-
-template <int AMode>
-__device__ __forceinline__ void load_a(float (&reg)[8], const float* a, const MatmulArgs& p, int64_t m0, int64_t k0) {
-    const int t = threadIdx.x;
-    if constexpr (AMode == kRowVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int64_t m = m0 + t / 4 + 64 * i;
-            const int64_t k = k0 + 4 * (t % 4);
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m < p.M && k < p.K) v = *reinterpret_cast<const float4*>(a + m * p.sa.r + k);
-            reg[4 * i + 0] = v.x;
-            reg[4 * i + 1] = v.y;
-            reg[4 * i + 2] = v.z;
-            reg[4 * i + 3] = v.w;
-        }
-    } else if constexpr (AMode == kColVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int64_t m = m0 + 4 * (t % 32);
-            const int64_t k = k0 + t / 32 + 8 * i;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m < p.M && k < p.K) v = *reinterpret_cast<const float4*>(a + k * p.sa.c + m);
-            reg[4 * i + 0] = v.x;
-            reg[4 * i + 1] = v.y;
-            reg[4 * i + 2] = v.z;
-            reg[4 * i + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = t + kThreads * i;
-            const int64_t m = m0 + idx / kBK;
-            const int64_t k = k0 + idx % kBK;
-            reg[i] = (m < p.M && k < p.K) ? a[m * p.sa.r + k * p.sa.c] : 0.f;
-        }
-    }
-}
-
-template <int AMode> __device__ __forceinline__ void store_a(float* As, const float (&reg)[8]) {
-    const int t = threadIdx.x;
-    if constexpr (AMode == kRowVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int row = t / 4 + 64 * i;
-            const int k = 4 * (t % 4);
-            *reinterpret_cast<float4*>(As + row * kAld + k) =
-                make_float4(reg[4 * i], reg[4 * i + 1], reg[4 * i + 2], reg[4 * i + 3]);
-        }
-    } else if constexpr (AMode == kColVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int m = 4 * (t % 32);
-            const int k = t / 32 + 8 * i;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) As[(m + e) * kAld + k] = reg[4 * i + e];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = t + kThreads * i;
-            As[(idx / kBK) * kAld + idx % kBK] = reg[i];
-        }
-    }
-}
-
-template <int BMode>
-__device__ __forceinline__ void load_b(float (&reg)[8], const float* b, const MatmulArgs& p, int64_t k0, int64_t n0) {
-    const int t = threadIdx.x;
-    if constexpr (BMode == kRowVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int64_t k = k0 + t / 32 + 8 * i;
-            const int64_t n = n0 + 4 * (t % 32);
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (k < p.K && n < p.N) v = *reinterpret_cast<const float4*>(b + k * p.sb.r + n);
-            reg[4 * i + 0] = v.x;
-            reg[4 * i + 1] = v.y;
-            reg[4 * i + 2] = v.z;
-            reg[4 * i + 3] = v.w;
-        }
-    } else if constexpr (BMode == kColVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int64_t n = n0 + t / 4 + 64 * i;
-            const int64_t k = k0 + 4 * (t % 4);
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (k < p.K && n < p.N) v = *reinterpret_cast<const float4*>(b + n * p.sb.c + k);
-            reg[4 * i + 0] = v.x;
-            reg[4 * i + 1] = v.y;
-            reg[4 * i + 2] = v.z;
-            reg[4 * i + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = t + kThreads * i;
-            const int64_t k = k0 + idx / kBN;
-            const int64_t n = n0 + idx % kBN;
-            reg[i] = (k < p.K && n < p.N) ? b[k * p.sb.r + n * p.sb.c] : 0.f;
-        }
-    }
-}
-
-template <int BMode> __device__ __forceinline__ void store_b(float* Bs, const float (&reg)[8]) {
-    const int t = threadIdx.x;
-    if constexpr (BMode == kRowVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int k = t / 32 + 8 * i;
-            const int n = 4 * (t % 32);
-            *reinterpret_cast<float4*>(Bs + k * kBld + n) =
-                make_float4(reg[4 * i], reg[4 * i + 1], reg[4 * i + 2], reg[4 * i + 3]);
-        }
-    } else if constexpr (BMode == kColVec) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int n = t / 4 + 64 * i;
-            const int k = 4 * (t % 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Bs[(k + e) * kBld + n] = reg[4 * i + e];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = t + kThreads * i;
-            Bs[(idx / kBN) * kBld + idx % kBN] = reg[i];
-        }
-    }
-}
-
-// Full tiles (M % 128 == 0, N % 128 == 0, K % 16 == 0, vector modes): each thread's two 16-byte
-// sources per operand stay fixed for the whole K loop and only a uniform offset advances, so a
-// K step issues its loads without bounds checks or 64-bit index products (the bounds-checked
-// loaders above cost ~8 % of the 4096^3 rate). Register order matches load_a / load_b.
-template <int AMode>
-__device__ __forceinline__ void a_origin(const float* a, const MatmulArgs& p, int64_t m0, const float* (&src)[2],
-                                         int64_t& step) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        if constexpr (AMode == kRowVec) src[i] = a + (m0 + t / 4 + 64 * i) * p.sa.r + 4 * (t % 4);
-        else src[i] = a + (t / 32 + 8 * i) * p.sa.c + m0 + 4 * (t % 32);
-    }
-    step = AMode == kRowVec ? kBK : kBK * p.sa.c;
-}
-
-template <int BMode>
-__device__ __forceinline__ void b_origin(const float* b, const MatmulArgs& p, int64_t n0, const float* (&src)[2],
-                                         int64_t& step) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        if constexpr (BMode == kRowVec) src[i] = b + (t / 32 + 8 * i) * p.sb.r + n0 + 4 * (t % 32);
-        else src[i] = b + (n0 + t / 4 + 64 * i) * p.sb.c + 4 * (t % 4);
-    }
-    step = BMode == kRowVec ? kBK * p.sb.r : kBK;
-}
-
-__device__ __forceinline__ void load_full(float (&reg)[8], const float* const (&src)[2], int64_t offset) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const float4 v = *reinterpret_cast<const float4*>(src[i] + offset);
-        reg[4 * i + 0] = v.x;
-        reg[4 * i + 1] = v.y;
-        reg[4 * i + 2] = v.z;
-        reg[4 * i + 3] = v.w;
-    }
-}
 
 // Maps the linear workgroup id to a (tile_m, tile_n) pair so that the workgroups that one XCD
 // runs (ids congruent mod 8 are dispatched to the same XCD) cover a compact block of tiles,
@@ -299,25 +82,361 @@ __device__ __forceinline__ void tile_of(int64_t id, int64_t tiles_m, int64_t til
     tn = in_group / rows_in_group;
 }
 
-template <int AMode, int BMode, bool Full, bool Bias = false>
-__global__ __launch_bounds__(kThreads) void mfma_f32_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                            float* __restrict__ out, MatmulArgs p) {
-    __shared__ float As[2][kAsize];
-    __shared__ float Bs[2][kBsize];
+// ---- pieces family (f32 on the bf16 matrix cores) ---------------------------------------------
+//
+// An f32 value is the exact sum of three bf16 values (8 + 8 + 8 significant bits, each piece the
+// remainder rounded to nearest), so a product of two f32 values is the sum of nine bf16 products, of
+// which the six above 2^-27 of it are taken: hi.hi on one accumulator, and lo.hi, hi.lo, mid.mid,
+// mid.hi, hi.mid on a second, both in f32 by v_mfma_f32_32x32x16_bf16, added at the end. The dropped
+// three are below half an f32 rounding of the product; what bounds the error is the rounding of the
+// running sum, and hi.hi's takes two roundings per 16 K where v_mfma_f32_32x32x2f32 takes sixteen.
+// Error against 64 bits, 2-norm, normal inputs, beside v_mfma_f32_32x32x2f32: K = 96 5.8e-8 (1.8e-7),
+// 256 8.9e-8 (2.1e-7), 2048 2.7e-7 (8.1e-7), 4096 1.9e-7 in splits (5.7e-7); of the column sums of
+// the result likewise, which the second accumulator is for: the bf16 instructions cut the low bits
+// of what they align below the accumulator towards minus infinity, and six products on one
+// accumulator leave a bias (2048: column sums 4.9e-6). bf16 has f32's exponents and the matrix cores
+// keep its subnormals, so any magnitude splits; infinities and NaN do not (inf - inf), see the end.
+//
+// The rate: 2.5 PFLOP/s / 6 = 417 TFLOP/s of f32 products against 157 on the f32 matrix cores.
+// Measured at 4096^3: 636 us (216 TFLOP/s: 1.30 PFLOP/s of bf16 products, where the vendor's bf16
+// product reaches 1.13 at this size and 1.36 at 8192^3; the clock falls to ~2.1 GHz under either)
+// against 966 us (142 TFLOP/s) on the f32 matrix cores.
+//
+// A workgroup owns a TM x TN tile and stages both operands through LDS as pieces: each 8-deep K group
+// of a row is one 16-byte unit per piece, [piece][group][row], so that a lane's MFMA operand is one
+// conflict-free 16-byte read. The split into pieces (5.5 VALU operations per element) runs between
+// the MFMAs of the step before. Global loads run two steps ahead (one step: 4096 x 256 x 768 on
+// 128 x 128 tiles 24 us, two 17). A partial K step comes first, with guarded loads; rows past M or N
+// repeat the last one and are not stored, so ragged sizes cost no tests in the loop. Element
+// alignment is all that the loads need (a global 16-byte load takes any 4-byte address).
 
-    const int64_t tiles_m = (p.M + kBM - 1) / kBM;
-    const int64_t tiles_n = (p.N + kBN - 1) / kBN;
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef float f4any __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void split_pieces(const float (&x)[8], bf8& hi, bf8& mid, bf8& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const bf2 h = __builtin_convertvector((f2v{x[e], x[e + 1]}), bf2);
+        const f2v r{x[e] - static_cast<float>(h[0]), x[e + 1] - static_cast<float>(h[1])};
+        const bf2 m = __builtin_convertvector(r, bf2);
+        const f2v q{r[0] - static_cast<float>(m[0]), r[1] - static_cast<float>(m[1])};
+        const bf2 l = __builtin_convertvector(q, bf2);
+        hi[e] = h[0];
+        hi[e + 1] = h[1];
+        mid[e] = m[0];
+        mid[e + 1] = m[1];
+        lo[e] = l[0];
+        lo[e + 1] = l[1];
+    }
+}
+
+// The LDS image of Rows (m of A, n of B) x BK of one operand. The 64 bytes after each group keep the
+// writes of a K-contiguous operand, whose neighbouring lanes hold neighbouring groups, off one
+// another's banks.
+template <int Rows, int BK> struct PieceTile {
+    static constexpr int kGroups = BK / 8;
+    static constexpr int kUnits = Rows * kGroups;
+    static constexpr int kGroup = Rows * 16 + 64;  // bytes
+    static constexpr int kPiece = kGroups * kGroup;
+    static constexpr int kBytes = 3 * kPiece;
+};
+
+// Row and group of unit `u`: neighbouring lanes along K where K is contiguous, along the rows elsewhere.
+template <bool KContig, int Rows, int BK> __device__ __forceinline__ void unit_of(int u, int& row, int& g) {
+    if constexpr (KContig) {
+        g = u % (BK / 8);
+        row = u / (BK / 8);
+    } else {
+        row = u % Rows;
+        g = u / Rows;
+    }
+}
+
+// One unit from `base` + `offset`; `ks` is the stride along K.
+template <bool KContig>
+__device__ __forceinline__ void load_unit(float (&x)[8], const float* base, int64_t offset, int64_t ks) {
+    if constexpr (KContig) {
+        const f4any v0 = *reinterpret_cast<const f4any*>(base + offset);
+        const f4any v1 = *reinterpret_cast<const f4any*>(base + offset + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[e] = v0[e];
+            x[4 + e] = v1[e];
+        }
+    } else {
+        const uint32_t off = static_cast<uint32_t>(offset);  // the host checks that it fits
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = (base + e * ks)[off];
+    }
+}
+
+// Its first `left` elements, then zeros.
+__device__ __forceinline__ void load_unit_part(float (&x)[8], const float* base, int64_t offset, int64_t ks, int left) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = e < left ? base[offset + e * ks] : 0.f;
+}
+
+// AK / BK_: K is contiguous in A / B; elsewhere any strides. WM x WN waves of (TM / WM) x (TN / WN)
+// outputs each. blockIdx.z is the K split: `k_split` deep, its partial sums `split_o` floats further
+// into `out`.
+template <bool AK, bool BKc, int TM, int TN, int WM, int WN, int BK, int Occ>
+__global__ __launch_bounds__(WM * WN * 64, Occ) void pieces_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                                   float* __restrict__ out, MatmulArgs p, int k_split,
+                                                                   int64_t split_o) {
+    constexpr int kLanes = WM * WN * 64;
+    using TA = PieceTile<TM, BK>;
+    using TB = PieceTile<TN, BK>;
+    constexpr int kUnits = TA::kUnits + TB::kUnits;
+    constexpr int kPer = (kUnits + kLanes - 1) / kLanes;
+    static_assert(TA::kUnits % 64 == 0 && TB::kUnits % 64 == 0);  // a wave's units are all of one operand
+    constexpr int IM = TM / WM / 32, JN = TN / WN / 32;
+    constexpr int kStage = TA::kBytes + TB::kBytes;
+    __shared__ __attribute__((aligned(16))) char lds[2 * kStage];
+
+    const int M = static_cast<int>(p.M), N = static_cast<int>(p.N);
     int64_t tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    const int64_t batch = blockIdx.y;
+    tile_of(blockIdx.x, (M + TM - 1) / TM, (N + TN - 1) / TN, tm, tn);
+    const int m0 = static_cast<int>(tm) * TM, n0 = static_cast<int>(tn) * TN;
+    const int64_t k_begin = static_cast<int64_t>(blockIdx.z) * k_split;
+    const int k_len = static_cast<int>(std::min<int64_t>(k_split, p.K - k_begin));
+    a += batch_offset(p, blockIdx.y, p.sa.b, p.ha) + k_begin * p.sa.c;
+    b += batch_offset(p, blockIdx.y, p.sb.b, p.hb) + k_begin * p.sb.r;
+    out += batch_offset(p, blockIdx.y, p.so.b, p.ho) + blockIdx.z * split_o;
+
+    const int t = threadIdx.x;
+    const int lane = t % 64, wave = t / 64;
+    const int wm = wave / WN, wn = wave % WN;
+    const int li = lane % 32, lh = lane / 32;
+
+    // This thread's units: element offset from the tile's corner, and LDS offset.
+    int64_t src[kPer];
+    int dst[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int u = t + kLanes * i;
+        int row, g;
+        if (u < TA::kUnits) {
+            unit_of<AK, TM, BK>(u, row, g);
+            dst[i] = g * TA::kGroup + row * 16;
+            src[i] = std::min(row, M - 1 - m0) * p.sa.r + 8 * g * p.sa.c;
+        } else {
+            unit_of<BKc, TN, BK>(u - TA::kUnits, row, g);
+            dst[i] = TA::kBytes + g * TB::kGroup + row * 16;
+            src[i] = std::min(row, N - 1 - n0) * p.sb.c + 8 * g * p.sb.r;
+        }
+    }
+    const auto has = [&](int i) {
+        return kLanes * (i + 1) <= kUnits || __builtin_amdgcn_readfirstlane(t) + kLanes * i < kUnits;
+    };
+    const auto is_a = [&](int i) {
+        if (TA::kUnits % kLanes == 0) return kLanes * i < TA::kUnits;
+        return __builtin_amdgcn_readfirstlane(t) + kLanes * i < TA::kUnits;
+    };
+    const int64_t a_step = BK * p.sa.c, b_step = BK * p.sb.r;
+    const float* at = a + m0 * p.sa.r;
+    const float* bt = b + n0 * p.sb.c;
+    typedef float Regs[kPer][8];
+    const auto fetch = [&](Regs& x) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (!has(i)) continue;
+            if (is_a(i)) load_unit<AK>(x[i], at, src[i], p.sa.c);
+            else load_unit<BKc>(x[i], bt, src[i], p.sb.r);
+        }
+    };
+    const auto fetch_part = [&](Regs& x, int whole, int left) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (!has(i)) continue;
+            int row, g;
+            if (is_a(i)) {
+                unit_of<AK, TM, BK>(t + kLanes * i, row, g);
+                load_unit_part(x[i], at + whole * a_step, src[i], p.sa.c, left - 8 * g);
+            } else {
+                unit_of<BKc, TN, BK>(t + kLanes * i - TA::kUnits, row, g);
+                load_unit_part(x[i], bt + whole * b_step, src[i], p.sb.r, left - 8 * g);
+            }
+        }
+    };
+    const auto stash = [&](const Regs& x, char* stage) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (!has(i)) continue;
+            bf8 hi, mid, lo;
+            split_pieces(x[i], hi, mid, lo);
+            const int piece = is_a(i) ? TA::kPiece : TB::kPiece;
+            char* d = stage + dst[i];
+            *reinterpret_cast<bf8*>(d) = hi;
+            *reinterpret_cast<bf8*>(d + piece) = mid;
+            *reinterpret_cast<bf8*>(d + 2 * piece) = lo;
+        }
+    };
+
+    v16f acc[IM][JN], small[IM][JN];
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = small[i][j][r] = 0.f;
+
+    // MFMA operands of lane (li, lh): row li of its block, k = 8 lh .. 8 lh + 7.
+    const int a_rd = lh * TA::kGroup + (wm * IM * 32 + li) * 16;
+    const int b_rd = TA::kBytes + lh * TB::kGroup + (wn * JN * 32 + li) * 16;
+    const auto multiply = [&](const char* stage) {
+#pragma unroll
+        for (int kk = 0; kk < BK / 16; ++kk) {
+            bf8 bf[JN][3];
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    bf[j][q] = *reinterpret_cast<const bf8*>(stage + b_rd + j * 512 + q * TB::kPiece + 2 * kk * TB::kGroup);
+            constexpr int kA[5] = {2, 0, 1, 1, 0}, kB[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+            for (int i = 0; i < IM; ++i) {
+                bf8 af[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    af[q] = *reinterpret_cast<const bf8*>(stage + a_rd + i * 512 + q * TA::kPiece + 2 * kk * TA::kGroup);
+#pragma unroll
+                for (int s = 0; s < 5; ++s)
+#pragma unroll
+                    for (int j = 0; j < JN; ++j)
+                        small[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kA[s]], bf[j][kB[s]], small[i][j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < JN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[0], bf[j][0], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    // The end of a step in which the next stage was also split and stored: its VALU work between the
+    // MFMAs, four operations after each.
+    const auto mix = [&]() {
+#pragma unroll
+        for (int q = 0; q < IM * JN * 6 * (BK / 16); ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+        }
+        __syncthreads();
+    };
+
+    const int whole = k_len / BK;
+    const int part = k_len - whole * BK;
+    int ahead = whole;  // whole steps not fetched yet
+    // The next whole step's elements; past the last one, that one again (unused).
+    const auto next = [&](Regs& x) {
+        fetch(x);
+        if (--ahead > 0) {
+            at += a_step;
+            bt += b_step;
+        }
+    };
+    Regs x0, x1;
+    if (part > 0) fetch_part(x0, whole, part);
+    else next(x0);
+    int steps = ahead;  // stages after the first
+    if (steps > 0) next(x1);
+    stash(x0, lds);
+    if (steps > 1) next(x0);
+    __syncthreads();
+    char* const s0 = lds;
+    char* const s1 = lds + kStage;
+    for (; steps > 1; steps -= 2) {
+        multiply(s0);
+        stash(x1, s1);
+        next(x1);
+        mix();
+        multiply(s1);
+        stash(x0, s0);
+        next(x0);
+        mix();
+    }
+    multiply(s0);
+    if (steps > 0) {
+        stash(x1, s1);
+        __syncthreads();
+        multiply(s1);
+    }
+
+    const int row0 = m0 + wm * IM * 32, col0 = n0 + wn * JN * 32;
+    // A sum that is not finite means an infinity or a NaN among the inputs, or an overflow. Pieces give
+    // NaN where the f32 product of an infinity is one, so the wave's outputs are computed again from
+    // the f32 operands on the f32 matrix cores. With finite inputs and sums this is never taken.
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < IM; ++i)
+#pragma unroll
+        for (int j = 0; j < JN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] += small[i][j][r];
+                odd |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+            }
+    if (__any(odd)) {
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+            for (int j = 0; j < JN; ++j) {
+                const float* ra = a + std::min(row0 + i * 32 + li, M - 1) * p.sa.r;
+                const float* rb = b + std::min(col0 + j * 32 + li, N - 1) * p.sb.c;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+                for (int k = lh; k - lh < k_len; k += 2) {
+                    const float av = k < k_len ? ra[k * p.sa.c] : 0.f;
+                    const float bv = k < k_len ? rb[k * p.sb.r] : 0.f;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[i][j], 0, 0, 0);
+                }
+            }
+    }
+    // Accumulator element r of lane (li, lh) is row 8*(r/4) + 4*lh + r%4, column li of its 32x32 block.
+#pragma unroll
+    for (int j = 0; j < JN; ++j) {
+        const int col = col0 + j * 32 + li;
+        if (col >= N) continue;
+        const float bv = p.bias != nullptr ? static_cast<const float*>(p.bias)[col] : 0.f;
+#pragma unroll
+        for (int i = 0; i < IM; ++i) {
+            const int first = row0 + i * 32 + 4 * lh;
+            float* to = out + first * p.so.r + col * p.so.c;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int up = 8 * (r / 4) + r % 4;
+                if (first + up < M) to[up * p.so.r] = p.bias != nullptr ? add_sep(acc[i][j][r], bv) : acc[i][j][r];
+            }
+        }
+    }
+}
+
+// ---- general family (f32, strides beyond 32-bit tile offsets) -----------------------------------
+
+constexpr int kBM = 128;
+constexpr int kBN = 128;
+constexpr int kBK = 16;
+constexpr int kAld = kBK + 4;   // A tile [m][k]: row stride 20 floats, conflict-free 16-byte reads
+constexpr int kBld = kBN + 4;   // B tile [k][n]
+
+// What pieces_kernel does not address (negative or very large strides): 128x128 workgroup tiles, four
+// waves of 2x2 v_mfma_f32_32x32x2f32 accumulators, K 16 at a time through double-buffered LDS, every
+// element loaded by its own 64-bit offset behind a bounds check.
+__global__ __launch_bounds__(kThreads) void general_f32_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                               float* __restrict__ out, MatmulArgs p) {
+    __shared__ float As[2][kBM * kAld];
+    __shared__ float Bs[2][kBK * kBld];
+
+    int64_t tm, tn;
+    tile_of(blockIdx.x, (p.M + kBM - 1) / kBM, (p.N + kBN - 1) / kBN, tm, tn);
     const int64_t m0 = tm * kBM;
     const int64_t n0 = tn * kBN;
-    a += batch_offset(p, batch, p.sa.b, p.ha);
-    b += batch_offset(p, batch, p.sb.b, p.hb);
-    out += batch_offset(p, batch, p.so.b, p.ho);
+    a += batch_offset(p, blockIdx.y, p.sa.b, p.ha);
+    b += batch_offset(p, blockIdx.y, p.sb.b, p.hb);
+    out += batch_offset(p, blockIdx.y, p.so.b, p.ho);
 
-    const int lane = threadIdx.x % 64;
-    const int wave = threadIdx.x / 64;
+    const int t = threadIdx.x;
+    const int lane = t % 64;
+    const int wave = t / 64;
     const int wm = wave / 2;  // wave tile row (0..1), 64 rows each
     const int wn = wave % 2;  // wave tile col (0..1), 64 cols each
     const int li = lane % 32;
@@ -332,41 +451,34 @@ __global__ __launch_bounds__(kThreads) void mfma_f32_kernel(const float* __restr
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     float ra[8], rb[8];
-    const int64_t ksteps = (p.K + kBK - 1) / kBK;
-    const float* a_src[2] = {nullptr, nullptr};
-    const float* b_src[2] = {nullptr, nullptr};
-    int64_t a_step = 0, b_step = 0;
-    if constexpr (Full) {
-        a_origin<AMode>(a, p, m0, a_src, a_step);
-        b_origin<BMode>(b, p, n0, b_src, b_step);
-        load_full(ra, a_src, 0);
-        load_full(rb, b_src, 0);
-    } else {
-        load_a<AMode>(ra, a, p, m0, 0);
-        load_b<BMode>(rb, b, p, 0, n0);
-    }
-    store_a<AMode>(As[0], ra);
-    store_b<BMode>(Bs[0], rb);
+    const auto fetch = [&](int64_t k0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int idx = t + kThreads * i;
+            const int64_t m = m0 + idx / kBK, ka = k0 + idx % kBK;
+            ra[i] = (m < p.M && ka < p.K) ? a[m * p.sa.r + ka * p.sa.c] : 0.f;
+            const int64_t kb = k0 + idx / kBN, n = n0 + idx % kBN;
+            rb[i] = (kb < p.K && n < p.N) ? b[kb * p.sb.r + n * p.sb.c] : 0.f;
+        }
+    };
+    const auto stash = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int idx = t + kThreads * i;
+            As[buf][(idx / kBK) * kAld + idx % kBK] = ra[i];
+            Bs[buf][(idx / kBN) * kBld + idx % kBN] = rb[i];
+        }
+    };
+    fetch(0);
+    stash(0);
     __syncthreads();
-
+    const int64_t ksteps = (p.K + kBK - 1) / kBK;
     for (int64_t ks = 0; ks < ksteps; ++ks) {
         const int cur = ks & 1;
         const bool more = ks + 1 < ksteps;
-        if (more) {
-            if constexpr (Full) {
-                load_full(ra, a_src, (ks + 1) * a_step);
-                load_full(rb, b_src, (ks + 1) * b_step);
-            } else {
-                load_a<AMode>(ra, a, p, m0, (ks + 1) * kBK);
-                load_b<BMode>(rb, b, p, (ks + 1) * kBK, n0);
-            }
-        }
+        if (more) fetch((ks + 1) * kBK);
         const float* as = As[cur];
         const float* bs = Bs[cur];
-        // Raised wave priority while this wave issues its MFMAs: the SIMD's arbiter then
-        // prefers waves with matrix work ready over waves issuing loads, which keeps the matrix
-        // pipe fed (measured +5 % at 4096^3).
-        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int kg = 0; kg < kBK; kg += 8) {
             // Lane (li, lh) feeds k = kg + 4*lh + s to MFMA step s (s = 0..3): the same k for
@@ -391,525 +503,22 @@ __global__ __launch_bounds__(kThreads) void mfma_f32_kernel(const float* __restr
                 }
             }
         }
-        __builtin_amdgcn_s_setprio(0);
-        if (more) {
-            store_a<AMode>(As[cur ^ 1], ra);
-            store_b<BMode>(Bs[cur ^ 1], rb);
-        }
+        if (more) stash(cur ^ 1);
         __syncthreads();
     }
 
-    // Accumulator element r of lane (li, lh) is row 8*(r/4) + 4*lh + r%4, column li of its
-    // 32x32 block.
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int64_t col = n0 + wn * 64 + j * 32 + li;
-            if (!Full && col >= p.N) continue;
-            if constexpr (Bias) {
-                const float bv = static_cast<const float*>(p.bias)[col];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = add_sep(acc[i][j][r], bv);
-            }
+            if (col >= p.N) continue;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int64_t row = m0 + wm * 64 + i * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
-                if (Full || row < p.M) out[row * p.so.r + col * p.so.c] = acc[i][j][r];
+                if (row < p.M) out[row * p.so.r + col * p.so.c] = plus_bias(acc[i][j][r], p.bias, col);
             }
         }
-}
-
-// Row-major A and B whose tiles are all full (M % 128 == 0, N % 128 == 0, K % 16 == 0) with
-// every per-batch extent below 2^31 elements: the headline and forward-pass shape. The same
-// tiles, LDS layout, MFMA order and wave priority as mfma_f32_kernel, but with 32-bit per-thread
-// offsets and leading dimensions, and the loop bound in a scalar register: on 4096^3 this runs
-// ~5 % faster than the general kernel's Full path, whose 64-bit index math and argument block
-// cost issue slots around the MFMAs. Results are bitwise those of mfma_f32_kernel.
-//
-// Split K (blockIdx.z = split): workgroup (tile, batch, split) multiplies the K slice that
-// starts split_a columns into A and split_b elements into B (K is the slice length) and writes
-// its partial product split_o floats further into the output, a workspace that
-// split_sum_kernel adds up in split order.
-__global__ __launch_bounds__(kThreads) void mfma_f32_rowmajor_kernel(const float* __restrict__ a,
-                                                                     const float* __restrict__ b,
-                                                                     float* __restrict__ out, int M, int N, int K,
-                                                                     int lda, int ldb, int ldo, int64_t batch_a,
-                                                                     int64_t batch_b, int64_t batch_o, int64_t split_a,
-                                                                     int64_t split_b, int64_t split_o) {
-    __shared__ float As[2][kAsize];
-    __shared__ float Bs[2][kBsize];
-    const int tiles_m = M / kBM;
-    const int tiles_n = N / kBN;
-    int64_t tm64, tn64;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm64, tn64);
-    const int m0 = static_cast<int>(tm64) * kBM;
-    const int n0 = static_cast<int>(tn64) * kBN;
-    a += blockIdx.y * batch_a + blockIdx.z * split_a;
-    b += blockIdx.y * batch_b + blockIdx.z * split_b;
-    out += blockIdx.y * batch_o + blockIdx.z * split_o;
-
-    const int t = threadIdx.x;
-    const int lane = t % 64;
-    const int wave = t / 64;
-    const int wm = wave / 2;
-    const int wn = wave % 2;
-    const int li = lane % 32;
-    const int lh = lane / 32;
-
-    v16f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    // Thread t moves A rows m0 + t/4 + 64i (4 floats at k = 4*(t%4)) and B rows t/32 + 8i (4
-    // floats at n = n0 + 4*(t%32)), as load_a / load_b do for the vector modes.
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    const int a_off[2] = {(m0 + t / 4) * lda + 4 * (t % 4), (m0 + t / 4 + 64) * lda + 4 * (t % 4)};
-    const int b_off[2] = {(t / 32) * ldb + n0 + 4 * (t % 32), (t / 32 + 8) * ldb + n0 + 4 * (t % 32)};
-    const int as_off[2] = {(t / 4) * kAld + 4 * (t % 4), (t / 4 + 64) * kAld + 4 * (t % 4)};
-    const int bs_off[2] = {(t / 32) * kBld + 4 * (t % 32), (t / 32 + 8) * kBld + 4 * (t % 32)};
-    f4 ra[2], rb[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        ra[i] = *reinterpret_cast<const f4*>(a + a_off[i]);
-        rb[i] = *reinterpret_cast<const f4*>(b + b_off[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        *reinterpret_cast<f4*>(&As[0][as_off[i]]) = ra[i];
-        *reinterpret_cast<f4*>(&Bs[0][bs_off[i]]) = rb[i];
-    }
-    __syncthreads();
-
-    const int ksteps = K / kBK;
-    for (int ks = 0; ks < ksteps; ++ks) {
-        const int cur = ks & 1;
-        const bool more = ks + 1 < ksteps;
-        if (more) {
-            const int ka = (ks + 1) * kBK;
-            const int kb = ka * ldb;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                ra[i] = *reinterpret_cast<const f4*>(a + a_off[i] + ka);
-                rb[i] = *reinterpret_cast<const f4*>(b + b_off[i] + kb);
-            }
-        }
-        const float* as = As[cur];
-        const float* bs = Bs[cur];
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int kg = 0; kg < kBK; kg += 8) {
-            f4 af[2];
-            float bf[2][4];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                af[i] = *reinterpret_cast<const f4*>(as + (wm * 64 + i * 32 + li) * kAld + kg + 4 * lh);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int s4 = 0; s4 < 4; ++s4) bf[j][s4] = bs[(kg + 4 * lh + s4) * kBld + wn * 64 + j * 32 + li];
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][s4], bf[j][s4], acc[i][j], 0, 0, 0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                *reinterpret_cast<f4*>(&As[cur ^ 1][as_off[i]]) = ra[i];
-                *reinterpret_cast<f4*>(&Bs[cur ^ 1][bs_off[i]]) = rb[i];
-            }
-        }
-        __syncthreads();
-    }
-
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + wn * 64 + j * 32 + li;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm * 64 + i * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
-                out[row * ldo + col] = acc[i][j][r];
-            }
-        }
-}
-
-// Whole-tile products with A and/or B read through a transposed view, 32-bit offsets: A
-// M-contiguous (AT: the weight gradient X^T . g of a Linear layer, reference
-// src/autograd/functions_linalg.cpp:44) and/or B K-contiguous (BT: the forward x . W^T,
-// src/nn/layers.cpp:43). The general kernel's transposed loaders store each 16-byte load as four
-// scalars down an LDS column (8-way bank conflicts for A). Here waves 0-1 load the A tile and
-// waves 2-3 the B tile, four 16-byte loads per thread: a transposed operand as a 4 x 4 block
-// (four consecutive rows of its contiguous dim, coalesced across lanes) that the thread writes
-// transposed as four 16-byte rows of the [m][k] / [k][n] LDS tile; a row-major operand as four
-// 16-byte rows. With AT the A tile's 16-byte column groups are XOR-swizzled by (row / 16) % 4,
-// which makes those transposed writes conflict-free; the MFMA reads apply the same swizzle. MFMA
-// order and results are those of mfma_f32_rowmajor_kernel (bit for bit). `lda` / `ldb` / `ldo`
-// are the strides between consecutive rows of the stored operands: of A's k (AT) or m rows, of
-// B's n (BT) or k rows, of the output's m rows.
-template <bool AT, bool BT, bool Bias = false, bool Deep = false>
-__global__ __launch_bounds__(kThreads) void mfma_f32_trans_kernel(const float* __restrict__ a,
-                                                                  const float* __restrict__ b,
-                                                                  float* __restrict__ out, int M, int N, int K,
-                                                                  int lda, int ldb, int ldo, BatchStrides bs) {
-    __shared__ float As[2][kAsize];
-    __shared__ float Bs[2][kBsize];
-    const int tiles_m = M / kBM;
-    const int tiles_n = N / kBN;
-    int64_t tm64, tn64;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm64, tn64);
-    const int m0 = static_cast<int>(tm64) * kBM;
-    const int n0 = static_cast<int>(tn64) * kBN;
-    {
-        int64_t oa, ob, oo;
-        batch_offsets(bs, oa, ob, oo);
-        a += oa;
-        b += ob;
-        out += oo;
-    }
-
-    const int t = threadIdx.x;
-    const int lane = t % 64;
-    const int wave = t / 64;
-    const int wm = wave / 2;
-    const int wn = wave % 2;
-    const int li = lane % 32;
-    const int lh = lane / 32;
-
-    v16f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    // Column (in floats) of 16-byte group `c4` of A tile row `row` after the swizzle.
-    const auto aswz = [](int row, int c4) { return AT ? c4 ^ (4 * ((row / 16) % 4)) : c4; };
-    const bool loads_a = t < kThreads / 2;
-    const int u = loads_a ? t : t - kThreads / 2;
-    // Per-thread source offset (element) of load j = 0..3 at K step 0, and the step per load j.
-    int g_off, g_row;
-    if (loads_a) {
-        if (AT) {  // A^T rows k = 4*(u/32) + j, columns m0 + 4*(u%32) .. +3
-            g_off = 4 * (u / 32) * lda + m0 + 4 * (u % 32);
-            g_row = lda;
-        } else {   // A rows m0 + u/4 + 32*j, columns k = 4*(u%4) .. +3
-            g_off = (m0 + u / 4) * lda + 4 * (u % 4);
-            g_row = 32 * lda;
-        }
-    } else {
-        if (BT) {  // B^T rows n0 + 4*(u/4) + j, columns k = 4*(u%4) .. +3
-            g_off = (n0 + 4 * (u / 4)) * ldb + 4 * (u % 4);
-            g_row = ldb;
-        } else {   // B rows k = 4*(u/32) + j, columns n0 + 4*(u%32) .. +3
-            g_off = 4 * (u / 32) * ldb + n0 + 4 * (u % 32);
-            g_row = ldb;
-        }
-    }
-    const int g_step = loads_a ? (AT ? kBK * lda : kBK) : (BT ? kBK : kBK * ldb);
-    const float* src = loads_a ? a : b;
-    const auto fetch = [&](f4 (&r)[4], int ks) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = *reinterpret_cast<const f4*>(src + g_off + ks * g_step + j * g_row);
-    };
-    const auto stash = [&](const f4 (&r)[4], int buf) {
-        if (loads_a) {
-            if (AT) {
-                // r[j][e] = A[m0 + 4*(u%32) + e][4*(u/32) + j]
-                const int c4 = 4 * (u / 32);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = 4 * (u % 32) + e;
-                    *reinterpret_cast<f4*>(&As[buf][row * kAld + aswz(row, c4)]) = f4{r[0][e], r[1][e], r[2][e], r[3][e]};
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(&As[buf][(u / 4 + 32 * j) * kAld + 4 * (u % 4)]) = r[j];
-            }
-        } else {
-            if (BT) {
-                // r[j][e] = B[4*(u%4) + e][n0 + 4*(u/4) + j]
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    *reinterpret_cast<f4*>(&Bs[buf][(4 * (u % 4) + e) * kBld + 4 * (u / 4)]) = f4{r[0][e], r[1][e], r[2][e], r[3][e]};
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(&Bs[buf][(4 * (u / 32) + j) * kBld + 4 * (u % 32)]) = r[j];
-            }
-        }
-    };
-    // This lane's A tile reads (rows wm*64 + i*32 + li, 16-byte groups kg + 4*lh) as LDS offsets.
-    int a_rd[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int row = wm * 64 + i * 32 + li;
-            a_rd[i][h] = row * kAld + aswz(row, 8 * h + 4 * lh);
-        }
-    const auto step = [&](int cur) {
-        const float* as = As[cur];
-        const float* bs = Bs[cur];
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int kg = 0; kg < kBK; kg += 8) {
-            f4 af[2];
-            float bf[2][4];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) af[i] = *reinterpret_cast<const f4*>(as + a_rd[i][kg / 8]);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int s4 = 0; s4 < 4; ++s4) bf[j][s4] = bs[(kg + 4 * lh + s4) * kBld + wn * 64 + j * 32 + li];
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][s4], bf[j][s4], acc[i][j], 0, 0, 0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-    };
-    const int ksteps = K / kBK;
-    if constexpr (Deep) {
-        // Grids of at most one workgroup per CU: a wave per SIMD cannot hide one step's load
-        // latency behind other waves, so the global loads run two K steps ahead (step s fetched
-        // into register set s % 2 at the start of step s - 2, written to LDS buffer s % 2 at the
-        // end of step s - 1). Same MFMA order, same results.
-        f4 r0[4], r1[4];
-        fetch(r0, 0);
-        if (ksteps > 1) fetch(r1, 1);
-        stash(r0, 0);
-        __syncthreads();
-        int ks = 0;
-        for (; ks + 1 < ksteps; ks += 2) {
-            if (ks + 2 < ksteps) fetch(r0, ks + 2);
-            step(0);
-            stash(r1, 1);
-            __syncthreads();
-            if (ks + 3 < ksteps) fetch(r1, ks + 3);
-            step(1);
-            if (ks + 2 < ksteps) stash(r0, 0);
-            __syncthreads();
-        }
-        if (ks < ksteps) step(0);  // an odd step count's last step
-    } else {
-        f4 r[4];
-        fetch(r, 0);
-        stash(r, 0);
-        __syncthreads();
-        for (int ks = 0; ks < ksteps; ++ks) {
-            const int cur = ks & 1;
-            const bool more = ks + 1 < ksteps;
-            if (more) fetch(r, ks + 1);
-            step(cur);
-            if (more) stash(r, cur ^ 1);
-            __syncthreads();
-        }
-    }
-
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + wn * 64 + j * 32 + li;
-            // the bias variant is its own instantiation: a runtime test here costs the
-            // headline kernel registers (116 -> 164 VGPRs, one wave per SIMD less)
-            const float bv = Bias ? bs.bias[col] : 0.f;
-#pragma unroll
-            for (int rr = 0; rr < 16; ++rr) {
-                const int row = m0 + wm * 64 + i * 32 + 8 * (rr / 4) + 4 * lh + (rr % 4);
-                if constexpr (Bias) out[row * ldo + col] = add_sep(acc[i][j][rr], bv);
-                else out[row * ldo + col] = acc[i][j][rr];
-            }
-        }
-}
-
-// ---- 64x64 tiles (f32, grids too small for 128x128 tiles) ---------------------------------------
-
-constexpr int kT64 = 64;
-constexpr int kT64K = 32;           // K per LDS stage
-constexpr int kT64Ald = kT64K + 4;  // A tile [m][k], row stride 36 floats
-constexpr int kT64Bld = kT64 + 4;   // B tile [k][n], row stride 68 floats
-
-// Whole 64x64 output tiles for products whose 128x128 grid would not give every CU a workgroup:
-// attention-sized batched products (128 x 128 x 64 per head), x . W^T with N = 256 over a folded
-// batch, split-K weight gradients. Four waves, each one 32x32 v_mfma_f32_32x32x2f32 accumulator of
-// the 2x2 wave grid; K advances 32 at a time through double-buffered LDS. Waves 0-1 load the A
-// tile and waves 2-3 the B tile, four 16-byte loads per thread, coalesced along each operand's
-// contiguous dim; a transposed operand (A^T: M contiguous, B^T: K contiguous) is written
-// transposed into the [m][k] / [k][n] LDS tile, A^T's 16-byte column groups XOR-swizzled by
-// (row / 4) % 8 so that those writes do not collide. Each output element accumulates K in the same
-// (k, k + 4) MFMA pairs and order as the 128x128 kernels, so without split K the results are
-// theirs bit for bit. Batches (or K splits: their offsets as batch strides) take blockIdx.y.
-// Ragged: M a multiple of 4 but not of 64 (the tied LM head's 96-row weight gradient): the last
-// tile row loads zeros past M and stores only rows below it.
-template <bool AT, bool BT, bool Ragged = false>
-__global__ __launch_bounds__(kThreads) void mfma_f32_t64_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                                float* __restrict__ out, int M, int N, int K, int lda,
-                                                                int ldb, int ldo, BatchStrides bs) {
-    __shared__ float As[2][kT64 * kT64Ald];
-    __shared__ float Bs[2][kT64K * kT64Bld];
-    const int tiles_m = (M + kT64 - 1) / kT64;
-    const int tiles_n = N / kT64;
-    int64_t tm64, tn64;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm64, tn64);
-    const int m0 = static_cast<int>(tm64) * kT64;
-    const int n0 = static_cast<int>(tn64) * kT64;
-    {
-        int64_t oa, ob, oo;
-        batch_offsets(bs, oa, ob, oo);
-        a += oa;
-        b += ob;
-        out += oo;
-    }
-
-    const int t = threadIdx.x;
-    const int lane = t % 64;
-    const int wave = t / 64;
-    const int wm = wave / 2;
-    const int wn = wave % 2;
-    const int li = lane % 32;
-    const int lh = lane / 32;
-
-    v16f acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    // Column (in floats) of 16-byte group `c4` of A tile row `row` after the swizzle.
-    const auto aswz = [](int row, int c4) { return AT ? c4 ^ (4 * ((row / 4) % 8)) : c4; };
-    const bool loads_a = t < kThreads / 2;
-    const int u = loads_a ? t : t - kThreads / 2;
-    // Per-thread source offset (element) of load j = 0..3 at K step 0, and the step per load j.
-    int g_off, g_row;
-    if (loads_a) {
-        if (AT) {  // A^T rows k = 4*(u/16) + j, columns m0 + 4*(u%16) .. +3
-            g_off = 4 * (u / 16) * lda + m0 + 4 * (u % 16);
-            g_row = lda;
-        } else {   // A rows m0 + u/8 + 16*j, columns k = 4*(u%8) .. +3
-            g_off = (m0 + u / 8) * lda + 4 * (u % 8);
-            g_row = 16 * lda;
-        }
-    } else {
-        if (BT) {  // B^T rows n0 + 4*(u/8) + j, columns k = 4*(u%8) .. +3
-            g_off = (n0 + 4 * (u / 8)) * ldb + 4 * (u % 8);
-            g_row = ldb;
-        } else {   // B rows k = 4*(u/16) + j, columns n0 + 4*(u%16) .. +3
-            g_off = 4 * (u / 16) * ldb + n0 + 4 * (u % 16);
-            g_row = ldb;
-        }
-    }
-    const int g_step = loads_a ? (AT ? kT64K * lda : kT64K) : (BT ? kT64K : kT64K * ldb);
-    const float* src = loads_a ? a : b;
-    // Ragged: whether load j of this thread stays inside A's M rows (A^T: its four columns, all in or
-    // all out as M is a multiple of 4; A: its row)
-    const auto inside = [&](int j) {
-        if constexpr (!Ragged) return true;
-        else if (!loads_a) return true;
-        else if (AT) return m0 + 4 * (u % 16) < M;
-        else return m0 + u / 8 + 16 * j < M;
-    };
-    const auto fetch = [&](f4 (&r)[4], int ks) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            r[j] = inside(j) ? *reinterpret_cast<const f4*>(src + g_off + ks * g_step + j * g_row) : f4{0.f, 0.f, 0.f, 0.f};
-    };
-    const auto stash = [&](const f4 (&r)[4], int buf) {
-        if (loads_a) {
-            if (AT) {
-                // r[j][e] = A[m0 + 4*(u%16) + e][4*(u/16) + j]
-                const int c4 = 4 * (u / 16);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = 4 * (u % 16) + e;
-                    *reinterpret_cast<f4*>(&As[buf][row * kT64Ald + aswz(row, c4)]) = f4{r[0][e], r[1][e], r[2][e], r[3][e]};
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(&As[buf][(u / 8 + 16 * j) * kT64Ald + 4 * (u % 8)]) = r[j];
-            }
-        } else {
-            if (BT) {
-                // r[j][e] = B[4*(u%8) + e][n0 + 4*(u/8) + j]
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    *reinterpret_cast<f4*>(&Bs[buf][(4 * (u % 8) + e) * kT64Bld + 4 * (u / 8)]) = f4{r[0][e], r[1][e], r[2][e], r[3][e]};
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) *reinterpret_cast<f4*>(&Bs[buf][(4 * (u / 16) + j) * kT64Bld + 4 * (u % 16)]) = r[j];
-            }
-        }
-    };
-    // This lane's A tile reads (row wm*32 + li, 16-byte groups kg + 4*lh) as LDS offsets.
-    const int arow = wm * 32 + li;
-    int a_rd[kT64K / 8];
-#pragma unroll
-    for (int h = 0; h < kT64K / 8; ++h) a_rd[h] = arow * kT64Ald + aswz(arow, 8 * h + 4 * lh);
-    const auto step = [&](int cur) {
-        const float* as = As[cur];
-        const float* bs = Bs[cur];
-#pragma unroll
-        for (int kg = 0; kg < kT64K; kg += 8) {
-            const f4 af = *reinterpret_cast<const f4*>(as + a_rd[kg / 8]);
-            float bf[4];
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) bf[s4] = bs[(kg + 4 * lh + s4) * kT64Bld + wn * 32 + li];
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[s4], bf[s4], acc, 0, 0, 0);
-        }
-    };
-    // Global loads run two K steps ahead of the MFMAs: a grid of at most a few workgroups per CU
-    // has too few waves to cover one step's load latency with the others' work. Step s is
-    // fetched into register set s % 2 at the start of step s - 2 and written to LDS buffer s % 2
-    // at the end of step s - 1.
-    const int ksteps = K / kT64K;
-    f4 r0[4], r1[4];
-    fetch(r0, 0);
-    if (ksteps > 1) fetch(r1, 1);
-    stash(r0, 0);
-    __syncthreads();
-    int ks = 0;
-    for (; ks + 1 < ksteps; ks += 2) {
-        if (ks + 2 < ksteps) fetch(r0, ks + 2);
-        step(0);
-        stash(r1, 1);
-        __syncthreads();
-        if (ks + 3 < ksteps) fetch(r1, ks + 3);
-        step(1);
-        if (ks + 2 < ksteps) stash(r0, 0);
-        __syncthreads();
-    }
-    if (ks < ksteps) step(0);  // an odd step count's last step
-
-    const int col = n0 + wn * 32 + li;
-    if (bs.bias == nullptr) {
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) {
-            const int row = m0 + wm * 32 + 8 * (rr / 4) + 4 * lh + (rr % 4);
-            if (!Ragged || row < M) out[row * ldo + col] = acc[rr];
-        }
-    } else {
-        const float bv = bs.bias[col];
-#pragma unroll
-        for (int rr = 0; rr < 16; ++rr) {
-            const int row = m0 + wm * 32 + 8 * (rr / 4) + 4 * lh + (rr % 4);
-            if (!Ragged || row < M) out[row * ldo + col] = add_sep(acc[rr], bv);
-        }
-    }
 }
 
 // ---- small family (f32, few output tiles) -----------------------------------------------------
@@ -917,16 +526,15 @@ __global__ __launch_bounds__(kThreads) void mfma_f32_t64_kernel(const float* __r
 constexpr int kSmallTile = 32;
 constexpr int kSmallWaves = 16;
 
-// Products whose 128x128 tiles would leave most CUs idle (C1's 512^3 has 16 of them) and whose K
-// is moderate: one workgroup of 16 waves per 32x32 output tile. Wave w multiplies the 8-deep K
-// groups g = w, w + 16, ... straight from global memory - lane (li, lh) reads row li of A and
-// column li of B at k = 8g + 4lh .. 8g + 4lh + 3, the operands of four v_mfma_f32_32x32x2f32
-// steps - with the next group's loads in flight during the current group's MFMAs. The 16
-// partial tiles are then added through LDS in wave order, so the result does not depend on
-// timing. One launch and no workspace, where the split-K path needs a second launch to add its
-// partial products. AVec: A is K-contiguous with 16-byte aligned rows (one 16-byte load per
-// lane and group).
-template <bool AVec>
+// Products of few output tiles and a short K (C1's 512^3, small MLP layers), where a launch and the
+// first loads are most of the time: one workgroup of 16 waves per 32x32 output tile, in one launch. Wave
+// w multiplies the 8-deep K groups g = w, w + 16, ... straight from global memory on the f32 matrix
+// cores - lane (li, lh) reads row li of A and column li of B at k = 8g + 4lh .. 8g + 4lh + 3, the
+// operands of four v_mfma_f32_32x32x2f32 steps - with the next group's loads in flight during the
+// current group's MFMAs. The 16 partial tiles are then added through LDS in wave order, so the result
+// does not depend on timing. AVec / BVec: K is contiguous in A / B (one 16-byte load per lane and group,
+// at any 4-byte address).
+template <bool AVec, bool BVec>
 __global__ __launch_bounds__(kSmallWaves * 64) void small_kernel(const float* __restrict__ a,
                                                                  const float* __restrict__ b,
                                                                  float* __restrict__ out, MatmulArgs p) {
@@ -957,15 +565,19 @@ __global__ __launch_bounds__(kSmallWaves * 64) void small_kernel(const float* __
         if (g >= groups) return;
         const int k = g * 8 + 4 * lh;
         if (AVec && k + 3 < K) {
-            if (mok) av = *reinterpret_cast<const f4*>(arow + k);
+            if (mok) av = *reinterpret_cast<const f4any*>(arow + k);
         } else {
 #pragma unroll
             for (int s = 0; s < 4; ++s)
                 if (mok && k + s < K) av[s] = arow[(k + s) * a_k];
         }
+        if (BVec && k + 3 < K) {
+            if (nok) bv = *reinterpret_cast<const f4any*>(bcol + k);
+        } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-            if (nok && k + s < K) bv[s] = bcol[(k + s) * b_k];
+            for (int s = 0; s < 4; ++s)
+                if (nok && k + s < K) bv[s] = bcol[(k + s) * b_k];
+        }
     };
     v16f acc;
 #pragma unroll
@@ -996,73 +608,7 @@ __global__ __launch_bounds__(kSmallWaves * 64) void small_kernel(const float* __
     }
 }
 
-// ---- skinny family (f32, small M) ------------------------------------------------------------
-
-constexpr int kSkinnyMaxM = 16;
-constexpr int kSkinnyCols = 256;  // 64 lanes x 4 columns
-
-// Partial sums of rows [0, M) x columns [n0, n0+256) over k in [k_begin, k_end): the four waves
-// take interleaved k, then combine in LDS in wave order. `partial` (if non-null) receives the
-// workgroup's sum for split index blockIdx.y; otherwise the result goes to `out` directly.
-template <int MT, bool BVec>
-__global__ __launch_bounds__(kThreads) void skinny_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                          float* __restrict__ out, float* __restrict__ partial,
-                                                          MatmulArgs p, int64_t k_chunk) {
-    __shared__ float red[4][MT][kSkinnyCols];
-    const int lane = threadIdx.x % 64;
-    const int wave = threadIdx.x / 64;
-    const int64_t batch = blockIdx.z;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kSkinnyCols + lane * 4;
-    const int64_t k_begin = static_cast<int64_t>(blockIdx.y) * k_chunk;
-    const int64_t k_end = std::min<int64_t>(p.K, k_begin + k_chunk);
-    a += batch_offset(p, batch, p.sa.b, p.ha);
-    b += batch_offset(p, batch, p.sb.b, p.hb);
-
-    float acc[MT][4];
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[m][c] = 0.f;
-
-    for (int64_t k = k_begin + wave; k < k_end; k += 4) {
-        float bv[4];
-        if (BVec && n0 + 3 < p.N) {
-            const float4 v = *reinterpret_cast<const float4*>(b + k * p.sb.r + n0);
-            bv[0] = v.x;
-            bv[1] = v.y;
-            bv[2] = v.z;
-            bv[3] = v.w;
-        } else {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) bv[c] = n0 + c < p.N ? b[k * p.sb.r + (n0 + c) * p.sb.c] : 0.f;
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (m < p.M) {
-                const float av = a[m * p.sa.r + k * p.sa.c];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc[m][c] += av * bv[c];
-            }
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) red[wave][m][lane * 4 + c] = acc[m][c];
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < MT * kSkinnyCols; idx += kThreads) {
-        const int m = idx / kSkinnyCols;
-        const int col = idx % kSkinnyCols;
-        const int64_t n = static_cast<int64_t>(blockIdx.x) * kSkinnyCols + col;
-        if (m >= p.M || n >= p.N) continue;
-        const float v = ((red[0][m][col] + red[1][m][col]) + red[2][m][col]) + red[3][m][col];
-        if (partial != nullptr) {
-            partial[((batch * gridDim.y + blockIdx.y) * p.M + m) * p.N + n] = v;
-        } else {
-            out[batch_offset(p, batch, p.so.b, p.ho) + m * p.so.r + n * p.so.c] = plus_bias(v, p.bias, n);
-        }
-    }
-}
+// ---- sums of split partials ---------------------------------------------------------------------
 
 // Adds the split partials in split order and writes the output.
 __global__ __launch_bounds__(kThreads) void split_sum_kernel(const float* __restrict__ partial, float* __restrict__ out,
@@ -1093,58 +639,34 @@ __global__ __launch_bounds__(kThreads) void split_sum_kernel(const float* __rest
     }
 }
 
-// ---- rowdot family (f32, small N) ---------------------------------------------------------------
-
-constexpr int kRowdotMaxN = 4;
-
-// One wave per (batch, row); lanes stride along K.
-template <bool AVec>
-__global__ __launch_bounds__(kThreads) void rowdot_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                          float* __restrict__ out, MatmulArgs p) {
-    const int lane = threadIdx.x % 64;
-    const int64_t row_id = static_cast<int64_t>(blockIdx.x) * (kThreads / 64) + threadIdx.x / 64;
-    if (row_id >= p.batches * p.M) return;
-    const int64_t batch = row_id / p.M;
-    const int64_t m = row_id % p.M;
-    const float* arow = a + batch_offset(p, batch, p.sa.b, p.ha) + m * p.sa.r;
-    const float* bb = b + batch_offset(p, batch, p.sb.b, p.hb);
-    float acc[kRowdotMaxN] = {0.f, 0.f, 0.f, 0.f};
-    if (AVec) {
-        const int64_t vecs = p.K / 4;
-        for (int64_t v = lane; v < vecs; v += 64) {
-            const float4 x = *reinterpret_cast<const float4*>(arow + 4 * v);
-            const int64_t k = 4 * v;
+// The same where the outputs are contiguous (rows of a multiple of 4, 16-byte aligned): four outputs
+// per thread and 32-bit indices. `total`, `per` (one batch's) and `n4` (a row's) are counts of four.
+__global__ __launch_bounds__(kThreads) void split_sum_flat_kernel(const float* __restrict__ partial,
+                                                                  float* __restrict__ out,
+                                                                  const float* __restrict__ bias, int total, int per,
+                                                                  int n4, int splits) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const f4* in = reinterpret_cast<const f4*>(partial);
+    for (int idx = blockIdx.x * kThreads + threadIdx.x; idx < total; idx += gridDim.x * kThreads) {
+        const int batch = per == total ? 0 : idx / per;
+        const f4* from = in + batch * splits * per + (idx - batch * per);
+        constexpr int kBatch = 8;  // in flight before the first add
+        f4 v = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = 0; s0 < splits; s0 += kBatch) {
+            f4 x[kBatch];
 #pragma unroll
-            for (int n = 0; n < kRowdotMaxN; ++n) {
-                if (n < p.N) {
-                    const float* bc = bb + n * p.sb.c;
-                    acc[n] += x.x * bc[k * p.sb.r] + x.y * bc[(k + 1) * p.sb.r] + x.z * bc[(k + 2) * p.sb.r] +
-                              x.w * bc[(k + 3) * p.sb.r];
-                }
-            }
+            for (int u = 0; u < kBatch; ++u)
+                if (s0 + u < splits) x[u] = from[(s0 + u) * per];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u)
+                if (s0 + u < splits) v += x[u];
         }
-        for (int64_t k = vecs * 4 + lane; k < p.K; k += 64) {
+        if (bias != nullptr) {
+            const f4 bv = reinterpret_cast<const f4*>(bias)[idx % n4];
 #pragma unroll
-            for (int n = 0; n < kRowdotMaxN; ++n)
-                if (n < p.N) acc[n] += arow[k] * bb[k * p.sb.r + n * p.sb.c];
+            for (int e = 0; e < 4; ++e) v[e] = add_sep(v[e], bv[e]);
         }
-    } else {
-        for (int64_t k = lane; k < p.K; k += 64) {
-            const float x = arow[k * p.sa.c];
-#pragma unroll
-            for (int n = 0; n < kRowdotMaxN; ++n)
-                if (n < p.N) acc[n] += x * bb[k * p.sb.r + n * p.sb.c];
-        }
-    }
-#pragma unroll
-    for (int n = 0; n < kRowdotMaxN; ++n) {
-#pragma unroll
-        for (int off = 32; off > 0; off /= 2) acc[n] += __shfl_xor(acc[n], off, 64);
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int n = 0; n < kRowdotMaxN; ++n)
-            if (n < p.N) out[batch_offset(p, batch, p.so.b, p.ho) + m * p.so.r + n * p.so.c] = plus_bias(acc[n], p.bias, n);
+        reinterpret_cast<f4*>(out)[idx] = v;
     }
 }
 
@@ -1223,344 +745,168 @@ int launch_status() {
     return e == hipSuccess ? KD_OK : ::kd::hip_fail(e, "kernel launch", __FILE__, __LINE__);
 }
 
-// 64x64 tiles (mfma_f32_t64_kernel) for whole-tile products (M, N multiples of 64, K of 32,
-// 32-bit offsets) whose 128x128 grid, batch included, would not give every CU a workgroup, or whose
-// M or N is not a multiple of 128 (the alternative is the bounds-checked general kernel). Measured
-// on C4's products: the attention batches (128 x 128 x 128 x 64) 6.5 us against 16.2 on the general
-// kernel, x . W^T over the folded batch with N = 256 22-29 us against 27-31 with split K. When
-// even the 64x64 grid fills at most half the CUs and K >= 512, K is split over the kernel's batch
-// slot into a workspace that split_sum_kernel adds in split order. Returns false when the product
-// does not take this path.
-template <bool AT, bool BT> bool launch_t64(const float* a, const float* b, float* out, const MatmulArgs& p, int* rc) {
+// ---- choosing the tiles of the pieces family ----------------------------------------------------
+
+// One instantiation of pieces_kernel. `alone_us` is what a 32-deep K step of one workgroup takes when
+// it has a CU to itself, `crowded_us` the CU's time per such step when `per_cu` of them share it (the
+// throughput), `end_us` the prologue and epilogue that nothing overlaps. Measured on 2^20-2^24-output
+// products with K of 256 to 50257, uniform inputs.
+struct Tiling {
+    int tm, tn, bk, per_cu;
+    double alone_us, crowded_us, end_us;
+};
+constexpr Tiling kTilings[] = {
+    {256, 128, 16, 1, 2.30, 2.48, 7.0},  // 8 waves of 64 x 64: the best rate (4096^3: 636 us; 128 x 128 below 662)
+    {128, 128, 16, 2, 1.35, 1.29, 5.0},  // two workgroups hide one another's ends (999 x 768 x 50257: 427 us; above 468)
+    {128, 128, 32, 1, 1.10, 1.37, 8.0},  // one workgroup per CU (2048^3: 94 us; 999 x 768 x 3072: 33)
+    {128, 64, 32, 2, 0.80, 0.76, 5.5},   // 1024 x 4096 x 256 in 8 splits: 21 us (128 x 128: 27)
+    {64, 64, 32, 3, 0.54, 0.44, 5.0},    // grids of a few hundred tiles (4096 x 256 x 256: 9.4 us; 128 x 128: 15)
+};
+constexpr int kTilingCount = sizeof kTilings / sizeof kTilings[0];
+
+template <bool AK, bool BKc>
+void launch_pieces(int tiling, dim3 grid, const float* a, const float* b, float* out, const MatmulArgs& p, int k_split,
+                   int64_t split_o) {
+    hipStream_t s = stream();
+    switch (tiling) {
+    case 0: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 256, 128, 4, 2, 16, 2>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
+    case 1: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 128, 128, 4, 2, 16, 4>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
+    case 2: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 128, 128, 4, 2, 32, 2>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
+    case 3: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 128, 64, 4, 2, 32, 4>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
+    default: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 64, 64, 2, 2, 32, 3>), grid, dim3(256), 0, s, a, b, out, p, k_split, split_o); break;
+    }
+}
+
+// A tiling, the number of K splits and their depth (a multiple of 32) for M x N x K, `batches` times.
+struct Plan {
+    int tiling;
+    int64_t splits, k_split;
+    double us;
+};
+
+// The cheapest by the times above: n workgroups per CU take steps * n * crowded (one alone its own
+// time), and the ends of those that run at once overlap. Splitting K adds the sum of the partials: a
+// launch and their way from memory (10 x 768 x 256: 3.9 us).
+Plan plan_pieces(int64_t M, int64_t N, int64_t K, int64_t batches) {
+    constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32, 48, 64};
+    const int64_t cus = compute_units();
+    const double outputs = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(batches);
+    Plan best{-1, 1, (K + 31) / 32 * 32, 0.0};
+    for (int c = 0; c < kTilingCount; ++c) {
+        const Tiling& tl = kTilings[c];
+        const int64_t tiles = (M + tl.tm - 1) / tl.tm * ((N + tl.tn - 1) / tl.tn) * batches;
+        int64_t last_k = 0;
+        for (const int want : kSplits) {
+            // at least 64 deep, at most four rounds of workgroups, and partials of at most 256 MiB
+            if (want > 1 && (K < want * 64 || tiles * want > 4 * cus * tl.per_cu || want * outputs > 0x1p26)) break;
+            const int64_t k_split = ((K + want - 1) / want + 31) / 32 * 32;
+            if (k_split == last_k) continue;
+            last_k = k_split;
+            const int64_t splits = want == 1 ? 1 : (K + k_split - 1) / k_split;
+            const double n = static_cast<double>((tiles * splits + cus - 1) / cus);
+            const double steps = static_cast<double>(k_split / 32);
+            double us = steps * (n > 1 ? std::max(tl.alone_us, n * tl.crowded_us) : tl.alone_us) +
+                        tl.end_us * std::ceil(n / tl.per_cu);
+            if (splits > 1) us += 2.5 + static_cast<double>(splits + 1) * outputs * 0.9e-6;
+            if (best.tiling < 0 || us < best.us) best = Plan{c, splits, k_split, us};
+        }
+    }
+    return best;
+}
+
+template <typename F> auto with_k_modes(bool ak, bool bk, F&& f) {
+    if (ak) return bk ? f(std::true_type{}, std::true_type{}) : f(std::true_type{}, std::false_type{});
+    return bk ? f(std::false_type{}, std::true_type{}) : f(std::false_type{}, std::false_type{});
+}
+
+// Enqueues split_sum_kernel over `p`'s outputs.
+int launch_split_sum(const float* partial, float* out, const MatmulArgs& p, int64_t splits) {
+    const int64_t total = p.batches * p.M * p.N;
+    const bool flat = p.heads == 1 && p.so.c == 1 && p.so.r == p.N && (p.batches == 1 || p.so.b == p.M * p.N) &&
+                      p.N % 4 == 0 && p.batches * splits * p.M * p.N < (int64_t{1} << 31) && aligned16(out) &&
+                      (p.bias == nullptr || aligned16(p.bias));
+    const int64_t items = flat ? total / 4 : total;
+    const int64_t blocks = std::min<int64_t>((items + kThreads - 1) / kThreads, int64_t{compute_units()} * 16);
+    if (flat)
+        hipLaunchKernelGGL(split_sum_flat_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, stream(), partial, out,
+                           static_cast<const float*>(p.bias), static_cast<int>(total / 4), static_cast<int>(p.M * p.N / 4),
+                           static_cast<int>(p.N / 4), static_cast<int>(splits));
+    else
+        hipLaunchKernelGGL(split_sum_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, stream(), partial, out, p,
+                           splits);
+    return launch_status();
+}
+
+// Whether pieces_kernel addresses the operands: 32-bit sizes, and for an operand whose K is not
+// contiguous offsets from its tile's corner that are not negative and fit 32 bits.
+bool pieces_addressable(const MatmulArgs& p) {
     constexpr int64_t kMax = int64_t{1} << 31;
-    const int64_t lda = AT ? p.sa.c : p.sa.r;
-    const int64_t ldb = BT ? p.sb.c : p.sb.r;
-    const int64_t a_extent = AT ? p.K * lda + p.M : p.M * lda + p.K;
-    const int64_t b_extent = BT ? p.N * ldb + p.K : p.K * ldb + p.N;
-    // a ragged last tile row (M a multiple of 4, one product): the tied LM head's 96 x 4096 x 256
-    // weight gradient, 20 us on the general kernel's split K
-    const bool ragged = p.M % kT64 != 0;
-    if ((ragged && (p.M % 4 != 0 || p.batches != 1)) || p.N % kT64 != 0 || p.K % kT64K != 0 || p.K == 0 ||
-        p.so.c != 1 || a_extent >= kMax || b_extent >= kMax || p.M * p.so.r + p.N >= kMax)
-        return false;
-    const int cus = compute_units();
-    const bool whole128 = p.M % kBM == 0 && p.N % kBN == 0 && p.K % kBK == 0;
-    // the batch folds into M when the batches share B and lie back to back in A and the output
-    const bool fold = !AT && p.heads == 1 && p.sb.b == 0 && p.sa.b == p.M * lda && p.so.b == p.M * p.so.r;
-    const int64_t rows = fold ? p.M * p.batches : p.M;
-    const int64_t batches = fold ? 1 : p.batches;
-    if (fold && (rows * lda >= kMax || rows * p.so.r >= kMax)) return false;
-    const int64_t tiles128 = (rows / kBM) * (p.N / kBN);
-    if (whole128 && tiles128 * batches >= cus) return false;
-    // One product with 5 or more 128x128 tiles splits K on them (C4's 256 x 4096 x 768 weight
-    // gradient: 28.7 us against 32.1 on 64x64 tiles split 4 ways); with at most 4 the 64x64 grid
-    // wins (256 x 4096 x 256: 13 us against 21).
-    if (whole128 && p.batches == 1 && tiles128 > 4) return false;
-    const int64_t tiles = (rows + kT64 - 1) / kT64 * (p.N / kT64);
-    if (batches > 65535) return false;
-    if (batches == 1 && tiles * 2 <= cus && p.K >= 512) {
-        int64_t splits = std::min<int64_t>(p.K / 256, (cus + tiles - 1) / tiles);
-        while (splits > 1 && p.K % (splits * kT64K) != 0) --splits;
-        const int64_t per = rows * p.N;
-        if (splits > 1 && splits * per < kMax) {
-            Workspace ws;  // held until split_sum_kernel is enqueued
-            if ((*rc = workspace(ws, static_cast<size_t>(splits * per) * sizeof(float)))) return true;
-            const int64_t kc = p.K / splits;
-            const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(splits));
-            const BatchStrides bs = batch_strides(AT ? kc * lda : kc, BT ? kc : kc * ldb, per);
-            if (ragged)
-                hipLaunchKernelGGL((mfma_f32_t64_kernel<AT, BT, true>), grid, dim3(kThreads), 0, stream(), a, b,
-                                   static_cast<float*>(ws.ptr), static_cast<int>(rows), static_cast<int>(p.N),
-                                   static_cast<int>(kc), static_cast<int>(lda), static_cast<int>(ldb),
-                                   static_cast<int>(p.N), bs);
-            else
-                hipLaunchKernelGGL((mfma_f32_t64_kernel<AT, BT>), grid, dim3(kThreads), 0, stream(), a, b,
-                                   static_cast<float*>(ws.ptr), static_cast<int>(rows), static_cast<int>(p.N),
-                                   static_cast<int>(kc), static_cast<int>(lda), static_cast<int>(ldb),
-                                   static_cast<int>(p.N), bs);
-            if ((*rc = launch_status())) return true;
-            MatmulArgs flat = p;
-            flat.batches = 1;
-            flat.M = rows;
-            const int64_t blocks = std::min<int64_t>((per + kThreads - 1) / kThreads, int64_t{cus} * 16);
-            hipLaunchKernelGGL(split_sum_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, stream(),
-                               static_cast<const float*>(ws.ptr), out, flat, splits);
-            *rc = launch_status();
-            return true;
-        }
-    }
-    const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(batches));
-    if (ragged)
-        hipLaunchKernelGGL((mfma_f32_t64_kernel<AT, BT, true>), grid, dim3(kThreads), 0, stream(), a, b, out,
-                           static_cast<int>(rows), static_cast<int>(p.N), static_cast<int>(p.K), static_cast<int>(lda),
-                           static_cast<int>(ldb), static_cast<int>(p.so.r), batch_strides(p));
-    else
-        hipLaunchKernelGGL((mfma_f32_t64_kernel<AT, BT>), grid, dim3(kThreads), 0, stream(), a, b, out,
-                           static_cast<int>(rows), static_cast<int>(p.N), static_cast<int>(p.K), static_cast<int>(lda),
-                           static_cast<int>(ldb), static_cast<int>(p.so.r), batch_strides(p));
-    *rc = launch_status();
-    return true;
+    const auto fits = [](int64_t rows, int64_t k) { return rows >= 0 && k >= 0 && rows < (kMax >> 9) && k < (kMax >> 6); };
+    return p.M < kMax - 256 && p.N < kMax - 256 && p.K < kMax - 256 && p.batches <= 65535 &&
+           (p.sa.c == 1 || fits(p.sa.r, p.sa.c)) && (p.sb.r == 1 || fits(p.sb.c, p.sb.r));
 }
 
-// mfma_f32_trans_kernel on `grid`: the instantiation that keeps two K steps of loads in flight
-// where the grid leaves at most two workgroups per CU (C4's products: 192-256 workgroups, one wave
-// per SIMD), the one-step pipeline (fewer registers, four waves per SIMD) otherwise.
-template <bool AT, bool BT, bool Bias = false>
-void launch_trans(dim3 grid, const float* a, const float* b, float* out, int64_t M, int64_t N, int64_t K, int64_t lda,
-                  int64_t ldb, int64_t ldo, const BatchStrides& bs) {
-    const int64_t groups = int64_t{grid.x} * grid.y * grid.z;
-    const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
-    const int la = static_cast<int>(lda), lb = static_cast<int>(ldb), lo = static_cast<int>(ldo);
-    if (groups <= 2 * int64_t{compute_units()})
-        hipLaunchKernelGGL((mfma_f32_trans_kernel<AT, BT, Bias, true>), grid, dim3(kThreads), 0, stream(), a, b, out, m,
-                           n, k, la, lb, lo, bs);
-    else
-        hipLaunchKernelGGL((mfma_f32_trans_kernel<AT, BT, Bias, false>), grid, dim3(kThreads), 0, stream(), a, b, out, m,
-                           n, k, la, lb, lo, bs);
-}
-
-template <int AMode, int BMode> int launch_mfma(const float* a, const float* b, float* out, const MatmulArgs& p) {
-    const int64_t tiles = ((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
-    if (p.batches > 65535) return fail(KD_E_INVALID, "kd_matmul: too many batches");
-    const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches));
-    if constexpr (AMode != kGeneric && BMode != kGeneric) {
-        int rc = KD_OK;
-        if (launch_t64<AMode == kColVec, BMode == kColVec>(a, b, out, p, &rc)) return rc;
+int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
+    // the batches fold into M when they share B and lie back to back in A and the output
+    if (p.batches > 1 && p.heads == 1 && p.sb.b == 0 && p.sa.b == p.M * p.sa.r && p.so.b == p.M * p.so.r &&
+        p.M * p.batches < (int64_t{1} << 31) - 256) {
+        p.M *= p.batches;
+        p.batches = 1;
     }
-    if constexpr (AMode == kRowVec && BMode == kRowVec) {
-        constexpr int64_t kMax = int64_t{1} << 31;
-        const bool small = p.M * p.sa.r < kMax && p.K * p.sb.r < kMax && p.M * p.so.r < kMax && p.so.c == 1;
-        if (small && p.M % kBM == 0 && p.N % kBN == 0 && p.K % kBK == 0) {
-            // Too few tiles to occupy the device (C1's 512^3 has 16): split K so that about one
-            // workgroup per CU is busy, partial products into the workspace, summed in split order.
-            const int cus = compute_units();
-            int64_t splits = 1;
-            if (p.heads == 1 && tiles * p.batches * 2 <= cus && p.K >= 256 &&
-                p.M * p.N * p.batches * (cus / tiles) < kMax) {
-                splits = std::min<int64_t>(p.K / 64, (cus + tiles * p.batches - 1) / (tiles * p.batches));
-                while (splits > 1 && p.K % (splits * kBK) != 0) --splits;
-            }
-            if (splits > 1) {
-                Workspace ws;  // held until split_sum_kernel is enqueued
-                const int64_t per = p.M * p.N;
-                if (int rc = workspace(ws, static_cast<size_t>(splits * p.batches * per) * sizeof(float))) return rc;
-                const int64_t kc = p.K / splits;
-                hipLaunchKernelGGL(mfma_f32_rowmajor_kernel,
-                                   dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches),
-                                        static_cast<uint32_t>(splits)),
-                                   dim3(kThreads), 0, stream(), a, b, static_cast<float*>(ws.ptr), static_cast<int>(p.M),
-                                   static_cast<int>(p.N), static_cast<int>(kc), static_cast<int>(p.sa.r),
-                                   static_cast<int>(p.sb.r), static_cast<int>(p.N), p.sa.b, p.sb.b, splits * per, kc,
-                                   kc * p.sb.r, per);
-                KD_LAUNCH_CHECK();
-                const int64_t total = p.batches * per;
-                const int64_t blocks = std::min<int64_t>((total + kThreads - 1) / kThreads, int64_t{cus} * 16);
-                hipLaunchKernelGGL(split_sum_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, stream(),
-                                   static_cast<const float*>(ws.ptr), out, p, splits);
-                KD_LAUNCH_CHECK();
-                return KD_OK;
-            }
-            // Whole tiles without split K: the same tiles and MFMA order on the loader of the
-            // transposed-operand family (waves 0-1 load A, waves 2-3 load B, four 16-byte loads
-            // each), which measured ~1 % faster than mfma_f32_rowmajor_kernel at 4096^3 with
-            // bit-identical results. The bounds checked above cover its 32-bit offsets.
-            if (p.bias != nullptr)
-                launch_trans<false, false, true>(grid, a, b, out, p.M, p.N, p.K, p.sa.r, p.sb.r, p.so.r, batch_strides(p));
-            else
-                launch_trans<false, false>(grid, a, b, out, p.M, p.N, p.K, p.sa.r, p.sb.r, p.so.r, batch_strides(p));
-            KD_LAUNCH_CHECK();
-            return KD_OK;
-        }
-    }
-    if constexpr ((AMode == kColVec || BMode == kColVec) && AMode != kGeneric && BMode != kGeneric) {
-        // A transposed and/or B transposed, whole tiles, 32-bit offsets: the conflict-free loaders.
-        constexpr bool at = AMode == kColVec;
-        constexpr bool bt = BMode == kColVec;
-        constexpr int64_t kMax = int64_t{1} << 31;
-        const int64_t lda = at ? p.sa.c : p.sa.r;
-        const int64_t ldb = bt ? p.sb.c : p.sb.r;
-        const int64_t a_extent = at ? p.K * lda + p.M : p.M * lda + p.K;
-        const int64_t b_extent = bt ? p.N * ldb + p.K : p.K * ldb + p.N;
-        if (a_extent < kMax && b_extent < kMax && p.M * p.so.r + p.N < kMax && p.so.c == 1 && p.M % kBM == 0 &&
-            p.N % kBN == 0 && p.K % kBK == 0) {
-            // Too few tiles to occupy the device, for one product (C4's weight gradient X^T . g:
-            // 256 x 768 outputs, 12 tiles, K = 4096) or for x . W^T over a batch with one shared
-            // weight (kael's Linear: B broadcast, A and the output batches back to back; C4's
-            // 4096 x 256 outputs have 64), whose batch folds into M: K is split, the splits
-            // taking the kernel's batch slot (their K offsets as batch strides) and writing
-            // partial products that split_sum_kernel adds in split order.
-            const int cus = compute_units();
-            const int64_t rows = p.M * p.batches;
-            const int64_t flat_tiles = (rows / kBM) * (p.N / kBN);
-            const bool fold = !at && p.heads == 1 && p.sb.b == 0 && p.sa.b == p.M * lda && p.so.b == p.M * p.so.r;
-            {
-                if ((p.batches == 1 || fold) && flat_tiles * 2 <= cus && p.K >= 256 &&
-                    (at || rows * lda < kMax) && rows * p.so.r < kMax) {
-                    int64_t splits = std::min<int64_t>(p.K / 64, (cus + flat_tiles - 1) / flat_tiles);
-                    while (splits > 1 && p.K % (splits * kBK) != 0) --splits;
-                    const int64_t per = rows * p.N;
-                    if (splits > 1 && splits * per < kMax) {
-                        Workspace ws;  // held until split_sum_kernel is enqueued
-                        if (int rc = workspace(ws, static_cast<size_t>(splits * per) * sizeof(float))) return rc;
-                        const int64_t kc = p.K / splits;
-                        launch_trans<at, bt>(dim3(static_cast<uint32_t>(flat_tiles), static_cast<uint32_t>(splits)), a, b,
-                                             static_cast<float*>(ws.ptr), rows, p.N, kc, lda, ldb, p.N,
-                                             batch_strides(at ? kc * lda : kc, bt ? kc : kc * ldb, per));
-                        KD_LAUNCH_CHECK();
-                        MatmulArgs flat = p;
-                        flat.batches = 1;
-                        flat.M = rows;
-                        const int64_t blocks = std::min<int64_t>((per + kThreads - 1) / kThreads, int64_t{cus} * 16);
-                        hipLaunchKernelGGL(split_sum_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0,
-                                           stream(), static_cast<const float*>(ws.ptr), out, flat, splits);
-                        KD_LAUNCH_CHECK();
-                        return KD_OK;
-                    }
-                }
-            }
-            if (p.bias != nullptr)
-                launch_trans<at, bt, true>(grid, a, b, out, p.M, p.N, p.K, lda, ldb, p.so.r, batch_strides(p));
-            else
-                launch_trans<at, bt>(grid, a, b, out, p.M, p.N, p.K, lda, ldb, p.so.r, batch_strides(p));
-            KD_LAUNCH_CHECK();
-            return KD_OK;
-        }
-    }
-    {
-        // Few tiles and a long K on the general kernel (a ragged M or N, any strides; C4's tied
-        // LM-head weight gradient, 96 x 256 outputs over K = 4096 tokens, is 2 tiles): K is split so
-        // that about one workgroup per CU is busy, the splits taking the kernel's batch slot (their
-        // K offsets as batch strides) and writing partial products that split_sum_kernel adds in
-        // split order, bias included.
-        const int cus = compute_units();
-        const int64_t per = p.M * p.N;
-        if (p.batches == 1 && p.heads == 1 && tiles * 2 <= cus && p.K >= 1024) {
-            int64_t splits = std::min<int64_t>(p.K / 64, cus / tiles);
-            while (splits > 1 && p.K % (splits * kBK) != 0) --splits;
-            if (splits > 1 && splits * per < (int64_t{1} << 31)) {
-                Workspace ws;  // held until split_sum_kernel is enqueued
-                if (int rc = workspace(ws, static_cast<size_t>(splits * per) * sizeof(float))) return rc;
-                MatmulArgs part = p;
-                part.batches = splits;
-                part.K = p.K / splits;
-                part.sa.b = part.K * p.sa.c;
-                part.sb.b = part.K * p.sb.r;
-                part.so = Strides3{per, p.N, 1};
-                part.bias = nullptr;
-                hipLaunchKernelGGL((mfma_f32_kernel<AMode, BMode, false>),
-                                   dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(splits)), dim3(kThreads), 0,
-                                   stream(), a, b, static_cast<float*>(ws.ptr), part);
-                KD_LAUNCH_CHECK();
-                const int64_t blocks = std::min<int64_t>((per + kThreads - 1) / kThreads, int64_t{cus} * 16);
-                hipLaunchKernelGGL(split_sum_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, stream(),
-                                   static_cast<const float*>(ws.ptr), out, p, splits);
-                KD_LAUNCH_CHECK();
-                return KD_OK;
-            }
-        }
-    }
-    bool full = false;
-    if constexpr (AMode != kGeneric && BMode != kGeneric) full = p.M % kBM == 0 && p.N % kBN == 0 && p.K % kBK == 0;
-    const bool bias = p.bias != nullptr;
-    if (full) {
-        if constexpr (AMode != kGeneric && BMode != kGeneric) {
-            if (bias) hipLaunchKernelGGL((mfma_f32_kernel<AMode, BMode, true, true>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-            else hipLaunchKernelGGL((mfma_f32_kernel<AMode, BMode, true>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-        }
-    } else {
-        if (bias) hipLaunchKernelGGL((mfma_f32_kernel<AMode, BMode, false, true>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-        else hipLaunchKernelGGL((mfma_f32_kernel<AMode, BMode, false>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-    }
-    KD_LAUNCH_CHECK();
-    return KD_OK;
-}
-
-template <int AMode> int launch_mfma_b(const float* a, const float* b, float* out, const MatmulArgs& p, int bmode) {
-    switch (bmode) {
-    case kRowVec: return launch_mfma<AMode, kRowVec>(a, b, out, p);
-    case kColVec: return launch_mfma<AMode, kColVec>(a, b, out, p);
-    default: return launch_mfma<AMode, kGeneric>(a, b, out, p);
-    }
+    const Plan plan = plan_pieces(p.M, p.N, p.K, p.batches);
+    const Tiling& tl = kTilings[plan.tiling];
+    const int64_t tiles = (p.M + tl.tm - 1) / tl.tm * ((p.N + tl.tn - 1) / tl.tn);
+    if (tiles > (int64_t{1} << 31) - 1) return fail(KD_E_INVALID, "kd_matmul: too many tiles");
+    const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches), static_cast<uint32_t>(plan.splits));
+    const auto launch = [&](float* to, const MatmulArgs& q, int64_t split_o) {
+        with_k_modes(q.sa.c == 1, q.sb.r == 1, [&](auto ak, auto bk) {
+            launch_pieces<decltype(ak)::value, decltype(bk)::value>(plan.tiling, grid, a, b, to, q,
+                                                                    static_cast<int>(plan.k_split), split_o);
+        });
+        return launch_status();
+    };
+    if (plan.splits == 1) return launch(out, p, 0);
+    Workspace ws;  // held until the sum is enqueued
+    const int64_t per = p.M * p.N;
+    if (int rc = workspace(ws, static_cast<size_t>(plan.splits * p.batches * per) * sizeof(float))) return rc;
+    MatmulArgs partial = p;
+    partial.bias = nullptr;
+    partial.ho = plan.splits * per;
+    partial.so = Strides3{p.heads * partial.ho, p.N, 1};
+    if (int rc = launch(static_cast<float*>(ws.ptr), partial, per)) return rc;
+    return launch_split_sum(static_cast<const float*>(ws.ptr), out, p, plan.splits);
 }
 
 int matmul_f32(const float* a, const float* b, float* out, const MatmulArgs& p) {
     const int cus = compute_units();
-    if (p.N <= kRowdotMaxN) {
-        const bool avec = p.sa.c == 1 && p.sa.r % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && aligned16(a);
-        const int64_t waves = p.batches * p.M;
-        const dim3 grid(static_cast<uint32_t>((waves + 3) / 4));
-        if (avec) hipLaunchKernelGGL((rowdot_kernel<true>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-        else hipLaunchKernelGGL((rowdot_kernel<false>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-        KD_LAUNCH_CHECK();
-        return KD_OK;
-    }
-    if (p.M <= kSkinnyMaxM) {
-        const bool bvec = p.sb.c == 1 && p.sb.r % 4 == 0 && p.sb.b % 4 == 0 && p.hb % 4 == 0 && aligned16(b);
-        const int64_t col_blocks = (p.N + kSkinnyCols - 1) / kSkinnyCols;
-        int64_t splits = 1;
-        const int64_t want = 2 * int64_t{cus};
-        if (col_blocks * p.batches < want) {
-            splits = std::min<int64_t>((want + col_blocks * p.batches - 1) / (col_blocks * p.batches),
-                                       std::max<int64_t>(1, p.K / 32));
-        }
-        const int64_t k_chunk = (p.K + splits - 1) / splits;
-        splits = (p.K + k_chunk - 1) / k_chunk;
-        if (splits < 1) splits = 1;
-        float* partial = nullptr;
-        Workspace ws;  // held (when split) until split_sum_kernel is enqueued
-        if (splits > 1) {
-            if (int rc = workspace(ws, static_cast<size_t>(p.batches * splits * p.M * p.N) * sizeof(float))) return rc;
-            partial = static_cast<float*>(ws.ptr);
-        }
-        if (p.batches > 65535 || splits > 65535) return fail(KD_E_INVALID, "kd_matmul: grid too large");
-        const dim3 grid(static_cast<uint32_t>(col_blocks), static_cast<uint32_t>(splits), static_cast<uint32_t>(p.batches));
-#define KD_SKINNY(MT)                                                                                               \
-    if (bvec) hipLaunchKernelGGL((skinny_kernel<MT, true>), grid, dim3(kThreads), 0, stream(), a, b, out, partial, p, k_chunk); \
-    else hipLaunchKernelGGL((skinny_kernel<MT, false>), grid, dim3(kThreads), 0, stream(), a, b, out, partial, p, k_chunk);
-        if (p.M <= 1) { KD_SKINNY(1) }
-        else if (p.M <= 4) { KD_SKINNY(4) }
-        else if (p.M <= 8) { KD_SKINNY(8) }
-        else { KD_SKINNY(16) }
-#undef KD_SKINNY
-        KD_LAUNCH_CHECK();
-        if (splits > 1) {
-            const int64_t total = p.batches * p.M * p.N;
-            const int64_t blocks = std::min<int64_t>((total + kThreads - 1) / kThreads, int64_t{cus} * 16);
-            hipLaunchKernelGGL(split_sum_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, stream(), partial,
-                               out, p, splits);
-            KD_LAUNCH_CHECK();
-        }
-        return KD_OK;
-    }
-    {
-        // Few 128x128 tiles (at most half the CUs busy) and K <= 2048: 32x32 tiles in one launch
-        // (512^3: 6.1 us against 15.6 us with split K; 64x784x128: 7.6 us against 65 us on one
-        // 128x128 tile). Longer K with few tiles stays with split K (128x4096x128: 25 us against
-        // 31 us), and so do grids of more than 2 small tiles per CU (1024^3: 32 us with split K).
-        const int64_t big = ((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN) * p.batches;
-        const int64_t gm = (p.M + kSmallTile - 1) / kSmallTile;
-        const int64_t gn = (p.N + kSmallTile - 1) / kSmallTile;
-        const bool fits32 = p.K * std::abs(p.sa.c) < (int64_t{1} << 31) && p.K * std::abs(p.sb.r) < (int64_t{1} << 31);
-        if (big * 2 <= cus && gm * gn * p.batches <= 2 * int64_t{cus} && p.K <= 2048 && fits32) {
-            if (p.batches > 65535 || gm > 65535) return fail(KD_E_INVALID, "kd_matmul: grid too large");
+    const bool pieces = pieces_addressable(p);
+    const int64_t gm = (p.M + kSmallTile - 1) / kSmallTile;
+    const int64_t gn = (p.N + kSmallTile - 1) / kSmallTile;
+    const bool fits32 = p.K * std::abs(p.sa.c) < (int64_t{1} << 31) && p.K * std::abs(p.sb.r) < (int64_t{1} << 31);
+    if (fits32 && gm <= 65535 && p.batches <= 65535 && gm * gn * p.batches <= 2 * int64_t{cus}) {
+        // Small tiles where they are estimated to be quicker than the pieces' best plan: a launch and its
+        // ends, and 0.85 us per 128 of K (16 waves of 8), 2 where a CU has two tiles. Measured, small /
+        // pieces: 512^3 6.5 / 11.4 us, 256^3 4.3 / 8.3, 128 x 64 x 784 2.9 / 6.0, 64 x 784 x 128 with B
+        // transposed 7.5 / 9.2, 600^3 10.3 / 14.5; 300 x 2000 x 300 18.3 / 14.0, 128 x 2048 x 128 17.3 /
+        // 10.7, 400 x 768 x 768 14.4 / 13.2.
+        const double rounds = static_cast<double>((p.K + 127) / 128);
+        const double us = 2.0 + rounds * (gm * gn * p.batches <= cus ? 0.85 : 2.0);
+        // (no plan takes less than 5.5 us)
+        if (!pieces || us < 5.5 || us < plan_pieces(p.M, p.N, p.K, p.batches).us) {
             const dim3 grid(static_cast<uint32_t>(gn), static_cast<uint32_t>(gm), static_cast<uint32_t>(p.batches));
-            const bool avec = p.sa.c == 1 && p.sa.r % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && aligned16(a);
-            if (avec) hipLaunchKernelGGL(small_kernel<true>, grid, dim3(kSmallWaves * 64), 0, stream(), a, b, out, p);
-            else hipLaunchKernelGGL(small_kernel<false>, grid, dim3(kSmallWaves * 64), 0, stream(), a, b, out, p);
-            KD_LAUNCH_CHECK();
-            return KD_OK;
+            with_k_modes(p.sa.c == 1, p.sb.r == 1, [&](auto ak, auto bk) {
+                hipLaunchKernelGGL((small_kernel<decltype(ak)::value, decltype(bk)::value>), grid, dim3(kSmallWaves * 64), 0,
+                                   stream(), a, b, out, p);
+            });
+            return launch_status();
         }
     }
-    int amode = kGeneric, bmode = kGeneric;
-    if (p.sa.c == 1 && p.sa.r % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && p.K % 4 == 0 && aligned16(a)) amode = kRowVec;
-    else if (p.sa.r == 1 && p.sa.c % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && p.M % 4 == 0 && aligned16(a)) amode = kColVec;
-    if (p.sb.c == 1 && p.sb.r % 4 == 0 && p.sb.b % 4 == 0 && p.hb % 4 == 0 && p.N % 4 == 0 && aligned16(b)) bmode = kRowVec;
-    else if (p.sb.r == 1 && p.sb.c % 4 == 0 && p.sb.b % 4 == 0 && p.hb % 4 == 0 && p.K % 4 == 0 && aligned16(b)) bmode = kColVec;
-    switch (amode) {
-    case kRowVec: return launch_mfma_b<kRowVec>(a, b, out, p, bmode);
-    case kColVec: return launch_mfma_b<kColVec>(a, b, out, p, bmode);
-    default: return launch_mfma_b<kGeneric>(a, b, out, p, bmode);
-    }
+    if (pieces) return matmul_pieces(a, b, out, p);
+    const int64_t tiles = ((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
+    if (p.batches > 65535) return fail(KD_E_INVALID, "kd_matmul: too many batches");
+    hipLaunchKernelGGL(general_f32_kernel, dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches)), dim3(kThreads),
+                       0, stream(), a, b, out, p);
+    return launch_status();
 }
 
 // ---- f64 on the FP64 matrix cores ------------------------------------------------------------
@@ -1729,16 +1075,20 @@ int dispatch(int dtype, const void* a, const void* b, void* out, const MatmulArg
 int matmul_split_parts(const float* a, const float* b, float* parts, int64_t M, int64_t N, int64_t K, int64_t lda,
                        int64_t ldb, int64_t splits) {
     constexpr int64_t kMax = int64_t{1} << 31;
-    if (M <= 0 || N <= 0 || splits < 1 || M % kT64 != 0 || N % kT64 != 0 || K % (kT64K * splits) != 0 || lda % 4 != 0 ||
-        ldb % 4 != 0 || !aligned16(a) || !aligned16(b) || !aligned16(parts) || M * lda >= kMax || K * ldb >= kMax ||
-        splits * M * N >= kMax || splits > 65535)
-        return fail(KD_E_INVALID, "matmul_split_parts: operands outside the 64x64 split-K kernel's bounds");
-    const int64_t tiles = (M / kT64) * (N / kT64);
-    const int64_t kc = K / splits;
-    hipLaunchKernelGGL((mfma_f32_t64_kernel<false, false>), dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(splits)),
-                       dim3(kThreads), 0, stream(), a, b, parts, static_cast<int>(M), static_cast<int>(N),
-                       static_cast<int>(kc), static_cast<int>(lda), static_cast<int>(ldb), static_cast<int>(N),
-                       batch_strides(kc, kc * ldb, M * N));
+    if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || splits > 65535 || K % (32 * splits) != 0 || splits * M * N >= kMax ||
+        K >= kMax - 256)
+        return fail(KD_E_INVALID, "matmul_split_parts: operands outside the split-K kernel's bounds");
+    MatmulArgs p;
+    p.batches = 1;
+    p.M = M;
+    p.K = K;
+    p.N = N;
+    p.sa = {0, lda, 1};
+    p.sb = {0, 1, ldb};
+    p.so = {0, N, 1};
+    const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64);
+    launch_pieces<true, true>(kTilingCount - 1, dim3(static_cast<uint32_t>(tiles), 1, static_cast<uint32_t>(splits)), a, b, parts,
+                              p, static_cast<int>(K / splits), M * N);
     return launch_status();
 }
 

@@ -1,0 +1,133 @@
+"""f32 products on the bf16 matrix cores (kd_matmul.hip's pieces family) at the edges of its tiles,
+K steps and splits, against the float64 product of the same f32 operands.
+
+Tolerance per element, from the arithmetic: every product keeps six of the nine products of the
+operands' pieces (the dropped three are below 3 * 2^-27 of it), and the running sums round at most
+twice per 8 of K and once per split; each rounding is at most 2^-24 of a partial sum, which is at most
+sum |a||b|. The same bound covers the small tiles and the general kernel (one rounding per K).
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import kd
+
+pytestmark = pytest.mark.gpu
+
+
+def product(kdb, a_store, b_store, sizes, sa, sb, out_strides=None, bias=None, out_len=None):
+    batches, m, k, n = sizes
+    so = out_strides or (m * n, n, 1)
+    da, db = kdb.to_device(a_store), kdb.to_device(b_store)
+    out = kdb.to_device(np.full(out_len or batches * m * n, np.nan, np.float32))
+    args = (kd.F32, da.ptr, db.ptr, out.ptr, kd.MatmulSizes(*sizes), kd.MatmulStrides(sa, sb, so))
+    if bias is None:
+        kdb.call("matmul_strided", *args)
+    else:
+        kdb.call("matmul_strided_bias", *args, kdb.to_device(bias).ptr)
+    return out.numpy()
+
+
+def check(got, a, b, bias=None):
+    """a [.., m, k] and b [.., k, n] as the call sees them."""
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    want, size, k = a @ b, np.abs(a) @ np.abs(b), a.shape[-1]
+    if bias is not None:
+        want, size = want + bias, size + np.abs(bias)
+    err = np.abs(got.reshape(want.shape) - want)
+    assert (err <= (k + 72) * 2.0 ** -24 * size).all(), (err / size).max() * 2 ** 24
+
+
+# (m, k, n): around the tiles of 64, 128 and 256 and the K steps of 16 and 32, one short K step, long K
+# in splits with a ragged last one, and outputs large enough for each of the tilings
+SIZES = [(63, 700, 65), (65, 1001, 63), (128, 999, 129), (127, 640, 200), (17, 4099, 5), (1, 2000, 70), (200, 3000, 1),
+         (700, 33, 900), (1000, 15, 1030), (999, 768, 770), (2049, 47, 2050), (4100, 40, 4000), (300, 5003, 260)]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("m,k,n", SIZES, ids=lambda v: str(v))
+def test_ragged_products(kdb, m, k, n, layout):
+    rng = np.random.default_rng(m + 7 * k + 31 * n)
+    a, b = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
+    at, bt = layout[0] == "t", layout[1] == "t"
+    bias = rng.normal(size=n).astype(np.float32) if layout == "nt" else None
+    got = product(kdb, a.T.copy() if at else a, b.T.copy() if bt else b, (1, m, k, n), (0, 1, m) if at else (0, k, 1),
+                  (0, 1, k) if bt else (0, n, 1), bias=bias)
+    check(got, a, b, bias)
+
+
+def test_magnitudes_that_one_bf16_cannot_hold(kdb):
+    """Operands whose low pieces are subnormal, and rows of very different sizes."""
+    rng = np.random.default_rng(3)
+    a, b = rng.normal(size=(130, 800)).astype(np.float32), rng.normal(size=(800, 90)).astype(np.float32)
+    a *= (10.0 ** rng.integers(-36, 30, (130, 1))).astype(np.float32)
+    b *= np.float32(1e-2)
+    check(product(kdb, a, b, (1, 130, 800, 90), (0, 800, 1), (0, 90, 1)), a, b)
+
+
+@pytest.mark.parametrize("k", [48, 3000])
+def test_infinities_and_nan_as_an_f32_product_has_them(kdb, k):
+    rng = np.random.default_rng(k)
+    m, n = 300, 520
+    a, b = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
+    # 3.4e38 rounds to infinity in bf16; its neighbours are small, so that no f32 product overflows but one
+    a[:, k - 2] *= np.float32(0.1)
+    b[k - 2] *= np.float32(0.1)
+    a[5, 3], a[40, k - 1], a[70, 0], a[200, k - 2] = np.inf, -np.inf, np.nan, 3.4e38
+    b[7, 130], b[k - 2, 519] = np.inf, 3.4e38
+    with np.errstate(all="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    got = product(kdb, a, b, (1, m, k, n), (0, k, 1), (0, n, 1)).reshape(m, n)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    plain = np.isfinite(want)
+    with np.errstate(all="ignore"):
+        size = np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64))
+    err = np.abs(got[plain].astype(np.float64) - want[plain])
+    assert (err <= (k + 72) * 2.0 ** -24 * size[plain]).all()
+
+
+@pytest.mark.parametrize("case", ["steps", "broadcast", "reversed", "output", "unaligned"])
+def test_strides_that_are_no_plain_matrix(kdb, case):
+    """Both strides of an operand above 1, rows that repeat, negative strides (the general kernel), an
+    output of strided columns, and operands that start and step at odd elements."""
+    rng = np.random.default_rng(11)
+    m, k, n = 150, 900, 140
+    store = rng.normal(size=2_000_000).astype(np.float32)
+    b = rng.normal(size=(k, n)).astype(np.float32)
+    sa, so, out_len, start = (0, k, 1), (0, n, 1), m * n, 0
+    if case == "steps":
+        sa = (0, 2 * k + 1, 2)
+    elif case == "broadcast":
+        sa = (0, 0, 3)
+    elif case == "reversed":
+        sa, start = (0, -k, -1), m * k - 1
+    elif case == "output":
+        so, out_len = (0, 3 * n, 3), 3 * m * n
+    else:
+        sa, start = (0, k + 3, 1), 1
+    index = start + np.arange(m)[:, None] * sa[1] + np.arange(k)[None] * sa[2]
+    da, db = kdb.to_device(store), kdb.to_device(b)
+    out = kdb.to_device(np.zeros(out_len, np.float32))
+    kdb.call("matmul_strided", kd.F32, ctypes.c_void_p(da.ptr + 4 * start), db.ptr, out.ptr, kd.MatmulSizes(1, m, k, n),
+             kd.MatmulStrides(sa, (0, n, 1), so))
+    got = out.numpy()
+    if case == "output":
+        assert (got.reshape(m, n, 3)[:, :, 1:] == 0).all()
+        got = got.reshape(m, n, 3)[:, :, 0]
+    check(got, store[index], b)
+
+
+def test_split_batches_of_heads(kdb):
+    """A two-level batch whose K is split: partial sums by batch and head."""
+    rng = np.random.default_rng(12)
+    outer, heads, m, k, n = 2, 3, 70, 2100, 66
+    a, b = (rng.normal(size=(outer, heads, *s)).astype(np.float32) for s in ((m, k), (k, n)))
+    da, db = kdb.to_device(a), kdb.to_device(b)
+    out = kdb.empty((outer, heads, m, n), np.float32)
+    sizes = kd.MatmulSizes(outer * heads, m, k, n)
+    strides = kd.MatmulStrides((heads * m * k, k, 1), (heads * k * n, n, 1), (heads * m * n, n, 1))
+    kdb.call("matmul_strided_heads", kd.F32, da.ptr, db.ptr, out.ptr, sizes, strides,
+             kd.MatmulHeads(heads, m * k, k * n, m * n))
+    check(out.numpy(), a, b)
