@@ -709,8 +709,10 @@ struct alignas(16) PickShared {  // hist rows are read 16 bytes at a time
     uint32_t appended;                                // keys appended to the unordered short list
     uint32_t nparts;                                  // head workgroups that may hold candidates
     int32_t cand_parts[kPickParts];
-    float kept_e[kPickLdsKept];       // kept entries, when at most kPickLdsKept
+    alignas(16) float kept_e[kPickLdsKept];  // kept entries, when at most kPickLdsKept
     int32_t kept_i[kPickLdsKept];
+    double sums[kPickWaves];          // per wave: sums of e, then of p
+    uint32_t first_past;              // parallel_pick: 2 * position + 1 where it is not certain
 };
 
 // Inclusive prefix sum of v over the workgroup's first `n` lanes (n a multiple of 64, at most
@@ -858,6 +860,90 @@ __device__ __forceinline__ int64_t ordered_compact(uint64_t mine, const Emit& em
     return total;
 }
 
+// The lane's share of the m kept entries: positions first .. first + 4 * kShare4 - 1, in index order.
+constexpr int kShare4 = kPickSlots / 4;
+typedef float f4pick __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ int share_of(int m) { return ((m + kPickThreads - 1) / kPickThreads + 3) / 4 * 4; }
+
+// The multinomial pick over m > 64 kept exponentials e (the lane's share in `e`, zeros past the list) by
+// the whole workgroup, where its position is certain to be the one that the sums in index order give;
+// -1 where it is not, and the caller folds them in order.
+//
+// kael adds the exponentials and then the weights p one by one in double: a chain of 2 m additions. Any
+// order of m positive terms is within m 2^-53 of their exact sum, relatively, so sums taken in parallel
+// are within m 2^-52 of kael's; `slack` doubles that. The f32 denominator is kael's when both ends of
+// the interval round to it, and a position is kael's when its running sum is past every possible point
+// and the one before it is past none: an f32 boundary falls within the interval in about 2 of 10^4 draws
+// at m = 50257, a running sum in 2 of 10^6. One wave took 965 us for GPT-2's vocabulary, of which the
+// dependent additions were 950; see pick_kernel for the time now.
+__device__ __forceinline__ int32_t parallel_pick(f4pick (&e)[kShare4], int m, double u, PickShared& sh) {
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const int share = share_of(m), first = tid * share;
+    const double slack = static_cast<double>(m) * 0x1p-51;
+    const auto lane_sum = [&]() {
+        double s = 0.0;
+#pragma unroll
+        for (int g = 0; g < kShare4; ++g)
+            if (4 * g < share)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s += static_cast<double>(e[g][c]);
+        return s;
+    };
+    double mine = wave_sum(lane_sum());
+    if (lane == 0) sh.sums[wave] = mine;
+    if (tid == 0) sh.first_past = ~0u;
+    __syncthreads();
+    double total = 0.0;
+    for (int w = 0; w < kPickWaves; ++w) total += sh.sums[w];
+    const float denominator = static_cast<float>(total - slack * total);
+    if (denominator != static_cast<float>(total + slack * total)) return -1;  // the same for every lane
+#pragma unroll
+    for (int g = 0; g < kShare4; ++g)
+        if (4 * g < share)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) e[g][c] = __fdiv_rn(e[g][c], denominator);
+    mine = lane_sum();
+    double through = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(through, off);
+        if (lane >= off) through += o;
+    }
+    double run = __shfl_up(through, 1);
+    if (lane == 0) run = 0.0;
+    __syncthreads();  // the first sums are read
+    if (lane == 63) sh.sums[wave] = through;
+    __syncthreads();
+    total = 0.0;
+    double before = 0.0;
+    for (int w = 0; w < kPickWaves; ++w) {
+        if (w == wave) before = total;
+        total += sh.sums[w];
+    }
+    run += before;
+    const double width = slack * total;
+    const double low = u * (total - width), high = u * (total + width);
+    if (run + mine + width >= low) {
+        bool found = false;
+#pragma unroll
+        for (int g = 0; g < kShare4; ++g)
+            if (4 * g < share && !found)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    run += static_cast<double>(e[g][c]);
+                    const int at = first + 4 * g + c;
+                    if (!found && at < m && run + width >= low) {
+                        found = true;
+                        atomicMin(&sh.first_past, 2u * at + (run - width > high ? 0u : 1u));
+                    }
+                }
+    }
+    __syncthreads();
+    const uint32_t past = sh.first_past;
+    return past == ~0u || (past & 1) != 0 ? -1 : static_cast<int32_t>(past >> 1);
+}
+
 __device__ __forceinline__ void sample_pick(const PickArgs& a, int64_t& token) {
     __shared__ PickShared sh;
     const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
@@ -887,7 +973,8 @@ __device__ __forceinline__ void sample_pick(const PickArgs& a, int64_t& token) {
     // key at or above it, so only their rows are read (head workgroup g wrote the rows of row
     // pairs g * 4 + w + j * 4 * parts, w < 4). Too many such workgroups or keys: the full scan.
     const int64_t parts = a.parts;
-    bool from_parts = top_k <= parts && parts <= kPickThreads;
+    const bool all = top_k >= V && parts <= kPickThreads;  // every entry is kept: only the extremes are needed
+    bool from_parts = all || (top_k <= parts && parts <= kPickThreads);
     if (from_parts) {
         const bool mine = tid < parts;
         const uint32_t phi = mine ? a.key_parts[2 * tid] : 0u;
@@ -914,14 +1001,14 @@ __device__ __forceinline__ void sample_pick(const PickArgs& a, int64_t& token) {
         }
         kmax = __builtin_amdgcn_readfirstlane(kmax);
         kmin = __builtin_amdgcn_readfirstlane(kmin);
-        low = max(1u, radix_select([&](const auto& f) { f(phi, mine); }, top_k, sh, 2));
-        if (mine && phi >= low) {
+        if (!all) low = max(1u, radix_select([&](const auto& f) { f(phi, mine); }, top_k, sh, 2));
+        if (!all && mine && phi >= low) {
             const uint32_t at = atomicAdd(&sh.nparts, 1u);
             if (at < kPickParts) sh.cand_parts[at] = tid;
         }
         __syncthreads();
         const uint32_t np = __builtin_amdgcn_readfirstlane(sh.nparts);
-        if (np <= kPickParts) {
+        if (!all && np <= kPickParts) {
             const int64_t pairs = (V + 1) / 2, stride = parts * (kThreads / 64);
             const int64_t per_part = 2 * (kThreads / 64) * ((pairs + stride - 1) / stride);  // rows, at most
             const int64_t items = int64_t{np} * per_part;
@@ -961,7 +1048,7 @@ __device__ __forceinline__ void sample_pick(const PickArgs& a, int64_t& token) {
                 listed_n = appended;
             }
         }
-        from_parts = unordered;
+        from_parts = all || unordered;
     }
     if (!from_parts) {  // the full scan
         uint32_t key[kPickSlots];
@@ -1051,9 +1138,11 @@ __device__ __forceinline__ void sample_pick(const PickArgs& a, int64_t& token) {
     // the k-th largest key and the kept entries (keys at or above it) in index order
     constexpr int kListGroups = kPickLdsKept / kPickThreads;
     int64_t m;
-    int32_t* kept;
-    float* kept_e;
-    if (listed) {
+    int32_t* kept = nullptr;
+    float* kept_e = nullptr;
+    if (all) {
+        m = V;
+    } else if (listed) {
         const auto listed_key = [&](int j) {
             const int64_t r = int64_t{j} * kPickThreads + tid;
             return r < listed_n ? sh.cand_key[r] : 0u;
@@ -1140,9 +1229,55 @@ __device__ __forceinline__ void sample_pick(const PickArgs& a, int64_t& token) {
     // again as head_kernel divides it; key_value recovers the largest x exactly
     const float temp = a.sp->temperature;
     const float mx = key_value(kmax);
-    for (int64_t r = tid; r < m; r += kPickThreads) kept_e[r] = expf(__fdiv_rn(a.logits[kept[r]], temp) - mx);
-    __syncthreads();
-    int32_t nonfinite = kmax > kFiniteKeyHigh || kmin < kFiniteKeyLow;
+    const auto exponential = [&](float logit) { return expf(__fdiv_rn(logit, temp) - mx); };
+    const int32_t nonfinite = kmax > kFiniteKeyHigh || kmin < kFiniteKeyLow;
+    const bool drawn = !nonfinite && draw < draws;
+    if (!all) {
+        for (int64_t r = tid; r < m; r += kPickThreads) kept_e[r] = exponential(a.logits[kept[r]]);
+        __syncthreads();
+    }
+    if (drawn && m > 64) {
+        f4pick e[kShare4];
+        const int n = __builtin_amdgcn_readfirstlane(static_cast<int>(m));
+        const int share = share_of(n), first = tid * share;
+        const float* from = all ? a.logits : kept_e;
+#pragma unroll
+        for (int g = 0; g < kShare4; ++g) {
+            if (4 * g >= share) continue;
+            const int at = first + 4 * g;
+            f4pick v = {0.f, 0.f, 0.f, 0.f};
+            if (at + 3 < n) {
+                v = *reinterpret_cast<const f4pick*>(from + at);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (at + c < n) v[c] = from[at + c];
+            }
+            e[g] = v;
+        }
+        if (all) {
+#pragma unroll
+            for (int g = 0; g < kShare4; ++g)
+                if (4 * g < share)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) e[g][c] = first + 4 * g + c < n ? exponential(e[g][c]) : 0.f;
+        }
+        const int32_t at = parallel_pick(e, n, u, sh);
+        if (at >= 0) {
+            if (tid == 0) a.sp->draw = draw + 1;
+            token = all ? at : kept[at];
+            return;
+        }
+    }
+    if (all) {  // the fold in order reads the list
+        kept = a.kept;
+        kept_e = a.kept_e;
+        for (int64_t r = tid; r < m; r += kPickThreads) {
+            kept[r] = static_cast<int32_t>(r);
+            kept_e[r] = exponential(a.logits[r]);
+        }
+        __syncthreads();
+    }
     if (wave != 0) return;
     // The sums below run in index order in double, as kael's CPU loops do: wave 0 loads 64 entries
     // at a time, one per lane, and folds them in lane order through readlane, so only one load per
