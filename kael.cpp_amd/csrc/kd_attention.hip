@@ -26,6 +26,7 @@
 // hardware exp2 (__expf: a few ulp), well inside the device tolerance kael's tests apply.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "kd_internal.h"
 
@@ -218,37 +219,50 @@ __device__ __forceinline__ v16f dot_rows(const float (&a)[32], const float (&b)[
 
 // ---- forward -----------------------------------------------------------------------------
 
+// Where the forward's heads lie: elements between batches, heads and rows of q, and of k and v.
+struct HeadViews {
+    const float *q, *k, *v;
+    int64_t q_batch, q_head, q_row;
+    int64_t kv_batch, kv_head, kv_row;
+};
+
+// Exact: exponentials by expf and the softmax's sum in double, as the GPT-2 engine's decode step has
+// them; otherwise the hardware exp2 and an f32 sum.
+template <bool Exact>
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float* __restrict__ out, float* __restrict__ lse,
-                                                                           const float* __restrict__ qkv,
-                                                                           AttentionShape sh) {
+                                                                           HeadViews in, AttentionShape sh) {
     __shared__ float tiles[kWaves * kTile];  // each wave's K, then V, tile of its current key block
     __shared__ float qtile[kTile];           // the query block
-    __shared__ float ms[kWaves][kBlock], ls[kWaves][kBlock];
+    typedef std::conditional_t<Exact, double, float> Sum;
+    const auto exponential = [](float x) { return Exact ? expf(x) : __expf(x); };
+    __shared__ float ms[kWaves][kBlock];
+    __shared__ Sum ls[kWaves][kBlock];
     const int blocks = (sh.length + kBlock - 1) / kBlock;
     const int units = sh.batch * sh.heads;
     const int bh = static_cast<int>(blockIdx.x % units);
     const int qb = blocks - 1 - static_cast<int>(blockIdx.x / units);  // longest rows first, all heads interleaved
     const int b = bh / sh.heads, h = bh % sh.heads;
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 32, lh = lane / 32;
-    const float* q = qkv + static_cast<int64_t>(b) * sh.length * sh.row + h * kD;
-    const float* k = q + sh.heads * kD;
-    const float* v = k + sh.heads * kD;
+    const float* __restrict__ q = in.q + b * in.q_batch + h * in.q_head;
+    const float* __restrict__ k = in.k + b * in.kv_batch + h * in.kv_head;
+    const float* __restrict__ v = in.v + b * in.kv_batch + h * in.kv_head;
     float* tile = tiles + wave * kTile;
     const int query = qb * kBlock + li;
 
     // every load in flight together: the wave's quarter of the query block, its first K and V tiles
     v4f qpart[kPartVec], kload[kTileVec], vload[kTileVec];
-    part_load(qpart, q, qb * kBlock, sh.length, sh.row, wave, lane);
+    part_load(qpart, q, qb * kBlock, sh.length, in.q_row, wave, lane);
     if (wave <= qb) {
-        tile_load(kload, k, wave * kBlock, sh.length, sh.row, lane);
-        tile_load(vload, v, wave * kBlock, sh.length, sh.row, lane);
+        tile_load(kload, k, wave * kBlock, sh.length, in.kv_row, lane);
+        tile_load(vload, v, wave * kBlock, sh.length, in.kv_row, lane);
     }
     part_store(qtile, qpart, wave, lane);
     __syncthreads();
     float qreg[32];
     lds_half_row(qreg, qtile, li, lh);
     v16f o[2] = {zero16(), zero16()};
-    float m = -INFINITY, l = 0.f;
+    float m = -INFINITY;
+    Sum l = 0;
     for (int kb = wave; kb <= qb; kb += kWaves) {
         const int j0 = kb * kBlock;
         float kreg[32];
@@ -260,8 +274,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
         wave_sync();
         const bool more = kb + kWaves <= qb;
         if (more) {  // the next block's loads run while this block computes
-            tile_load(kload, k, j0 + kWaves * kBlock, sh.length, sh.row, lane);
-            tile_load(vload, v, j0 + kWaves * kBlock, sh.length, sh.row, lane);
+            tile_load(kload, k, j0 + kWaves * kBlock, sh.length, in.kv_row, lane);
+            tile_load(vload, v, j0 + kWaves * kBlock, sh.length, in.kv_row, lane);
         }
         v16f s = dot_rows(kreg, qreg);
         // scale, mask, block max of this query's scores (16 here, 16 in lane li + 32)
@@ -275,15 +289,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
         }
         bmax = halves_max(bmax);
         const float mnew = fmaxf(m, bmax);
-        const float alpha = mnew == -INFINITY ? 1.f : __expf(m - mnew);
-        float bsum = 0.f;
+        const float alpha = mnew == -INFINITY ? 1.f : exponential(m - mnew);
+        Sum bsum = 0;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float p = s[r] == -INFINITY ? 0.f : __expf(s[r] - mnew);
+            const float p = s[r] == -INFINITY ? 0.f : exponential(s[r] - mnew);
             s[r] = p;
             bsum += p;
         }
-        bsum = halves_sum(bsum);
+        if constexpr (Exact) bsum += __shfl_xor(bsum, 32);
+        else bsum = halves_sum(bsum);
         l = l * alpha + bsum;
         m = mnew;
 #pragma unroll
@@ -318,19 +333,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
         float mx = ms[0][row];
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, ms[w][row]);
-        float total = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        Sum total = 0;
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            const float f = ms[w][row] == -INFINITY ? 0.f : __expf(ms[w][row] - mx);
+            const float f = ms[w][row] == -INFINITY ? 0.f : exponential(ms[w][row] - mx);
             total += f * ls[w][row];
 #pragma unroll
             for (int c = 0; c < 8; ++c) acc[c] += f * tiles[w * kTile + row * kLd + c0 + c];
         }
-        const float inv = 1.f / total;
+        const float inv = 1.f / static_cast<float>(total);
         float* dst = out + (static_cast<int64_t>(b) * sh.length + t) * sh.out_row + h * kD + c0;
         *reinterpret_cast<v4f*>(dst) = v4f{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
         *reinterpret_cast<v4f*>(dst + 4) = v4f{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
-        if (lane % 8 == 0) lse[static_cast<int64_t>(bh) * sh.length + t] = mx + logf(total);
+        if (lse != nullptr && lane % 8 == 0) lse[static_cast<int64_t>(bh) * sh.length + t] = mx + logf(static_cast<float>(total));
     }
 }
 
@@ -703,7 +719,22 @@ int check_shape(int dtype, int64_t batch, int64_t length, int64_t heads, int64_t
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+template <bool Exact> int launch_forward(float* out, float* lse, const HeadViews& in, const AttentionShape& sh) {
+    const int64_t blocks = (sh.length + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(attention_forward_kernel<Exact>, dim3(static_cast<uint32_t>(sh.batch * sh.heads * blocks)), dim3(kWaves * 64),
+                       0, stream(), out, lse, in, sh);
+    KD_LAUNCH_CHECK();
+    return KD_OK;
+}
+
 } // namespace
+
+int causal_attention_heads(float* out, const float* q, int64_t q_row, const float* k, const float* v, int64_t kv_head,
+                           int64_t length, int64_t heads) {
+    AttentionShape sh;
+    if (int rc = check_shape(KD_F32, 1, length, heads, kD, sh, "causal_attention_heads")) return rc;
+    return launch_forward<true>(out, nullptr, HeadViews{q, k, v, 0, kD, q_row, 0, kv_head, kD}, sh);
+}
 
 } // namespace kd
 
@@ -716,11 +747,10 @@ extern "C" int kd_causal_attention(int dtype, void* out, void* lse, const void* 
     if (out == nullptr || qkv == nullptr || lse == nullptr || !aligned16(out) || !aligned16(qkv))
         return fail(KD_E_INVALID, "kd_causal_attention: out, lse and qkv must be given, out and qkv 16-byte aligned");
     if (int rc = ensure_device()) return rc;
-    const int64_t blocks = (length + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(attention_forward_kernel, dim3(static_cast<uint32_t>(batch * heads * blocks)), dim3(kWaves * 64), 0,
-                       stream(), static_cast<float*>(out), static_cast<float*>(lse), static_cast<const float*>(qkv), sh);
-    KD_LAUNCH_CHECK();
-    return KD_OK;
+    const float* q = static_cast<const float*>(qkv);
+    const int64_t width = heads * kD, tokens = length * sh.row;
+    return launch_forward<false>(static_cast<float*>(out), static_cast<float*>(lse),
+                          HeadViews{q, q + width, q + 2 * width, tokens, kD, sh.row, tokens, kD, sh.row}, sh);
 }
 
 extern "C" int kd_causal_attention_backward(int dtype, void* dqkv, const void* dout, const void* qkv, const void* out,

@@ -1576,10 +1576,11 @@ __global__ __launch_bounds__(kThreads) void attention_kernel(const Step* st, con
 // ---- batched prefill ---------------------------------------------------------------------------
 //
 // The prompt's T positions pass each layer together: row LayerNorms, the four Linear products
-// as GEMMs on the MFMA matmul path (weights in [in, out] copies made once so that both operands
-// are row-major; prompts of up to 128 positions as split-K partial products on 64x64 tiles, longer
-// ones on the backend's matmul path), epilogue kernels for the partial
-// sums, the bias, residual, GELU and the K/V rows into the cache, and a causal attention kernel.
+// on the matrix cores (prompts of up to 128 positions as split-K partial products on 64x64 tiles,
+// longer ones as the main product family plans them), epilogue kernels for the partial sums, the
+// bias, residual, GELU and the K/V rows into the cache, and causal attention: kd_attention.hip's
+// forward with the engine's exponentials and sums where the head dim is 64 (1000 positions, 12 heads:
+// 135 us a layer on the kernel below, 2.38 ms a prompt from 3.51), the kernel below elsewhere.
 // Same arithmetic as the decode step; only the summation order of the dot products differs.
 
 // The row LayerNorm H[t] = LayerNorm(X[t]) of a row that lane i of the workgroup has just
@@ -1644,6 +1645,8 @@ __global__ __launch_bounds__(kThreads) void prefill_embed_kernel(const int64_t* 
 // (P the sum of `splits` partials `split_stride` apart, added in split order), then, with ln_w,
 // H[t] = LayerNorm(X[t]) for the next product (the following LayerNorm, computed in the same
 // workgroup instead of a launch of its own).
+// Batch: the partials loaded before the first add, the fewest of 4, 8 and 16 that cover the splits.
+template <int Batch>
 __global__ __launch_bounds__(kThreads) void prefill_residual_kernel(const float* P, int64_t splits, int64_t split_stride,
                                                                     const float* bias, float* X, const float* ln_w,
                                                                     const float* ln_b, float* H, int64_t d) {
@@ -1666,10 +1669,10 @@ __global__ __launch_bounds__(kThreads) void prefill_residual_kernel(const float*
 #pragma unroll
         for (int j = 0; j < 4; ++j) p[j] = P[t * d + std::min<int64_t>(threadIdx.x + j * kThreads, d - 1)];
     }
-    for (int64_t s0 = 0; s0 < splits && splits > 1; s0 += kSplitBatch) {
-        float v[kSplitBatch][4];
+    for (int64_t s0 = 0; s0 < splits && splits > 1; s0 += Batch) {
+        float v[Batch][4];
 #pragma unroll
-        for (int q = 0; q < kSplitBatch; ++q) {
+        for (int q = 0; q < Batch; ++q) {
             const int64_t sq = std::min<int64_t>(s0 + q, splits - 1);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -1678,7 +1681,7 @@ __global__ __launch_bounds__(kThreads) void prefill_residual_kernel(const float*
             }
         }
 #pragma unroll
-        for (int q = 0; q < kSplitBatch; ++q)  // added in split order
+        for (int q = 0; q < Batch; ++q)  // added in split order
             if (s0 + q < splits) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) p[j] = s0 + q == 0 ? v[q][j] : __fadd_rn(p[j], v[q][j]);
@@ -1855,8 +1858,7 @@ struct Engine {
     float* pf_q = nullptr;    // [pf_rows, d] queries
     float* pf_a = nullptr;    // [pf_rows, d] attention output
     float* pf_f = nullptr;    // [pf_rows, ff] GELU output
-    float* pf_p = nullptr;    // [pf_rows, max(3d, ff)] product before its epilogue
-    float* pf_parts = nullptr;  // split-K partial products of prompts of at most 128 positions
+    float* pf_parts = nullptr;  // products before their epilogues: one, or split-K partials
 
     const float* p(const std::string& name) const { return params + offsets.at(name).first; }
 
@@ -2016,8 +2018,7 @@ struct Engine {
     int ensure_prefill_buffers() {
         if (pf_x != nullptr) return KD_OK;
         pf_rows = (cfg.max_positions + 127) / 128 * 128;
-        for (auto [ptr, cols] : {std::pair<float**, int64_t>{&pf_x, d}, {&pf_h, d}, {&pf_q, d}, {&pf_a, d}, {&pf_f, ff},
-                                 {&pf_p, std::max(3 * d, ff)}}) {
+        for (auto [ptr, cols] : {std::pair<float**, int64_t>{&pf_x, d}, {&pf_h, d}, {&pf_q, d}, {&pf_a, d}, {&pf_f, ff}}) {
             void* mem = nullptr;
             KD_HIP(hipMalloc(&mem, static_cast<size_t>(pf_rows * cols) * sizeof(float)));
             *ptr = static_cast<float*>(mem);
@@ -2028,11 +2029,16 @@ struct Engine {
         return KD_OK;
     }
 
-    // Prompts of at most kShortPrompt positions: the products split over K into pf_parts (at most one 64x64-tile workgroup per CU, or one whole product), which the
-    // epilogue adds in split order.
+    // Prompts of at most kShortPrompt positions: the products split over K (at most one 64x64-tile
+    // workgroup per CU, or one whole product). (256: the same at 129 to 256 positions.)
     static constexpr int64_t kShortPrompt = 128;
+    // Up to so many, longer prompts leave their partials to the epilogue as well (129 positions 1.03 ms, 1.10
+    // with a sum of its own); beyond, the epilogues, a workgroup per row, take longer over the partials
+    // than that sum (1000 positions: 2.48 ms against 2.38).
+    static constexpr int64_t kPartsPrompt = 256;
     int64_t parts_floats() const {
-        return std::max<int64_t>(int64_t{compute_units()} * 64 * 64, kShortPrompt * std::max(3 * d, ff));
+        const int64_t splits = int64_t{compute_units()} * 64 * 64, rows = (cfg.max_positions + 127) / 128 * 128;
+        return std::max({splits, rows * std::max(3 * d, ff), kPartsPrompt * 16 * d});
     }
 
     // A product ready for its epilogue: P (row stride N), or `splits` partials `stride` apart.
@@ -2046,7 +2052,7 @@ struct Engine {
     // kShortPrompt positions with K a multiple of 32: K split so that the 64x64-tile grid holds up to
     // one workgroup per CU (GPT-2 small at T = 64: qkv 36 tiles x 6, proj 12 x 12, fc1 48 x 4,
     // fc2 12 x 16), the partials left for the epilogue to add; each product reads its weights once.
-    // Otherwise the backend's matmul path.
+    // Otherwise the main product family, its splits left for the epilogue too up to kPartsPrompt.
     int product(const float* A, const float* W, int64_t T, int64_t K, int64_t N, Product* out) const {
         if (T <= kShortPrompt && K % 32 == 0) {
             const int64_t tiles = (T + 63) / 64 * ((N + 63) / 64);
@@ -2057,10 +2063,16 @@ struct Engine {
             *out = Product{pf_parts, splits, T * N};
             return kd::matmul_split_parts(A, W, pf_parts, T, N, K, K, K, splits);
         }
-        const kd_matmul_sizes sz{1, T, K, N};
-        const kd_matmul_strides st{{0, K, 1}, {0, 1, K}, {0, N, 1}};
-        *out = Product{pf_p, 1, 0};
-        return kd_matmul_strided(KD_F32, A, W, pf_p, &sz, &st);
+        if (T > kPartsPrompt) {
+            const kd_matmul_sizes sz{1, T, K, N};
+            const kd_matmul_strides st{{0, K, 1}, {0, 1, K}, {0, N, 1}};
+            *out = Product{pf_parts, 1, 0};
+            return kd_matmul_strided(KD_F32, A, W, pf_parts, &sz, &st);
+        }
+        int64_t splits = 1;
+        if (int rc = kd::matmul_linear_parts(A, W, pf_parts, parts_floats(), T, N, K, &splits)) return rc;
+        *out = Product{pf_parts, splits, T * N};
+        return KD_OK;
     }
 
     template <int Epi>
@@ -2095,8 +2107,14 @@ struct Engine {
         // X += P + bias per row, then H = the next LayerNorm of X (none after the last block: the
         // head kernel normalises the last row itself)
         const auto residual = [&](const float* bias, const float* ln_w, const float* ln_b) {
-            hipLaunchKernelGGL(prefill_residual_kernel, dim3(static_cast<uint32_t>(T)), dim3(kThreads), 0, s, pr.P, pr.splits,
-                               pr.stride, bias, pf_x, ln_w, ln_b, pf_h, d);
+            const dim3 rows(static_cast<uint32_t>(T));
+            const auto launch = [&](auto batch) {
+                hipLaunchKernelGGL(prefill_residual_kernel<decltype(batch)::value>, rows, dim3(kThreads), 0, s, pr.P, pr.splits,
+                                   pr.stride, bias, pf_x, ln_w, ln_b, pf_h, d);
+            };
+            if (pr.splits <= 4) launch(std::integral_constant<int, 4>{});
+            else if (pr.splits <= 8) launch(std::integral_constant<int, 8>{});
+            else launch(std::integral_constant<int, kSplitBatch>{});
         };
         for (int64_t l = 0; l < cfg.layers; ++l) {
             const std::string b = "blocks." + std::to_string(l) + ".";
@@ -2106,9 +2124,13 @@ struct Engine {
             float* vc = vcache + l * cfg.heads * cfg.max_positions * hd;
             if (int rc = product(pf_h, p(b + "attn.qkv.weight"), T, d, 3 * d, &pr)) return rc;
             epilogue<kQkv>(pr, p(b + "attn.qkv.bias"), pf_q, T, 3 * d, kc, vc);
-            hipLaunchKernelGGL(prefill_attention_kernel, dim3(static_cast<uint32_t>(cfg.heads), static_cast<uint32_t>(T)),
-                               dim3(kThreads), static_cast<size_t>(T) * sizeof(float), s, pf_q, kc, vc, pf_a, d, hd,
-                               cfg.max_positions, divisor);
+            if (hd == 64) {
+                if (int rc = kd::causal_attention_heads(pf_a, pf_q, d, kc, vc, cfg.max_positions * hd, T, cfg.heads)) return rc;
+            } else {
+                hipLaunchKernelGGL(prefill_attention_kernel, dim3(static_cast<uint32_t>(cfg.heads), static_cast<uint32_t>(T)),
+                                   dim3(kThreads), static_cast<size_t>(T) * sizeof(float), s, pf_q, kc, vc, pf_a, d, hd,
+                                   cfg.max_positions, divisor);
+            }
             if (int rc = product(pf_a, p(b + "attn.proj.weight"), T, d, d, &pr)) return rc;
             residual(p(b + "attn.proj.bias"), p(b + "ln2.weight"), p(b + "ln2.bias"));
             if (int rc = product(pf_h, p(b + "mlp.fc1.weight"), T, d, ff, &pr)) return rc;
@@ -2201,7 +2223,7 @@ struct Engine {
     ~Engine() {
         if (graph) (void)hipGraphExecDestroy(graph);
         for (void* ptr : {static_cast<void*>(pf_x), static_cast<void*>(pf_h), static_cast<void*>(pf_q),
-                          static_cast<void*>(pf_a), static_cast<void*>(pf_f), static_cast<void*>(pf_p), static_cast<void*>(pf_parts)})
+                          static_cast<void*>(pf_a), static_cast<void*>(pf_f), static_cast<void*>(pf_parts)})
             if (ptr) (void)hipFree(ptr);
         for (void* ptr : {static_cast<void*>(params), static_cast<void*>(kcache), static_cast<void*>(vcache),
                           static_cast<void*>(x), static_cast<void*>(q), static_cast<void*>(partials.m),

@@ -60,6 +60,17 @@ int workspace(Workspace& lease, size_t bytes);
 int matmul_split_parts(const float* a, const float* b, float* parts, int64_t M, int64_t N, int64_t K, int64_t lda,
                        int64_t ldb, int64_t splits);
 
+// The same for longer operands, on the tiles and splits that kd_matmul's main family would take, as far as
+// `capacity` floats hold the partials (at least M * N); *splits says how many there are.
+int matmul_linear_parts(const float* a, const float* b, float* parts, int64_t capacity, int64_t M, int64_t N, int64_t K,
+                        int64_t* splits);
+
+// kd_causal_attention's forward for one sequence whose heads lie apart (the GPT-2 engine's prefill):
+// q [length, heads * 64] with `q_row` floats between rows, k and v [heads][..][64] with `kv_head` floats
+// between heads, out [length, heads * 64]; every pointer 16-byte aligned, strides multiples of 4.
+int causal_attention_heads(float* out, const float* q, int64_t q_row, const float* k, const float* v, int64_t kv_head,
+                           int64_t length, int64_t heads);
+
 inline int64_t dtype_size(int dtype) {
     switch (dtype) {
     case KD_F32: return 4;

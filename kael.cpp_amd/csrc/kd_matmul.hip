@@ -883,7 +883,7 @@ struct Plan {
 // The cheapest by the times above: n workgroups per CU take steps * n * crowded (one alone its own
 // time), and the ends of those that run at once overlap. Splitting K adds the sum of the partials: a
 // launch and their way from memory (10 x 768 x 256: 3.9 us).
-Plan plan_pieces(int64_t M, int64_t N, int64_t K, int64_t batches) {
+Plan plan_pieces(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t most_splits = 64) {
     constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32, 48, 64};
     const int64_t cus = compute_units();
     const double outputs = static_cast<double>(M) * static_cast<double>(N) * static_cast<double>(batches);
@@ -894,7 +894,7 @@ Plan plan_pieces(int64_t M, int64_t N, int64_t K, int64_t batches) {
         int64_t last_k = 0;
         for (const int want : kSplits) {
             // at least 64 deep, at most four rounds of workgroups, and partials of at most 256 MiB
-            if (want > 1 && (K < want * 64 || tiles * want > 4 * cus * tl.per_cu || want * outputs > 0x1p26)) break;
+            if (want > 1 && (want > most_splits || K < want * 64 || tiles * want > 4 * cus * tl.per_cu || want * outputs > 0x1p26)) break;
             const int64_t k_split = ((K + want - 1) / want + 31) / 32 * 32;
             if (k_split == last_k) continue;
             last_k = k_split;
@@ -942,6 +942,19 @@ bool pieces_addressable(const MatmulArgs& p) {
            (p.sa.c == 1 || fits(p.sa.r, p.sa.c)) && (p.sb.r == 1 || fits(p.sb.c, p.sb.r));
 }
 
+// Enqueues `plan` for p; split s writes split_o * s floats into `out`.
+int launch_plan(const Plan& plan, const float* a, const float* b, float* out, const MatmulArgs& p, int64_t split_o) {
+    const Tiling& tl = kTilings[plan.tiling];
+    const int64_t tiles = (p.M + tl.tm - 1) / tl.tm * ((p.N + tl.tn - 1) / tl.tn);
+    if (tiles > (int64_t{1} << 31) - 1) return fail(KD_E_INVALID, "kd_matmul: too many tiles");
+    const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches), static_cast<uint32_t>(plan.splits));
+    with_k_modes(p.sa.c == 1, p.sb.r == 1, [&](auto ak, auto bk) {
+        launch_pieces<decltype(ak)::value, decltype(bk)::value>(plan.tiling, grid, a, b, out, p, static_cast<int>(plan.k_split),
+                                                                split_o);
+    });
+    return launch_status();
+}
+
 int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
     // the batches fold into M when they share B and lie back to back in A and the output
     if (p.batches > 1 && p.heads == 1 && p.sb.b == 0 && p.sa.b == p.M * p.sa.r && p.so.b == p.M * p.so.r &&
@@ -950,18 +963,7 @@ int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
         p.batches = 1;
     }
     const Plan plan = plan_pieces(p.M, p.N, p.K, p.batches);
-    const Tiling& tl = kTilings[plan.tiling];
-    const int64_t tiles = (p.M + tl.tm - 1) / tl.tm * ((p.N + tl.tn - 1) / tl.tn);
-    if (tiles > (int64_t{1} << 31) - 1) return fail(KD_E_INVALID, "kd_matmul: too many tiles");
-    const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches), static_cast<uint32_t>(plan.splits));
-    const auto launch = [&](float* to, const MatmulArgs& q, int64_t split_o) {
-        with_k_modes(q.sa.c == 1, q.sb.r == 1, [&](auto ak, auto bk) {
-            launch_pieces<decltype(ak)::value, decltype(bk)::value>(plan.tiling, grid, a, b, to, q,
-                                                                    static_cast<int>(plan.k_split), split_o);
-        });
-        return launch_status();
-    };
-    if (plan.splits == 1) return launch(out, p, 0);
+    if (plan.splits == 1) return launch_plan(plan, a, b, out, p, 0);
     Workspace ws;  // held until the sum is enqueued
     const int64_t per = p.M * p.N;
     if (int rc = workspace(ws, static_cast<size_t>(plan.splits * p.batches * per) * sizeof(float))) return rc;
@@ -969,7 +971,7 @@ int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
     partial.bias = nullptr;
     partial.ho = plan.splits * per;
     partial.so = Strides3{p.heads * partial.ho, p.N, 1};
-    if (int rc = launch(static_cast<float*>(ws.ptr), partial, per)) return rc;
+    if (int rc = launch_plan(plan, a, b, static_cast<float*>(ws.ptr), partial, per)) return rc;
     return launch_split_sum(static_cast<const float*>(ws.ptr), out, p, plan.splits);
 }
 
@@ -1181,6 +1183,23 @@ int matmul_split_parts(const float* a, const float* b, float* parts, int64_t M, 
     if (deep % 64 == 0) hipLaunchKernelGGL((parts_kernel<64>), grid, dim3(kThreads), 0, stream(), a, b, parts, m, n, deep, la, lb);
     else hipLaunchKernelGGL((parts_kernel<32>), grid, dim3(kThreads), 0, stream(), a, b, parts, m, n, deep, la, lb);
     return launch_status();
+}
+
+int matmul_linear_parts(const float* a, const float* b, float* parts, int64_t capacity, int64_t M, int64_t N, int64_t K,
+                        int64_t* splits) {
+    MatmulArgs p;
+    p.batches = 1;
+    p.M = M;
+    p.K = K;
+    p.N = N;
+    p.sa = {0, K, 1};
+    p.sb = {0, 1, K};
+    p.so = {0, N, 1};
+    if (M <= 0 || N <= 0 || K <= 0 || capacity < M * N || !pieces_addressable(p))
+        return fail(KD_E_INVALID, "matmul_linear_parts: operands outside the product's bounds");
+    const Plan plan = plan_pieces(M, N, K, 1, capacity / (M * N));
+    *splits = plan.splits;
+    return launch_plan(plan, a, b, parts, p, M * N);
 }
 
 } // namespace kd
