@@ -612,15 +612,17 @@ __global__ __launch_bounds__(kSmallWaves * 64) void small_kernel(const float* __
 // ---- parts family (f32, the GPT-2 engine's short prompts) ---------------------------------------
 
 constexpr int kPartTile = 64;
+constexpr int kPartStages = 2;  // stages of loads in flight
 
 // Split-K partial products x . W^T of prompts of 33 to 128 positions on the f32 matrix cores: 64x64
-// tiles, blockIdx.y the K split, `k_split` deep (a multiple of 32). Such a product streams its weights
+// tiles, blockIdx.y the K split, `k_split` deep (a multiple of Deep). Such a product streams its weights
 // once and is a chain of a few loads, so what counts is the time from the first load to the last store:
-// four waves of one 32x32 accumulator, K 32 at a time through double-buffered LDS, loads two stages
-// ahead. The pieces of 64x64 tiles take 2 us longer here for the split into pieces (GPT-2 small, 64
-// positions: a prefill 0.73 ms on this kernel, 0.85 on pieces, 0.86 on the small tiles), and win from
-// a few hundred deep. Waves 0-1 load A, waves 2-3 load B (K-contiguous rows, written transposed);
-// rows past M and N repeat the last and are not stored.
+// four waves of one 32x32 accumulator, K 64 at a time through double-buffered LDS, so that a row's load
+// is 256 contiguous bytes (32 at a time, 128 bytes: 9.1 us a launch against 8.3), loads two stages ahead
+// (three: no change). GPT-2 small, 64 positions: a prefill 0.75 ms on this kernel, 0.85 on the pieces of
+// 64x64 tiles, whose split takes 2 us of such a launch, and 0.86 on the small tiles, which win up to 32
+// positions (0.60 against 0.67). Waves 0-1 load A, waves 2-3 load B; rows past M and N repeat the last
+// and are not stored.
 template <int Deep>
 __global__ __launch_bounds__(kThreads) void parts_kernel(const float* __restrict__ a, const float* __restrict__ b,
                                                          float* __restrict__ parts, int M, int N, int k_split, int lda,
@@ -629,8 +631,8 @@ __global__ __launch_bounds__(kThreads) void parts_kernel(const float* __restrict
     constexpr int kLd = Deep + 4;       // tiles [row][k]: conflict-free 16-byte reads and writes
     constexpr int kLanes = Deep / 4;    // lanes that load a row's stage
     constexpr int kRows = kThreads / 2 / kLanes, kLoads = kPartTile / kRows;
-    __shared__ __attribute__((aligned(16))) float As[2][kPartTile * kLd];
-    __shared__ __attribute__((aligned(16))) float Bs[2][kPartTile * kLd];
+    __shared__ __attribute__((aligned(16))) float As[kPartStages][kPartTile * kLd];
+    __shared__ __attribute__((aligned(16))) float Bs[kPartStages][kPartTile * kLd];
     int64_t tm, tn;
     tile_of(blockIdx.x, (M + kPartTile - 1) / kPartTile, (N + kPartTile - 1) / kPartTile, tm, tn);
     const int m0 = static_cast<int>(tm) * kPartTile;
@@ -678,23 +680,23 @@ __global__ __launch_bounds__(kThreads) void parts_kernel(const float* __restrict
         }
     };
     const int steps = k_split / Deep;
-    f4 r0[kLoads], r1[kLoads];
-    fetch(r0, 0);
-    if (steps > 1) fetch(r1, 1);
-    stash(r0, 0);
+    f4 r[kPartStages][kLoads];
+#pragma unroll
+    for (int q = 0; q < kPartStages; ++q)
+        if (q < steps) fetch(r[q], q);
+    stash(r[0], 0);
     __syncthreads();
-    int ks = 0;
-    for (; ks + 1 < steps; ks += 2) {
-        if (ks + 2 < steps) fetch(r0, ks + 2);
-        step(0);
-        stash(r1, 1);
-        __syncthreads();
-        if (ks + 3 < steps) fetch(r1, ks + 3);
-        step(1);
-        if (ks + 2 < steps) stash(r0, 0);
-        __syncthreads();
+    for (int s0 = 0; s0 < steps; s0 += kPartStages) {
+#pragma unroll
+        for (int q = 0; q < kPartStages; ++q) {
+            const int s = s0 + q;
+            if (s >= steps) break;
+            if (s + kPartStages < steps) fetch(r[q], s + kPartStages);
+            step(q);
+            if (s + 1 < steps) stash(r[(q + 1) % kPartStages], (q + 1) % kPartStages);
+            __syncthreads();
+        }
     }
-    if (ks < steps) step(0);  // an odd step count's last step
     const int col = n0 + wn * 32 + li;
     if (col >= N) return;
 #pragma unroll
@@ -1176,6 +1178,20 @@ int matmul_split_parts(const float* a, const float* b, float* parts, int64_t M, 
     if (M <= 0 || N <= 0 || K <= 0 || M >= kMax || N >= kMax || K >= kMax || lda >= kMax || ldb >= kMax || splits < 1 ||
         splits > 65535 || K % (32 * splits) != 0)
         return fail(KD_E_INVALID, "matmul_split_parts: operands outside the split-K kernel's bounds");
+    if (M <= kSmallTile) {  // the small tiles, the splits as batches: their K offsets as batch strides
+        MatmulArgs p;
+        p.batches = splits;
+        p.M = M;
+        p.K = K / splits;
+        p.N = N;
+        p.sa = {p.K, lda, 1};
+        p.sb = {p.K, 1, ldb};
+        p.so = {M * N, N, 1};
+        hipLaunchKernelGGL((small_kernel<true, true>),
+                           dim3(static_cast<uint32_t>((N + kSmallTile - 1) / kSmallTile), 1, static_cast<uint32_t>(splits)),
+                           dim3(kSmallWaves * 64), 0, stream(), a, b, parts, p);
+        return launch_status();
+    }
     const int64_t tiles = (M + kPartTile - 1) / kPartTile * ((N + kPartTile - 1) / kPartTile);
     const dim3 grid(static_cast<uint32_t>(tiles), static_cast<uint32_t>(splits));
     const int m = static_cast<int>(M), n = static_cast<int>(N), deep = static_cast<int>(K / splits);
