@@ -34,7 +34,7 @@ ARCH = "gfx950"
 HIP_FLAGS = [
     "-O3", "-std=c++20", "-fPIC", f"--offload-arch={ARCH}",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-Wall", "-Wno-unused-function", "-I", str(INCLUDE), "-I", str(CSRC),
+    "-Wall", "-Wno-unused-function", "-I", str(INCLUDE), "-I", str(CSRC), "-I", str(HOST),
 ]
 HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-Wall", "-I", str(INCLUDE)]
 

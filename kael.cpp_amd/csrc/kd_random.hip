@@ -22,11 +22,25 @@
 //
 // Device layout: draw e is element e. The draws split into blocks that follow the twists: block 0
 // is what is left of the current state (words pos..311), block j >= 1 the 312 words of the j-th
-// twist. Every workgroup runs the twist chain in LDS (two barriers per 312 draws) and handles the
-// blocks j with j % gridDim.x == blockIdx.x: it tempers their words, compares, and loads and
-// stores their elements, the input of its next block loaded one block ahead. The memory traffic is
-// spread over the chip; only the cheap chain is serial. The workgroup of the last block writes the
-// final state to a second buffer (others may still be reading the first).
+// twist. The twists are a serial chain: in a workgroup three waves twist from one half of an LDS buffer
+// into the other while five temper, compare, load and store the elements of the current block, with one
+// barrier a block (0.24 us; with all waves twisting behind two barriers 0.37, and the elements after it).
+//
+// Few draws (up to kSerialBlocks blocks): every workgroup runs the chain and handles the blocks j with
+// j % gridDim.x == blockIdx.x. The workgroup of the last block writes the final state to a second
+// buffer (others may still be reading the first).
+//
+// More: rounds of up to 64 chains of 64 blocks, each chain's first words reached by a jump
+// (kd_mt_jump.h): one workgroup writes the round's first 65 blocks of words; the words that each other
+// chain starts from are sums of about 10^4 of them, taken by 16 workgroups a chain that each add
+// the words of a range of coefficients (exclusive or: any order gives the same); then a workgroup
+// per chain walks its own 64 blocks. 2^20 draws: 1.26 ms on one chain, 0.13 ms so, of which the three
+// kernels take 20, 50 (LDS reads: 17 MB a chain) and 39 us. At 300 blocks the two are even (0.10 ms).
+#include "kd_mt_jump.h"
+
+#include <algorithm>
+#include <mutex>
+
 #include "kd_internal.h"
 
 namespace kd {
@@ -39,6 +53,16 @@ constexpr uint64_t kMatrixA = 0xB5026F5AA96619E9ull;
 constexpr uint64_t kUpperMask = 0xFFFFFFFF80000000ull;  // the top 33 bits
 constexpr uint64_t kLowerMask = 0x000000007FFFFFFFull;  // the low 31 bits
 constexpr int kRngThreads = 320;                         // 312 words, rounded up to whole waves
+constexpr int kTwistThreads = 192;                       // the waves that twist (156 words)
+constexpr int kChainThreads = kTwistThreads + kRngThreads;
+constexpr int64_t kSerialBlocks = 300;
+constexpr int64_t kRoundBlocks = int64_t{kJumpBlocks} * kJumpChains;
+constexpr int kJumpSplits = 16;                          // workgroups that share a chain's jump
+constexpr int kJumpWords = (kWords + kJumpSplits - 1) / kJumpSplits;  // coefficient words of each
+static_assert(kWords == kMtWords && kJumpBlocks * kWords >= kMtDegree + 1);  // 65 blocks hold every word a jump adds
+
+// The jump polynomials, copied here before the first launch that reads them.
+__device__ uint64_t g_jump[(kJumpChains - 1) * kWords];
 
 __host__ __device__ __forceinline__ uint64_t twist_word(uint64_t first, uint64_t second, uint64_t far) {
     const uint64_t y = (first & kUpperMask) | (second & kLowerMask);
@@ -79,72 +103,187 @@ struct RngArgs {
     double p;            // the compare threshold (keep for dropout)
 };
 
-// Dropout = true: out = in * (u < p) / T(p) (and mask = T(u < p) when asked for). Dropout = false:
-// out = T(u < p).
-template <typename T, bool Dropout>
-__global__ __launch_bounds__(kRngThreads) void mt_kernel(RngArgs a, T keep_t) {
-    __shared__ uint64_t mt[2][kWords];
-    const int t = threadIdx.x;
-    if (t < kWords) mt[0][t] = a.state[t];
-    const int64_t pos = static_cast<int64_t>(a.state[kWords]);
+// The next 312 words after `old`, into `nw`, by three waves: thread k < 156 makes words k and k + 156. A
+// word's second half mixes the same thread's word of the first half (the last one also word 0, which its
+// thread makes too), so a twist is one round of LDS reads, without a barrier inside.
+__device__ __forceinline__ void twist(const uint64_t* __restrict__ old, uint64_t* __restrict__ nw, int k) {
+    if (k >= kShift) return;
+    const uint64_t m0 = old[k + kShift];
+    const uint64_t first = twist_word(old[k], old[k + 1], m0);
+    const uint64_t second = k + 1 < kShift ? old[k + kShift + 1] : twist_word(old[0], old[1], old[kShift]);
+    nw[k] = first;
+    nw[k + kShift] = twist_word(m0, second, first);
+}
+
+// One workgroup's walk from the words of block `first` in mt[0] to block `last`: the first three waves
+// twist to the next block while the others (t = 0 .. 319) visit the current one, then all meet. Returns
+// which half of `mt` holds the last block's words.
+template <class Visit>
+__device__ __forceinline__ int walk(uint64_t (&mt)[2][kWords], int64_t first, int64_t last, const Visit& visit) {
     int cur = 0;
-    const int64_t G = gridDim.x;
-    const int64_t mine = static_cast<int64_t>(blockIdx.x);
-    // element range of block j
-    auto start = [&](int64_t j) { return j == 0 ? int64_t{0} : a.first + (j - 1) * kWords; };
-    auto size = [&](int64_t j) {
+    for (int64_t j = first;; ++j) {
+        if (threadIdx.x >= kTwistThreads) visit(j, mt[cur]);
+        else if (j < last) twist(mt[cur], mt[cur ^ 1], threadIdx.x);
+        if (j >= last) return cur;
+        __syncthreads();
+        cur ^= 1;
+    }
+}
+
+// A thread's elements of the blocks that its workgroup handles: thread t element t of each. Dropout =
+// true: out = in * (u < p) / T(p) (and mask = T(u < p) when asked for). Dropout = false: out = T(u < p).
+template <typename T, bool Dropout> struct Elements {
+    const RngArgs& a;
+    const int t;
+    const T keep;
+    const int64_t pos, last;
+    T x = T(0), y = T(0);  // the inputs of the next two blocks (a block takes less than a load's way from memory)
+
+    __device__ __forceinline__ int64_t start(int64_t j) const { return j == 0 ? int64_t{0} : a.first + (j - 1) * kWords; }
+    __device__ __forceinline__ int64_t size(int64_t j) const {
         return j == 0 ? a.first : std::min<int64_t>(kWords, a.count - start(j));
-    };
-    const T* in = static_cast<const T*>(a.in);
-    T* out = static_cast<T*>(a.out);
-    T* mask = static_cast<T*>(a.mask);
-    // the input of this workgroup's next block, loaded a block ahead
-    T x = T(0);
-    if constexpr (Dropout) {
-        if (mine < a.blocks && t < size(mine)) x = in[start(mine) + t];
     }
+    __device__ __forceinline__ T input(int64_t j) const {
+        if constexpr (Dropout) {
+            if (j <= last && t < size(j)) return static_cast<const T*>(a.in)[start(j) + t];
+        }
+        return T(0);
+    }
+    // before the first block, `step` apart
+    __device__ __forceinline__ void begin(int64_t j, int64_t step) {
+        x = input(j);
+        y = input(j + step);
+    }
+    // block j from its words; `next` is the block after the next, whose input is loaded meanwhile
+    __device__ __forceinline__ void draw(int64_t j, const uint64_t* words, int64_t next) {
+        const T mine = x;
+        x = y;
+        y = input(next);
+        if (t >= size(j)) return;
+        const int64_t e = start(j) + t;
+        const bool hit = canonical(temper(words[(j == 0 ? pos : 0) + t])) < a.p;
+        if constexpr (Dropout) {
+            static_cast<T*>(a.out)[e] = dropped<T>(mine, hit, keep);
+            if (a.mask != nullptr) static_cast<T*>(a.mask)[e] = hit ? T(1) : T(0);
+        } else {
+            static_cast<T*>(a.out)[e] = hit ? T(1) : T(0);
+        }
+    }
+};
+
+// The state after the last draw: the current words and the index past the last one used.
+__device__ __forceinline__ void store_state(const RngArgs& a, const uint64_t (&words)[kWords], int64_t pos, int t) {
     const int64_t last = a.blocks - 1;
-    const int64_t own_last = mine <= last ? last - (last - mine) % G : -1;  // this workgroup's last block
+    if (t < kWords) a.next[t] = words[t];
+    if (t == 0)
+        a.next[kWords] = static_cast<uint64_t>(last == 0 ? pos + a.first
+                                                         : std::min<int64_t>(kWords, a.count - (a.first + (last - 1) * kWords)));
+}
+
+template <typename T, bool Dropout>
+__global__ __launch_bounds__(kChainThreads) void mt_kernel(RngArgs a, T keep_t) {
+    __shared__ uint64_t mt[2][kWords];
+    const int t = static_cast<int>(threadIdx.x) - kTwistThreads;  // below 0: a twisting wave
+    if (t >= 0 && t < kWords) mt[0][t] = a.state[t];
+    const int64_t pos = static_cast<int64_t>(a.state[kWords]);
+    const int64_t G = gridDim.x, mine = blockIdx.x, last = a.blocks - 1;
+    if (mine > last) return;
+    const int64_t own_last = last - (last - mine) % G;  // this workgroup's last block
+    Elements<T, Dropout> elements{a, t, keep_t, pos, own_last};
+    if (t >= 0) elements.begin(mine, G);
+    int64_t next = mine;
     __syncthreads();
-    for (int64_t j = 0; j <= own_last; ++j) {
-        if (j > 0) {
-            const uint64_t* old = mt[cur];
-            uint64_t* nw = mt[cur ^ 1];
-            if (t < kShift) nw[t] = twist_word(old[t], old[t + 1], old[t + kShift]);
-            __syncthreads();
-            if (t >= kShift && t < kWords) {
-                const uint64_t second = t + 1 < kWords ? old[t + 1] : nw[0];
-                nw[t] = twist_word(old[t], second, nw[t - kShift]);
-            }
-            __syncthreads();
-            cur ^= 1;
-        }
-        if (j % G == mine) {
-            const int64_t n = size(j);
-            const int64_t word = j == 0 ? pos : 0;
-            const int64_t e = start(j) + t;
-            T xn = T(0);
-            if constexpr (Dropout) {
-                const int64_t next = j + G;
-                if (next <= last && t < size(next)) xn = in[start(next) + t];
-            }
-            if (t < n) {
-                const bool hit = canonical(temper(mt[cur][word + t])) < a.p;
-                if constexpr (Dropout) {
-                    out[e] = dropped<T>(x, hit, keep_t);
-                    if (mask != nullptr) mask[e] = hit ? T(1) : T(0);
-                } else {
-                    out[e] = hit ? T(1) : T(0);
-                }
-            }
-            x = xn;
-        }
+    const int cur = walk(mt, 0, own_last, [&](int64_t j, const uint64_t* words) {
+        if (j != next) return;
+        next += G;
+        elements.draw(j, words, j + 2 * G);
+    });
+    if (own_last == last && t >= 0) store_state(a, mt[cur], pos, t);
+}
+
+// The words of a round's first 65 blocks, from its first block's in a.state (first round) or the block
+// before it in `before`, and zeros for the chains' starts.
+__global__ __launch_bounds__(kChainThreads) void round_words_kernel(RngArgs a, const uint64_t* before, uint64_t* words,
+                                                                    uint64_t* starts, int chains) {
+    __shared__ uint64_t mt[2][kWords];
+    const int t = static_cast<int>(threadIdx.x) - kTwistThreads;
+    for (int i = threadIdx.x; i < (chains - 1) * kWords; i += kChainThreads) starts[i] = 0;
+    const int skip = before != nullptr ? 1 : 0;
+    if (t >= 0 && t < kWords) mt[0][t] = skip ? before[t] : a.state[t];
+    __syncthreads();
+    walk(mt, 0, kJumpBlocks + skip, [&](int64_t j, const uint64_t* block) {
+        if (j >= skip && t < kWords) words[(j - skip) * kWords + t] = block[t];
+    });
+}
+
+// Workgroup (s, c): the sum of the words that coefficient words s * kJumpWords .. of chain c + 1's
+// polynomial select, added to the chain's start.
+__global__ __launch_bounds__(kRngThreads) void jump_kernel(const uint64_t* words, uint64_t* starts) {
+    constexpr int kSpan = kJumpWords * 64 + kWords;
+    __shared__ uint64_t w[kSpan];
+    const int t = threadIdx.x;
+    const int first = blockIdx.x * kJumpWords;
+    // coefficient k selects words k + 1 .. k + 312, all within the 65 blocks; past them no coefficient is set
+    for (int i = t; i < kSpan; i += kRngThreads) {
+        const int at = first * 64 + 1 + i;
+        w[i] = at < (kJumpBlocks + 1) * kWords ? words[at] : 0;
     }
-    if (mine == last % G) {
-        // state after the last draw: the current words and the index past the last one used
-        if (t < kWords) a.next[t] = mt[cur][t];
-        if (t == 0) a.next[kWords] = static_cast<uint64_t>(last == 0 ? pos + a.first : size(last));
+    __syncthreads();
+    const uint64_t* p = g_jump + blockIdx.y * kWords;
+    uint64_t sum = 0;
+    const int mine = t < kWords ? t : 0;
+    for (int q = 0; q < kJumpWords && first + q < kWords; ++q) {
+        const uint64_t coefficients = p[first + q];  // the same for every lane: scalar, as are its bit numbers
+        uint64_t bits = (uint64_t{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(coefficients >> 32)))} << 32) |
+                        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(coefficients)));
+        const uint64_t* from = w + q * 64 + mine;
+        const auto lowest = [&]() {
+            const int k = __ffsll(static_cast<unsigned long long>(bits)) - 1;
+            bits &= bits - 1;
+            return k;
+        };
+        for (int n = __popcll(bits) / 8; n > 0; --n) {  // eight reads in flight
+            uint64_t x[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = from[lowest()];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum ^= x[i];
+        }
+        while (bits != 0) sum ^= from[lowest()];
     }
+    if (t < kWords)
+        atomicXor(reinterpret_cast<unsigned long long*>(starts + blockIdx.y * kWords + t), static_cast<unsigned long long>(sum));
+}
+
+// Chain blockIdx.x of the round that starts at block `round`: its own blocks, and the last chain's last
+// words for the next round.
+template <typename T, bool Dropout>
+__global__ __launch_bounds__(kChainThreads) void chain_kernel(RngArgs a, T keep_t, int64_t round, const uint64_t* words,
+                                                              const uint64_t* starts, uint64_t* after) {
+    __shared__ uint64_t mt[2][kWords];
+    const int t = static_cast<int>(threadIdx.x) - kTwistThreads;
+    const int64_t chain = blockIdx.x;
+    if (t >= 0 && t < kWords) mt[0][t] = chain == 0 ? words[t] : starts[(chain - 1) * kWords + t];
+    const int64_t pos = static_cast<int64_t>(a.state[kWords]);
+    const int64_t first = round + chain * kJumpBlocks, last = std::min<int64_t>(a.blocks, first + kJumpBlocks) - 1;
+    Elements<T, Dropout> elements{a, t, keep_t, pos, last};
+    if (t >= 0) elements.begin(first, 1);
+    __syncthreads();
+    const int cur = walk(mt, first, last, [&](int64_t j, const uint64_t* block) { elements.draw(j, block, j + 2); });
+    if (t < 0) return;
+    if (last == a.blocks - 1) store_state(a, mt[cur], pos, t);
+    else if (chain == kJumpChains - 1 && t < kWords) after[t] = mt[cur][t];
+}
+
+// The polynomials on the device, copied once (a first call per device; kd_dropout and kd_bernoulli block).
+int ensure_jump(const uint64_t* polynomials) {
+    static std::mutex mutex;
+    static bool ready = false;
+    std::lock_guard<std::mutex> lock(mutex);
+    if (ready) return KD_OK;
+    KD_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_jump), polynomials, sizeof g_jump, 0, hipMemcpyHostToDevice));
+    ready = true;
+    return KD_OK;
 }
 
 template <typename T, bool Dropout>
@@ -158,17 +297,40 @@ int run_rng(void* out, void* mask, const void* in, int64_t count, double p, uint
     a.first = std::min<int64_t>(kWords - pos, count);
     a.blocks = 1 + (count - a.first + kWords - 1) / kWords;
     a.p = p;
+    const uint64_t* polynomials = a.blocks > kSerialBlocks ? mt_jump_polynomials() : nullptr;
+    if (polynomials != nullptr)
+        if (int rc = ensure_jump(polynomials)) return rc;
+    // the state, the state after, then (for rounds) a round's words, its chains' starts, and its last words
+    constexpr int64_t kRoundWords = int64_t{kJumpBlocks + 1} * kWords;
+    const int64_t words = 2 * (kWords + 1) + (polynomials != nullptr ? kRoundWords + int64_t{kJumpChains} * kWords : 0);
     Workspace lease;
-    if (int rc = workspace(lease, 2 * (kWords + 1) * sizeof(uint64_t))) return rc;
+    if (int rc = workspace(lease, static_cast<size_t>(words) * sizeof(uint64_t))) return rc;
     uint64_t* dev_state = static_cast<uint64_t*>(lease.ptr);
     a.state = dev_state;
     a.next = dev_state + kWords + 1;
     hipStream_t s = stream();
     KD_HIP(hipMemcpyAsync(dev_state, host_state, (kWords + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, s));
-    // Enough workgroups that each handles a few blocks, at most two per CU.
-    const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(a.blocks, 2 * int64_t{compute_units()}));
-    hipLaunchKernelGGL((mt_kernel<T, Dropout>), dim3(static_cast<uint32_t>(grid)), dim3(kRngThreads), 0, s, a,
-                       static_cast<T>(p));
+    if (polynomials != nullptr) {
+        uint64_t* round_words = dev_state + 2 * (kWords + 1);
+        uint64_t* starts = round_words + kRoundWords;
+        uint64_t* after = starts + (kJumpChains - 1) * kWords;
+        for (int64_t round = 0; round < a.blocks; round += kRoundBlocks) {
+            const int64_t left = std::min<int64_t>(kRoundBlocks, a.blocks - round);
+            const int chains = static_cast<int>((left + kJumpBlocks - 1) / kJumpBlocks);
+            hipLaunchKernelGGL(round_words_kernel, dim3(1), dim3(kChainThreads), 0, s, a, round == 0 ? nullptr : after,
+                               round_words, starts, chains);
+            if (chains > 1)
+                hipLaunchKernelGGL(jump_kernel, dim3(kJumpSplits, static_cast<uint32_t>(chains - 1)), dim3(kRngThreads), 0, s,
+                                   round_words, starts);
+            hipLaunchKernelGGL((chain_kernel<T, Dropout>), dim3(static_cast<uint32_t>(chains)), dim3(kChainThreads), 0, s, a,
+                               static_cast<T>(p), round, round_words, starts, after);
+        }
+    } else {
+        // Enough workgroups that each handles a few blocks, at most two per CU.
+        const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(a.blocks, 2 * int64_t{compute_units()}));
+        hipLaunchKernelGGL((mt_kernel<T, Dropout>), dim3(static_cast<uint32_t>(grid)), dim3(kChainThreads), 0, s, a,
+                           static_cast<T>(p));
+    }
     KD_LAUNCH_CHECK();
     KD_HIP(hipMemcpyAsync(host_state, a.next, (kWords + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     KD_HIP(hipStreamSynchronize(s));
