@@ -768,6 +768,63 @@ __global__ __launch_bounds__(kThreads) void split_sum_flat_kernel(const float* _
     }
 }
 
+// ---- rowdot family (f32, N <= 4 over more batches than a grid's second dimension holds) -----------
+
+constexpr int kRowdotMaxN = 4;
+constexpr int64_t kGridBatches = 65535;
+
+// One wave per (batch, row), all in the grid's first dimension; lanes stride along K. Up to kGridBatches
+// batches the small tiles and the pieces are quicker (4096 x 4096 x 4: 22 us against 116 here).
+template <bool AVec>
+__global__ __launch_bounds__(kThreads) void rowdot_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                          float* __restrict__ out, MatmulArgs p) {
+    const int lane = threadIdx.x % 64;
+    const int64_t row_id = static_cast<int64_t>(blockIdx.x) * (kThreads / 64) + threadIdx.x / 64;
+    if (row_id >= p.batches * p.M) return;
+    const int64_t batch = row_id / p.M;
+    const int64_t m = row_id % p.M;
+    const float* arow = a + batch_offset(p, batch, p.sa.b, p.ha) + m * p.sa.r;
+    const float* bb = b + batch_offset(p, batch, p.sb.b, p.hb);
+    float acc[kRowdotMaxN] = {0.f, 0.f, 0.f, 0.f};
+    if (AVec) {
+        const int64_t vecs = p.K / 4;
+        for (int64_t v = lane; v < vecs; v += 64) {
+            const float4 x = *reinterpret_cast<const float4*>(arow + 4 * v);
+            const int64_t k = 4 * v;
+#pragma unroll
+            for (int n = 0; n < kRowdotMaxN; ++n) {
+                if (n < p.N) {
+                    const float* bc = bb + n * p.sb.c;
+                    acc[n] += x.x * bc[k * p.sb.r] + x.y * bc[(k + 1) * p.sb.r] + x.z * bc[(k + 2) * p.sb.r] +
+                              x.w * bc[(k + 3) * p.sb.r];
+                }
+            }
+        }
+        for (int64_t k = vecs * 4 + lane; k < p.K; k += 64) {
+#pragma unroll
+            for (int n = 0; n < kRowdotMaxN; ++n)
+                if (n < p.N) acc[n] += arow[k] * bb[k * p.sb.r + n * p.sb.c];
+        }
+    } else {
+        for (int64_t k = lane; k < p.K; k += 64) {
+            const float x = arow[k * p.sa.c];
+#pragma unroll
+            for (int n = 0; n < kRowdotMaxN; ++n)
+                if (n < p.N) acc[n] += x * bb[k * p.sb.r + n * p.sb.c];
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < kRowdotMaxN; ++n) {
+#pragma unroll
+        for (int off = 32; off > 0; off /= 2) acc[n] += __shfl_xor(acc[n], off, 64);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int n = 0; n < kRowdotMaxN; ++n)
+            if (n < p.N) out[batch_offset(p, batch, p.so.b, p.ho) + m * p.so.r + n * p.so.c] = plus_bias(acc[n], p.bias, n);
+    }
+}
+
 // ---- tiled family (f64 / i64) ----------------------------------------------------------------------
 
 constexpr int kTT = 64;  // tile edge
@@ -940,7 +997,7 @@ int launch_split_sum(const float* partial, float* out, const MatmulArgs& p, int6
 bool pieces_addressable(const MatmulArgs& p) {
     constexpr int64_t kMax = int64_t{1} << 31;
     const auto fits = [](int64_t rows, int64_t k) { return rows >= 0 && k >= 0 && rows < (kMax >> 9) && k < (kMax >> 6); };
-    return p.M < kMax - 256 && p.N < kMax - 256 && p.K < kMax - 256 && p.batches <= 65535 &&
+    return p.M < kMax - 256 && p.N < kMax - 256 && p.K < kMax - 256 && p.batches <= kGridBatches &&
            (p.sa.c == 1 || fits(p.sa.r, p.sa.c)) && (p.sb.r == 1 || fits(p.sb.c, p.sb.r));
 }
 
@@ -979,11 +1036,19 @@ int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
 
 int matmul_f32(const float* a, const float* b, float* out, const MatmulArgs& p) {
     const int cus = compute_units();
+    if (p.batches > kGridBatches) {
+        if (p.N > kRowdotMaxN) return fail(KD_E_INVALID, "kd_matmul: too many batches");
+        const bool avec = p.sa.c == 1 && p.sa.r % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && aligned16(a);
+        const dim3 grid(static_cast<uint32_t>((p.batches * p.M + 3) / 4));
+        if (avec) hipLaunchKernelGGL((rowdot_kernel<true>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
+        else hipLaunchKernelGGL((rowdot_kernel<false>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
+        return launch_status();
+    }
     const bool pieces = pieces_addressable(p);
     const int64_t gm = (p.M + kSmallTile - 1) / kSmallTile;
     const int64_t gn = (p.N + kSmallTile - 1) / kSmallTile;
     const bool fits32 = p.K * std::abs(p.sa.c) < (int64_t{1} << 31) && p.K * std::abs(p.sb.r) < (int64_t{1} << 31);
-    if (fits32 && gm <= 65535 && p.batches <= 65535 && gm * gn * p.batches <= 2 * int64_t{cus}) {
+    if (fits32 && gm <= 65535 && gm * gn * p.batches <= 2 * int64_t{cus}) {
         // Small tiles where they are estimated to be quicker than the pieces' best plan: a launch and its
         // ends, and 0.85 us per 128 of K (16 waves of 8), 2 where a CU has two tiles. Measured, small /
         // pieces: 512^3 6.5 / 11.4 us, 256^3 4.3 / 8.3, 128 x 64 x 784 2.9 / 6.0, 64 x 784 x 128 with B
@@ -1003,7 +1068,6 @@ int matmul_f32(const float* a, const float* b, float* out, const MatmulArgs& p) 
     }
     if (pieces) return matmul_pieces(a, b, out, p);
     const int64_t tiles = ((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
-    if (p.batches > 65535) return fail(KD_E_INVALID, "kd_matmul: too many batches");
     hipLaunchKernelGGL(general_f32_kernel, dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches)), dim3(kThreads),
                        0, stream(), a, b, out, p);
     return launch_status();

@@ -131,3 +131,16 @@ def test_split_batches_of_heads(kdb):
     kdb.call("matmul_strided_heads", kd.F32, da.ptr, db.ptr, out.ptr, sizes, strides,
              kd.MatmulHeads(heads, m * k, k * n, m * n))
     check(out.numpy(), a, b)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4])
+@pytest.mark.parametrize("k", [6, 64])
+def test_few_columns_over_more_batches_than_a_grid_dimension(kdb, k, n):
+    """Over 65535 batches: up to 4 columns run, more are refused."""
+    rng = np.random.default_rng(n)
+    a, b = rng.normal(size=(65536 + 5, 2, k)).astype(np.float32), rng.normal(size=(65536 + 5, k, n)).astype(np.float32)
+    sizes = (len(a), 2, k, n)
+    check(product(kdb, a, b, sizes, (2 * k, k, 1), (k * n, n, 1)), a, b)
+    x = kdb.to_device(a)
+    strides = kd.MatmulStrides((2 * k, k, 1), (0, 5, 1), (10, 5, 1))
+    assert kdb.lib.kd_matmul_strided(kd.F32, x.ptr, x.ptr, x.ptr, kd.MatmulSizes(len(a), 2, k, 5), strides) != 0
