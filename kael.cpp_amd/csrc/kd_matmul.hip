@@ -1021,7 +1021,11 @@ int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
         p.M *= p.batches;
         p.batches = 1;
     }
-    const Plan plan = plan_pieces(p.M, p.N, p.K, p.batches);
+    // A graph would hold on to partials in the shared workspace, which a later call may free to grow it, and
+    // growing it is no call to make under capture: a captured product is not split.
+    hipStreamCaptureStatus captured = hipStreamCaptureStatusNone;
+    if (stream() != nullptr) KD_HIP(hipStreamIsCapturing(stream(), &captured));
+    const Plan plan = plan_pieces(p.M, p.N, p.K, p.batches, captured == hipStreamCaptureStatusNone ? 64 : 1);
     if (plan.splits == 1) return launch_plan(plan, a, b, out, p, 0);
     Workspace ws;  // held until the sum is enqueued
     const int64_t per = p.M * p.N;

@@ -144,3 +144,41 @@ def test_few_columns_over_more_batches_than_a_grid_dimension(kdb, k, n):
     x = kdb.to_device(a)
     strides = kd.MatmulStrides((2 * k, k, 1), (0, 5, 1), (10, 5, 1))
     assert kdb.lib.kd_matmul_strided(kd.F32, x.ptr, x.ptr, x.ptr, kd.MatmulSizes(len(a), 2, k, 5), strides) != 0
+
+
+@pytest.mark.parametrize("m,k,n", [(300, 3000, 260), (64, 5000, 64)])
+def test_captured_products_keep_no_workspace(kdb, m, k, n):
+    """A product that runs in splits when it is called is one kernel of a captured graph, and its replays do not depend on
+    what other calls do to the shared workspace between them."""
+    lib = kdb.lib
+    rng = np.random.default_rng(m)
+    a, b = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(k, n)).astype(np.float32)
+    da, db, out = kdb.to_device(a), kdb.to_device(b), kdb.empty((m, n), np.float32)
+    eager = kdb.empty((m, n), np.float32)
+    sizes = kd.MatmulSizes(1, m, k, n)
+    stream, graph, run, nodes = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t()
+    kdb.call("matmul", kd.F32, da.ptr, db.ptr, eager.ptr, sizes)  # the kernels are loaded outside the capture
+    assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
+    lib.kd_get_stream.restype = ctypes.c_void_p
+    before = ctypes.c_void_p(lib.kd_get_stream())
+    kdb.synchronize()
+    try:
+        lib.kd_set_stream(stream)
+        assert lib.hipStreamBeginCapture(stream, 1) == 0  # thread-local
+        rc = lib.kd_matmul(kd.F32, da.ptr, db.ptr, out.ptr, sizes)
+        assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0 and rc == 0
+        assert lib.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 1
+        assert lib.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+        for _ in range(3):
+            kdb.call("matmul", kd.F32, da.ptr, db.ptr, eager.ptr, sizes)
+            assert lib.hipGraphLaunch(run, stream) == 0
+            assert lib.hipStreamSynchronize(stream) == 0
+            check(out.numpy(), a, b)
+            check(eager.numpy(), a, b)
+    finally:
+        lib.kd_set_stream(before)
+        if run:
+            lib.hipGraphExecDestroy(run)
+        if graph:
+            lib.hipGraphDestroy(graph)
+        lib.hipStreamDestroy(stream)
