@@ -12,6 +12,8 @@
 // output is written in the merged-head layout and the row's log-sum-exp m + log(l) is kept for
 // the backward.
 //
+// Many queries take attention_forward_pieces_kernel: the same sums with the products on the bf16 matrix cores.
+//
 // Backward (the gradient of every op of kael's chain: the products, the scale, the mask and
 // softmax backward y (g - sum(g y))): with delta_i = sum_d dO[i][d] O[i][d] (= sum_j P dP over
 // the row) and P recomputed from the log-sum-exp, dS = P (dP - delta) / sqrt(D), one launch of two
@@ -29,6 +31,7 @@
 #include <type_traits>
 
 #include "kd_internal.h"
+#include "kd_pieces.h"
 
 namespace kd {
 
@@ -350,6 +353,259 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
     }
 }
 
+// ---- forward on pieces ---------------------------------------------------------------------
+//
+// The products in three bf16 pieces per operand (kd_matmul.hip): 96 MFMAs of 32 cycles a block pair
+// would be 4096 cycles in f32, 48 here take 1536. What the split costs decides the layout: a workgroup
+// of four waves takes 128 queries, 32 a wave with their pieces in registers, and walks the key blocks
+// together, each K and V block split once (16 elements a thread) into double-buffered LDS and read by
+// all four. An LDS unit is 8 k-values of one row, 16 bytes a piece, as an MFMA takes them: K by 8
+// features, V by the 8 keys that a lane's score registers hold, so that P is an operand as it stands.
+// Every query's keys pass through one wave, which needs no merge.
+//
+// 8 x 1024 tokens, 12 heads: 154 -> 100 us (129 TFLOP/s). A step of a workgroup alone takes 1.8 us, 0.7 of
+// it MFMAs; two workgroups of a CU overlap, and the VALU work (the split, the exponentials) is what is left.
+// The next block's split runs between the MFMAs of the scores: 105 -> 100 us, alone 77 -> 62. Error of the
+// output against 64 bits 2.0e-7 -> 1.4e-7.
+//
+// A workgroup that meets a value above 1e18, an infinity or a NaN (pieces or their products may be infinite)
+// starts again on the f32 matrix cores, straight from memory.
+constexpr int kWide = 128;                             // queries of a workgroup
+constexpr int kKeyGroup = kBlock * 16 + 32;            // bytes of 8 features of the keys; 32 against bank conflicts
+constexpr int kKeyPiece = kD / 8 * kKeyGroup;
+constexpr int kValueGroup = kD * 16;                   // bytes of 8 keys of the features
+constexpr int kValuePiece = kBlock / 8 * kValueGroup;
+constexpr int kStage = 3 * (kKeyPiece + kValuePiece);
+constexpr float kPieceLimit = 1e18f;
+
+__device__ __forceinline__ bool past_limit(const float (&x)[8]) {
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum += fabsf(x[e]);
+    return !(sum <= kPieceLimit);
+}
+
+__device__ __forceinline__ void store_pieces(char* unit, int piece, const float (&x)[8]) {
+    bf8 hi, mid, lo;
+    split_pieces(x, hi, mid, lo);
+    *reinterpret_cast<bf8*>(unit) = hi;
+    *reinterpret_cast<bf8*>(unit + piece) = mid;
+    *reinterpret_cast<bf8*>(unit + 2 * piece) = lo;
+}
+
+// hi and small accumulate one 16-deep product of pieces.
+__device__ __forceinline__ void multiply_pieces(const bf8 (&a)[3], const bf8 (&b)[3], v16f& hi, v16f& small) {
+    constexpr int kA[5] = {2, 0, 1, 1, 0}, kB[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+    for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kA[q]], b[kB[q]], small, 0, 0, 0);
+    hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], hi, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kernel(float* __restrict__ out, float* __restrict__ lse,
+                                                                                  HeadViews in, AttentionShape sh) {
+    __shared__ __attribute__((aligned(16))) char stages[2][kStage];
+    __shared__ int bad[2];  // the last block (+ 1) of each stage that pieces cannot hold
+    const int tiles = (sh.length + kWide - 1) / kWide;
+    const int units = sh.batch * sh.heads;
+    const int bh = static_cast<int>(blockIdx.x % units);
+    const int q0 = (tiles - 1 - static_cast<int>(blockIdx.x / units)) * kWide;  // longest rows first, all heads interleaved
+    const int b = bh / sh.heads, h = bh % sh.heads;
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 32, lh = lane / 32;
+    const float* __restrict__ q = in.q + b * in.q_batch + h * in.q_head;
+    const float* __restrict__ k = in.k + b * in.kv_batch + h * in.kv_head;
+    const float* __restrict__ v = in.v + b * in.kv_batch + h * in.kv_head;
+    const int query = q0 + wave * kBlock + li;
+    const int blocks = min(q0 + kWide, sh.length - 1 + kBlock) / kBlock;  // of keys, up to the workgroup's last query
+    const int last = q0 / kBlock + wave;                                  // this wave's last block
+
+    // A thread's part of a block: 8 features of one key, and one feature of 8 keys.
+    const int key = threadIdx.x / 8, feature = 8 * (threadIdx.x % 8);
+    float kx[8], vx[8];
+    const auto load = [&](int kb) {
+        const int j0 = kb * kBlock;
+        const v4f a = row_piece(k, j0 + key, sh.length, in.kv_row, feature / 4);
+        const v4f c = row_piece(k, j0 + key, sh.length, in.kv_row, feature / 4 + 1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            kx[e] = a[e];
+            kx[4 + e] = c[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int row = j0 + block_row(8 * (wave / 2) + e, wave % 2);
+            const float x = v[static_cast<int64_t>(min(row, sh.length - 1)) * in.kv_row + lane];
+            vx[e] = row < sh.length ? x : 0.f;
+        }
+    };
+    const auto store = [&](int kb) {
+        char* stage = stages[kb % 2];
+        store_pieces(stage + feature / 8 * kKeyGroup + key * 16, kKeyPiece, kx);
+        store_pieces(stage + 3 * kKeyPiece + wave * kValueGroup + lane * 16, kValuePiece, vx);
+        if (past_limit(kx) || past_limit(vx)) bad[kb % 2] = kb + 1;
+    };
+
+    if (threadIdx.x < 2) bad[threadIdx.x] = 0;
+    load(0);
+    bf8 qp[kD / 16][3];
+    bool far = false;
+    const float* qrow = q + static_cast<int64_t>(min(query, sh.length - 1)) * in.q_row;
+#pragma unroll
+    for (int s = 0; s < kD / 16; ++s) {
+        const v4f a = *reinterpret_cast<const v4f*>(qrow + 16 * s + 8 * lh);
+        const v4f c = *reinterpret_cast<const v4f*>(qrow + 16 * s + 8 * lh + 4);
+        const float x[8] = {a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+        split_pieces(x, qp[s][0], qp[s][1], qp[s][2]);
+        far = far || past_limit(x);
+    }
+    __syncthreads();
+    store(0);
+    if (far) bad[0] = 1;
+    load(1);  // (past the last block: the last row again, never used)
+    __syncthreads();
+
+    v16f o[2] = {zero16(), zero16()}, o_small[2] = {zero16(), zero16()};
+    float m = -INFINITY, l = 0.f;
+    bool redo = false;
+    for (int kb = 0; kb < blocks; ++kb) {
+        redo = bad[kb % 2] == kb + 1;  // the same for every wave: the stage is written again after the next barrier
+        if (redo) break;
+        const bool mine = kb <= last;  // a wave past its diagonal only loads
+        const char* stage = stages[kb % 2];
+        v16f s = zero16();
+        if (mine) {
+            v16f small = zero16();
+#pragma unroll
+            for (int g = 0; g < kD / 16; ++g) {
+                bf8 kp[3];
+#pragma unroll
+                for (int w = 0; w < 3; ++w)
+                    kp[w] = *reinterpret_cast<const bf8*>(stage + w * kKeyPiece + (2 * g + lh) * kKeyGroup + li * 16);
+                multiply_pieces(kp, qp[g], s, small);
+            }
+            store(kb + 1);
+#pragma unroll
+            for (int g = 0; g < kD / 16 * 6; ++g) {  // the split's VALU work between these MFMAs
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+            }
+            s += small;
+        } else {
+            store(kb + 1);
+        }
+        load(kb + 2);
+        if (mine) {
+            // scale and mask; the scores are finite, and every query has a key in block 0
+            float bmax = -INFINITY;
+            if (kb == last) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[r] = block_row(r, lh) > li ? -INFINITY : s[r] * sh.inv_scale;
+                    bmax = fmaxf(bmax, s[r]);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[r] *= sh.inv_scale;
+                    bmax = fmaxf(bmax, s[r]);
+                }
+            }
+            const float mnew = fmaxf(m, halves_max(bmax));
+            const float alpha = __expf(m - mnew);
+            float bsum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = __expf(s[r] - mnew);
+                bsum += s[r];
+            }
+            l = l * alpha + halves_sum(bsum);
+            m = mnew;
+            if (__any(alpha != 1.f)) {
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        o[dt][r] *= alpha;
+                        o_small[dt][r] *= alpha;
+                    }
+            }
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const float x[8] = {s[8 * g], s[8 * g + 1], s[8 * g + 2], s[8 * g + 3],
+                                    s[8 * g + 4], s[8 * g + 5], s[8 * g + 6], s[8 * g + 7]};
+                bf8 pp[3];
+                split_pieces(x, pp[0], pp[1], pp[2]);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    bf8 vp[3];
+#pragma unroll
+                    for (int w = 0; w < 3; ++w)
+                        vp[w] = *reinterpret_cast<const bf8*>(stage + 3 * kKeyPiece + w * kValuePiece +
+                                                              (2 * g + lh) * kValueGroup + (32 * dt + li) * 16);
+                    multiply_pieces(vp, pp, o[dt], o_small[dt]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (redo) {
+        m = -INFINITY;
+        l = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) o[dt] = o_small[dt] = zero16();
+#pragma unroll 1
+        for (int kb = 0; kb <= min(last, blocks - 1); ++kb) {
+            const int j0 = kb * kBlock;
+            const float* krow = k + static_cast<int64_t>(min(j0 + li, sh.length - 1)) * in.kv_row;
+            v16f s = zero16();
+#pragma unroll 1
+            for (int f = 0; f < 32; ++f) s = mfma(krow[32 * lh + f], qrow[32 * lh + f], s);
+            float bmax = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int j = j0 + block_row(r, lh);
+                s[r] = (j > query || j >= sh.length) ? -INFINITY : s[r] * sh.inv_scale;
+                bmax = fmaxf(bmax, s[r]);
+            }
+            const float mnew = fmaxf(m, halves_max(bmax));
+            const float alpha = mnew == -INFINITY ? 1.f : __expf(m - mnew);
+            float bsum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = s[r] == -INFINITY ? 0.f : __expf(s[r] - mnew);
+                bsum += s[r];
+            }
+            l = l * alpha + halves_sum(bsum);
+            m = mnew;
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                const int row = j0 + block_row(t, lh);
+                const float* vrow = v + static_cast<int64_t>(min(row, sh.length - 1)) * in.kv_row + li;
+                o[0] = mfma(row < sh.length ? vrow[0] : 0.f, s[t], o[0]);
+                o[1] = mfma(row < sh.length ? vrow[32] : 0.f, s[t], o[1]);
+            }
+        }
+    }
+    // o[dt][r] = O^T[32 dt + block_row(r, lh)][query li]
+    if (query < sh.length) {
+        const float inv = 1.f / l;
+        float* dst = out + (static_cast<int64_t>(b) * sh.length + query) * sh.out_row + h * kD;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                v4f x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = (o[dt][r + e] + o_small[dt][r + e]) * inv;
+                *reinterpret_cast<v4f*>(dst + 32 * dt + block_row(r, lh)) = x;
+            }
+        if (lse != nullptr && lh == 0) lse[static_cast<int64_t>(bh) * sh.length + query] = m + logf(l);
+    }
+}
+
 // ---- backward ----------------------------------------------------------------------------
 //
 // One launch holds both kinds of workgroup: first the dK / dV groups (a key block each, the longer
@@ -362,6 +618,25 @@ __device__ __forceinline__ float row_delta(const float (&g)[32], const float (&o
 #pragma unroll
     for (int t = 0; t < 32; ++t) part += g[t] * o[t];
     return halves_sum(part);
+}
+
+// A row's log-sum-exp L as P = exp(S - L) takes it: exp2(S log2(e) - at) times `factor`, which holds what
+// L log2(e) rounded off (at |L| of 7 as much as 3e-7 of every P of the row), with no more operations an
+// element than exp(S - L).
+struct RowScale {
+    float at, factor;
+};
+constexpr float kLog2e = 1.44269504088896341f;
+constexpr float kLog2eRest = 1.92596299e-8f;  // log2(e) - kLog2e
+
+__device__ __forceinline__ RowScale row_scale(float lse) {
+    const float at = lse * kLog2e;
+    const float rest = fmaf(lse, kLog2eRest, fmaf(lse, kLog2e, -at));
+    return {at, fabsf(lse) < 1e30f ? __builtin_amdgcn_exp2f(-rest) : 1.f};
+}
+
+__device__ __forceinline__ float row_probability(float s, float inv_scale, float at, float factor) {
+    return __builtin_amdgcn_exp2f(fmaf(s, inv_scale * kLog2e, -at)) * factor;
 }
 
 // The dQ group `group`: lds holds 7 tiles.
@@ -393,7 +668,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     part_load(qpart, q, i0, sh.length, sh.row, wave, lane);
     part_load(gpart, go, i0, sh.length, sh.out_row, wave, lane);
     part_load(opart, o, i0, sh.length, sh.out_row, wave, lane);
-    const float row_lse = query < sh.length ? lse[static_cast<int64_t>(bh) * sh.length + query] : 0.f;
+    const RowScale scale = row_scale(query < sh.length ? lse[static_cast<int64_t>(bh) * sh.length + query] : 0.f);
     if (wave <= qb) {
         tile_load(kload, k, wave * kBlock, sh.length, sh.row, lane);
         tile_load(vload, v, wave * kBlock, sh.length, sh.row, lane);
@@ -429,7 +704,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
         {
             float kreg[32];
             lds_half_row(kreg, tile, li, lh);
-            s = dot_rows(kreg, qreg);  // the forward's product, term for term
+            s = dot_rows(kreg, qreg);
         }
         if (kb + kWaves <= qb) {  // the next block's loads run while this block finishes
             tile_load(kload, k, j0 + kWaves * kBlock, sh.length, sh.row, lane);
@@ -440,7 +715,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
         for (int r = 0; r < 16; ++r) {
             const int key = j0 + block_row(r, lh);
             const bool live = key <= query && key < sh.length && query < sh.length;
-            const float p = live ? __expf(s[r] * sh.inv_scale - row_lse) : 0.f;
+            const float p = live ? row_probability(s[r], sh.inv_scale, scale.at, scale.factor) : 0.f;
             s[r] = p * (dp[r] - dl) * sh.inv_scale;
         }
         // dQ[i][d] += sum_j dS[i][j] K[j][d]: A = dS (lane li: query li), B = K (feature 32 dt + li)
@@ -458,7 +733,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     store_tile_sum(dqkv + tok0 * sh.row + h * kD, tiles, i0, sh.length, sh.row, wave, lane);
 }
 
-// The dK / dV group `group`: lds holds 9 tiles and 2 x 4 rows of 32.
+// The dK / dV group `group`: lds holds 9 tiles and 3 x 4 rows of 32.
 __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, float* __restrict__ dqkv,
                                           const float* __restrict__ dout, const float* __restrict__ qkv,
                                           const float* __restrict__ out, const float* __restrict__ lse,
@@ -466,7 +741,8 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     float* tiles = lds;                        // each wave's Q (O first) and dO tiles; the first holds K at the start
     float* vtile = lds + 2 * kWaves * kTile;   // the key block's V
     float (*lses)[kBlock] = reinterpret_cast<float (*)[kBlock]>(vtile + kTile);
-    float (*deltas)[kBlock] = lses + kWaves;
+    float (*factors)[kBlock] = lses + kWaves;  // of the rows' RowScale, as lses
+    float (*deltas)[kBlock] = factors + kWaves;
     const int blocks = (sh.length + kBlock - 1) / kBlock;
     const int units = sh.batch * sh.heads;
     const int bh = group % units;
@@ -511,7 +787,11 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     const auto block_products = [&](int i0) {
         tile_store(qtile, oload, lane);  // O first, for the rows' delta (the previous block's reads are done)
         tile_store(gtile, gload, lane);
-        if (lane < kBlock) lses[wave][lane] = lload;
+        if (lane < kBlock) {
+            const RowScale scale = row_scale(lload);
+            lses[wave][lane] = scale.at;
+            factors[wave][lane] = scale.factor;
+        }
         wave_sync();
         {
             float greg[32], oreg[32];
@@ -542,7 +822,7 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
             const int local = block_row(r, lh);
             const int query = i0 + local;
             const bool live = key <= query && query < sh.length && key < sh.length;
-            p[r] = live ? __expf(s[r] * sh.inv_scale - lses[wave][local]) : 0.f;
+            p[r] = live ? row_probability(s[r], sh.inv_scale, lses[wave][local], factors[wave][local]) : 0.f;
             s[r] = p[r] * (dp[r] - deltas[wave][local]) * sh.inv_scale;
         }
         // dV[j][d] += sum_i P[i][j] dO[i][d], dK[j][d] += sum_i dS[i][j] Q[i][d]:
@@ -575,7 +855,7 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     store_tile_sum(dstk + sh.heads * kD, tiles + kWaves * kTile, j0, sh.length, sh.row, wave, lane);
 }
 
-constexpr int kBackwardLds = (2 * kWaves + 1) * kTile + 2 * kWaves * kBlock;  // the dK / dV group's, the larger
+constexpr int kBackwardLds = (2 * kWaves + 1) * kTile + 3 * kWaves * kBlock;  // the dK / dV group's, the larger
 
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_backward_kernel(float* __restrict__ dqkv,
                                                                             const float* __restrict__ dout,
@@ -720,6 +1000,20 @@ int check_shape(int dtype, int64_t batch, int64_t length, int64_t heads, int64_t
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 template <bool Exact> int launch_forward(float* out, float* lse, const HeadViews& in, const AttentionShape& sh) {
+    if constexpr (!Exact) {
+        // One of these workgroups is a longer chain (1.8 us a key block, where the four waves of the f32 kernel share
+        // a query block's keys), so they need more than one a CU, and more queries than the f32 kernel's block. f32 /
+        // pieces, us, and workgroups of the latter: 8 x 1024 x 12 154 / 100 (768), 16 x 300 x 16 63 / 41 (768),
+        // 8 x 512 x 12 48 / 38 (384), 128 x 33 x 8 27 / 20 (1024), 3 x 1024 x 12 65 / 64 (288); 4 x 1024 x 8
+        // 58 / 62 (256), 8 x 250 x 8 12 / 20 (128), 32 x 128 x 4 9.0 / 12.8 (128), 256 x 32 x 8 26.6 / 28.2 (2048).
+        const int64_t wide = int64_t{sh.batch} * sh.heads * ((sh.length + kWide - 1) / kWide);
+        if (sh.length > kBlock && wide > compute_units()) {
+            hipLaunchKernelGGL(attention_forward_pieces_kernel, dim3(static_cast<uint32_t>(wide)), dim3(kWaves * 64), 0, stream(),
+                               out, lse, in, sh);
+            KD_LAUNCH_CHECK();
+            return KD_OK;
+        }
+    }
     const int64_t blocks = (sh.length + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(attention_forward_kernel<Exact>, dim3(static_cast<uint32_t>(sh.batch * sh.heads * blocks)), dim3(kWaves * 64),
                        0, stream(), out, lse, in, sh);

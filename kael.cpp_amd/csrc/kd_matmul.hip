@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "kd_internal.h"
+#include "kd_pieces.h"
 
 namespace kd {
 
@@ -111,27 +112,7 @@ __device__ __forceinline__ void tile_of(int64_t id, int64_t tiles_m, int64_t til
 // repeat the last one and are not stored, so ragged sizes cost no tests in the loop. Element
 // alignment is all that the loads need (a global 16-byte load takes any 4-byte address).
 
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-typedef float f2v __attribute__((ext_vector_type(2)));
 typedef float f4any __attribute__((ext_vector_type(4), aligned(4)));
-
-__device__ __forceinline__ void split_pieces(const float (&x)[8], bf8& hi, bf8& mid, bf8& lo) {
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-        const bf2 h = __builtin_convertvector((f2v{x[e], x[e + 1]}), bf2);
-        const f2v r{x[e] - static_cast<float>(h[0]), x[e + 1] - static_cast<float>(h[1])};
-        const bf2 m = __builtin_convertvector(r, bf2);
-        const f2v q{r[0] - static_cast<float>(m[0]), r[1] - static_cast<float>(m[1])};
-        const bf2 l = __builtin_convertvector(q, bf2);
-        hi[e] = h[0];
-        hi[e + 1] = h[1];
-        mid[e] = m[0];
-        mid[e + 1] = m[1];
-        lo[e] = l[0];
-        lo[e + 1] = l[1];
-    }
-}
 
 // The LDS image of Rows (m of A, n of B) x BK of one operand. The 64 bytes after each group keep the
 // writes of a K-contiguous operand, whose neighbouring lanes hold neighbouring groups, off one

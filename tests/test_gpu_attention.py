@@ -50,6 +50,39 @@ def test_attention_matches_the_oracle(kdb, oracle, shape):
         np.testing.assert_array_equal(g, a)
 
 
+# More than one workgroup of 128 queries per CU: the forward's products run in bf16 pieces. Around the blocks of
+# 32 keys and the tiles of 128 queries.
+WIDE = [(33, 33, 8), (11, 128, 24), (22, 130, 6), (10, 257, 9), (3, 385, 22)]
+
+
+@pytest.mark.parametrize("shape", WIDE, ids=["x".join(map(str, s)) for s in WIDE])
+def test_attention_over_many_queries(kdb, oracle, shape):
+    test_attention_matches_the_oracle(kdb, oracle, shape)
+
+
+def test_values_that_pieces_cannot_hold(kdb):
+    """Infinities, NaN and values near the largest: what the f32 kernel gives for each batch alone. Finite values
+    differ by the rounding of the two kernels (each within 2e-6 of the mathematics at these sizes)."""
+    b, t, h = 13, 300, 8
+    qkv = np.random.default_rng(4).normal(size=(b, t, 3, h, 64)).astype(np.float32)
+    qkv[1, 40, 1, 2, 5] = np.inf  # a key: its scores are infinite, of either sign
+    qkv[2, 130, 2, 3, 7] = np.inf  # values
+    qkv[3, 299, 2, 0, 1] = -np.inf
+    qkv[4, 150, 0, 1, 9] = np.nan  # a query
+    qkv[5, 200, 2, 4, 60] = 3.4e38  # finite, infinite as one bf16
+    qkv[6, 3, 1, 7, 33] = -3e30
+    dev, width = kdb.to_device(qkv), h * 64
+    out, lse = kdb.empty((b, t, width), np.float32), kdb.empty((b, h, t), np.float32)
+    kdb.call("causal_attention", kd.F32, out.ptr, lse.ptr, dev.ptr, b, t, h, 64)
+    out, lse = out.numpy(), lse.numpy()
+    for i in range(8):
+        one = kdb.to_device(qkv[i])
+        want, want_lse = kdb.empty((t, width), np.float32), kdb.empty((h, t), np.float32)
+        kdb.call("causal_attention", kd.F32, want.ptr, want_lse.ptr, one.ptr, 1, t, h, 64)
+        for got, w in ((out[i], want.numpy()), (lse[i], want_lse.numpy())):
+            np.testing.assert_allclose(got, w, rtol=1e-5, atol=4e-6)
+
+
 def test_attention_rejects_unsupported_shapes(kdb):
     x = kdb.to_device(np.zeros(3 * 64 * 4, np.float32))
     with pytest.raises(kd.KdError):
