@@ -11,7 +11,7 @@ section carries kael's CPU path on the same workload as its cpu_baseline.
 Timing: W untimed warm-up steps, then K steps bracketed by kd_synchronize(); the kernel time comes
 from HIP events recorded on the backend stream (the stream every kd_* launch uses). The GPU's
 clocks ramp up from idle over tens of milliseconds (the 4096^3 matmul measures ~127 TFLOP/s after
-5 warm-up steps and ~140 after 50), so W defaults to 50 for the headline; the secondary sections,
+5 warm-up steps and ~140 after 50 on the f32 matrix cores), so W defaults to 50 for the headline; the secondary sections,
 whose steps take microseconds, warm up for at least MIN_WARMUP_S of steps.
 The CPU baseline is kael's own CPU matmul (oracle/_ref, built from the reference sources,
 threaded over the host cores) on a bounded sample, reported beside the GPU figure.
@@ -39,11 +39,11 @@ import kd  # noqa: E402
 FP32_MFMA_PEAK_TFLOPS = 157.3   # MI355X dense FP32 matrix (AMD spec)
 FP64_MFMA_PEAK_TFLOPS = 78.6    # MI355X dense FP64 matrix (AMD spec)
 HBM_PEAK_GBPS = 8000.0          # MI355X HBM3E
-# HBM bytes one 4096^3 launch of the headline kernel (mfma_f32_trans_kernel<false,false>) moves,
-# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (198 999 KiB and 65 536 KiB per dispatch), scaled
+# HBM bytes one 4096^3 launch of the headline kernel (pieces_kernel on 256 x 128 tiles) moves,
+# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (327 823 KiB and 65 536 KiB per dispatch), scaled
 # by the factors a plain 256 MiB copy gives the same counters (x2.0 fetch, x1.0 write). The PMC
 # runs and commands are kept in profiles/.
-MATMUL_4096_TRAFFIC_BYTES = (2 * 198999 + 65536) * 1024
+MATMUL_4096_TRAFFIC_BYTES = (2 * 327823 + 65536) * 1024
 
 
 class Timer:
