@@ -620,24 +620,10 @@ __device__ __forceinline__ float row_delta(const float (&g)[32], const float (&o
     return halves_sum(part);
 }
 
-// A row's log-sum-exp L as P = exp(S - L) takes it: exp2(S log2(e) - at) times `factor`, which holds what
-// L log2(e) rounded off (at |L| of 7 as much as 3e-7 of every P of the row), with no more operations an
-// element than exp(S - L).
-struct RowScale {
-    float at, factor;
-};
-constexpr float kLog2e = 1.44269504088896341f;
-constexpr float kLog2eRest = 1.92596299e-8f;  // log2(e) - kLog2e
-
-__device__ __forceinline__ RowScale row_scale(float lse) {
-    const float at = lse * kLog2e;
-    const float rest = fmaf(lse, kLog2eRest, fmaf(lse, kLog2e, -at));
-    return {at, fabsf(lse) < 1e30f ? __builtin_amdgcn_exp2f(-rest) : 1.f};
-}
-
-__device__ __forceinline__ float row_probability(float s, float inv_scale, float at, float factor) {
-    return __builtin_amdgcn_exp2f(fmaf(s, inv_scale * kLog2e, -at)) * factor;
-}
+// P from a row's log-sum-exp. The score and the log-sum-exp take the same steps (1 / 8 is exact), so that the exponent
+// is 0 and P exactly 1 for a key that alone makes up its row, whatever the score's size: a constant's rounding on one
+// side of the difference alone would grow with it.
+__device__ __forceinline__ float row_probability(float s, float inv_scale, float lse) { return __expf(s * inv_scale - lse); }
 
 // The dQ group `group`: lds holds 7 tiles.
 __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, float* __restrict__ dqkv,
@@ -668,7 +654,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     part_load(qpart, q, i0, sh.length, sh.row, wave, lane);
     part_load(gpart, go, i0, sh.length, sh.out_row, wave, lane);
     part_load(opart, o, i0, sh.length, sh.out_row, wave, lane);
-    const RowScale scale = row_scale(query < sh.length ? lse[static_cast<int64_t>(bh) * sh.length + query] : 0.f);
+    const float row_lse = query < sh.length ? lse[static_cast<int64_t>(bh) * sh.length + query] : 0.f;
     if (wave <= qb) {
         tile_load(kload, k, wave * kBlock, sh.length, sh.row, lane);
         tile_load(vload, v, wave * kBlock, sh.length, sh.row, lane);
@@ -715,7 +701,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
         for (int r = 0; r < 16; ++r) {
             const int key = j0 + block_row(r, lh);
             const bool live = key <= query && key < sh.length && query < sh.length;
-            const float p = live ? row_probability(s[r], sh.inv_scale, scale.at, scale.factor) : 0.f;
+            const float p = live ? row_probability(s[r], sh.inv_scale, row_lse) : 0.f;
             s[r] = p * (dp[r] - dl) * sh.inv_scale;
         }
         // dQ[i][d] += sum_j dS[i][j] K[j][d]: A = dS (lane li: query li), B = K (feature 32 dt + li)
@@ -733,7 +719,7 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     store_tile_sum(dqkv + tok0 * sh.row + h * kD, tiles, i0, sh.length, sh.row, wave, lane);
 }
 
-// The dK / dV group `group`: lds holds 9 tiles and 3 x 4 rows of 32.
+// The dK / dV group `group`: lds holds 9 tiles and 2 x 4 rows of 32.
 __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, float* __restrict__ dqkv,
                                           const float* __restrict__ dout, const float* __restrict__ qkv,
                                           const float* __restrict__ out, const float* __restrict__ lse,
@@ -741,8 +727,7 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     float* tiles = lds;                        // each wave's Q (O first) and dO tiles; the first holds K at the start
     float* vtile = lds + 2 * kWaves * kTile;   // the key block's V
     float (*lses)[kBlock] = reinterpret_cast<float (*)[kBlock]>(vtile + kTile);
-    float (*factors)[kBlock] = lses + kWaves;  // of the rows' RowScale, as lses
-    float (*deltas)[kBlock] = factors + kWaves;
+    float (*deltas)[kBlock] = lses + kWaves;
     const int blocks = (sh.length + kBlock - 1) / kBlock;
     const int units = sh.batch * sh.heads;
     const int bh = group % units;
@@ -787,11 +772,7 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     const auto block_products = [&](int i0) {
         tile_store(qtile, oload, lane);  // O first, for the rows' delta (the previous block's reads are done)
         tile_store(gtile, gload, lane);
-        if (lane < kBlock) {
-            const RowScale scale = row_scale(lload);
-            lses[wave][lane] = scale.at;
-            factors[wave][lane] = scale.factor;
-        }
+        if (lane < kBlock) lses[wave][lane] = lload;
         wave_sync();
         {
             float greg[32], oreg[32];
@@ -822,7 +803,7 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
             const int local = block_row(r, lh);
             const int query = i0 + local;
             const bool live = key <= query && query < sh.length && key < sh.length;
-            p[r] = live ? row_probability(s[r], sh.inv_scale, lses[wave][local], factors[wave][local]) : 0.f;
+            p[r] = live ? row_probability(s[r], sh.inv_scale, lses[wave][local]) : 0.f;
             s[r] = p[r] * (dp[r] - deltas[wave][local]) * sh.inv_scale;
         }
         // dV[j][d] += sum_i P[i][j] dO[i][d], dK[j][d] += sum_i dS[i][j] Q[i][d]:
@@ -855,7 +836,7 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     store_tile_sum(dstk + sh.heads * kD, tiles + kWaves * kTile, j0, sh.length, sh.row, wave, lane);
 }
 
-constexpr int kBackwardLds = (2 * kWaves + 1) * kTile + 3 * kWaves * kBlock;  // the dK / dV group's, the larger
+constexpr int kBackwardLds = (2 * kWaves + 1) * kTile + 2 * kWaves * kBlock;  // the dK / dV group's, the larger
 
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_backward_kernel(float* __restrict__ dqkv,
                                                                             const float* __restrict__ dout,

@@ -21,7 +21,8 @@ import pytest
 
 import kd
 import support
-from test_oracle_attention import cached_module, close, inputs, module_grads, oracle_attention, oracle_cached, qkv_views
+from test_oracle_attention import (cached_module, close, inputs, module_grads, numpy_attention, oracle_attention,
+                                   oracle_cached, qkv_views)
 
 pytestmark = pytest.mark.gpu
 
@@ -81,6 +82,51 @@ def test_values_that_pieces_cannot_hold(kdb):
         kdb.call("causal_attention", kd.F32, want.ptr, want_lse.ptr, one.ptr, 1, t, h, 64)
         for got, w in ((out[i], want.numpy()), (lse[i], want_lse.numpy())):
             np.testing.assert_allclose(got, w, rtol=1e-5, atol=4e-6)
+
+
+def scores_of_size(b, t, h, size):
+    """Operands whose scores are `size` times a permutation of 1 / t .. 1 in each head (to f32's rounding): from about
+    20 t on, one key makes up each row."""
+    rng = np.random.default_rng(b + t + h)
+    qkv, dout = rng.uniform(-1, 1, (b, t, 3, h, 64)), rng.uniform(-1, 1, (b, t, h * 64))
+    along = rng.normal(size=(b, 1, h, 64))
+    along *= np.sqrt(8 * abs(size) / (along ** 2).sum(-1, keepdims=True))
+    order = rng.permuted(np.tile(np.arange(1, t + 1) / t, (b, h, 1)), axis=-1).transpose(0, 2, 1)[..., None]
+    qkv[:, :, 0], qkv[:, :, 1] = along, along * order * np.sign(size)
+    return qkv.astype(np.float32), dout.astype(np.float32)
+
+
+def check_large_scores(kdb, qkv, dout, size):
+    """Against the mathematics in float64. A score is rounded by some 3e-7 of its size, which moves P by that share of
+    P (1 - P), twice with the row's sum; the row's log-sum-exp L is rounded by up to 2^-24 |L|, but by no more than
+    the sum of the keys beside the largest. So a key that alone makes up its row has P = 1 at any score. The other
+    sums run over the 64 features and the keys, a few roundings of 2^-24 of the running sum for each term: below 1e-5
+    of the sum of magnitudes."""
+    b, t, _, h, _ = qkv.shape
+    got = device_attention(kdb, qkv.reshape(b, t, -1), dout, b, t, h)[2]
+    assert np.isfinite(got).all()
+    got = got.reshape(b, t, 3, h, 64)
+    x = qkv.astype(np.float64)
+    q, k, v = (x[:, :, i].transpose(0, 2, 1, 3) for i in range(3))
+    go = dout.astype(np.float64).reshape(b, t, h, 64).transpose(0, 2, 1, 3)
+    s = np.where(np.triu(np.ones((t, t), bool), 1), -np.inf, q @ k.transpose(0, 1, 3, 2) / 8)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    o, rest = p @ v, 1 - p
+    p_err = p * (1e-5 + 6e-7 * abs(size) * rest + np.minimum(rest, 1.2e-7 * abs(size)))
+    term = p_err * (np.abs(go) @ np.abs(v).transpose(0, 1, 3, 2) + (np.abs(go) * np.abs(o)).sum(-1, keepdims=True)) / 8
+    want = numpy_attention(qkv.reshape(b, t, -1), dout, b, t, h, 64)[2].reshape(b, t, 3, h, 64)
+    bounds = term @ np.abs(k), term.transpose(0, 1, 3, 2) @ np.abs(q), p_err.transpose(0, 1, 3, 2) @ np.abs(go)
+    for i, (bound, what) in enumerate(zip(bounds, "qkv")):
+        err, bound = np.abs(got[:, :, i] - want[:, :, i]), bound.transpose(0, 2, 1, 3)
+        assert (err <= bound + 1e-30).all(), (what, (err / (bound + 1e-30)).max())
+
+
+@pytest.mark.parametrize("size", [10, 100, -100, 1.2e3, -1.2e4, 1.2e6, -1.2e6, 1.2e8, -1.2e9, 1.2e10, 1e12, -1e12])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 37, 3), (1, 300, 1)], ids=["1x1x1", "2x37x3", "1x300x1"])
+def test_gradients_at_large_scores(kdb, shape, size):
+    """P is exactly 1 where one key makes up the row (row 0 of every sequence, one dominating key), at any score."""
+    check_large_scores(kdb, *scores_of_size(*shape, size), size)
 
 
 def test_attention_rejects_unsupported_shapes(kdb):
