@@ -10,7 +10,9 @@
 //          cores accumulated in f32; tiles from 64x64 to 256x128 and a K split chosen by size.
 //   small  f32, few tiles and a short K (C1's 512^3, small MLP layers): 32x32 tiles, one workgroup of 16
 //          waves each, the waves splitting K and reading their operands straight from global memory,
-//          their partial tiles added in LDS in wave order.
+//          their partial tiles added in LDS in wave order. Many batches of tiles that fill less than 64x64 too.
+//   rowdot f32, at most 4 columns: a wave per output row.
+//   skinny f32, at most 8 rows and a short K: a wave per 256 columns and a quarter of K.
 //   parts  f32, split-K partials for the GPT-2 engine's short prompts.
 //   general f32 operands whose strides pieces cannot address, on the f32 matrix cores.
 //   f64    64x64 tiles on the FP64 matrix cores.
@@ -749,13 +751,87 @@ __global__ __launch_bounds__(kThreads) void split_sum_flat_kernel(const float* _
     }
 }
 
-// ---- rowdot family (f32, N <= 4 over more batches than a grid's second dimension holds) -----------
+// ---- skinny family (f32, few rows) ------------------------------------------------------------
+
+constexpr int kSkinnyMaxM = 8;
+constexpr int kSkinnyCols = 256;  // 64 lanes x 4 columns
+
+// Rows [0, M) x 256 columns: the four waves take interleaved k, then combine in LDS in wave order. Nothing is staged,
+// so that a product that is its traffic runs at memory's rate: 4096 x (1 x 64 x 1024) takes 182 us (5.9 TB/s) where
+// the 64x64 tiles take 510, 65535 x (1 x 16 x 64) 107 where they take 315.
+template <int MT, bool BVec>
+__global__ __launch_bounds__(kThreads) void skinny_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                          float* __restrict__ out, MatmulArgs p) {
+    __shared__ float red[4][MT][kSkinnyCols];
+    const int lane = threadIdx.x % 64;
+    const int wave = threadIdx.x / 64;
+    const int64_t batch = blockIdx.y;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kSkinnyCols + lane * 4;
+    a += batch_offset(p, batch, p.sa.b, p.ha);
+    b += batch_offset(p, batch, p.sb.b, p.hb);
+
+    float total[MT][4];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) total[m][c] = 0.f;
+
+    // a sum per 64 of K, so that a long one rounds less (K = 256: 1.5e-7 of the result, 2-norm, in one sum)
+    for (int64_t k0 = wave; k0 < p.K; k0 += 64) {
+        const int64_t end = std::min<int64_t>(p.K, k0 + 64);
+        float acc[MT][4];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[m][c] = 0.f;
+        for (int64_t k = k0; k < end; k += 4) {
+            float bv[4];
+            if (BVec && n0 + 3 < p.N) {
+                const float4 v = *reinterpret_cast<const float4*>(b + k * p.sb.r + n0);
+                bv[0] = v.x;
+                bv[1] = v.y;
+                bv[2] = v.z;
+                bv[3] = v.w;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) bv[c] = n0 + c < p.N ? b[k * p.sb.r + (n0 + c) * p.sb.c] : 0.f;
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                if (m < p.M) {
+                    const float av = a[m * p.sa.r + k * p.sa.c];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[m][c] += av * bv[c];
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) total[m][c] += acc[m][c];
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) red[wave][m][lane * 4 + c] = total[m][c];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < MT * kSkinnyCols; idx += kThreads) {
+        const int m = idx / kSkinnyCols;
+        const int col = idx % kSkinnyCols;
+        const int64_t n = static_cast<int64_t>(blockIdx.x) * kSkinnyCols + col;
+        if (m >= p.M || n >= p.N) continue;
+        const float v = ((red[0][m][col] + red[1][m][col]) + red[2][m][col]) + red[3][m][col];
+        out[batch_offset(p, batch, p.so.b, p.ho) + m * p.so.r + n * p.so.c] = plus_bias(v, p.bias, n);
+    }
+}
+
+// ---- rowdot family (f32, few columns) ---------------------------------------------------------------
 
 constexpr int kRowdotMaxN = 4;
 constexpr int64_t kGridBatches = 65535;
 
-// One wave per (batch, row), all in the grid's first dimension; lanes stride along K. Up to kGridBatches
-// batches the small tiles and the pieces are quicker (4096 x 4096 x 4: 22 us against 116 here).
+// One wave per (batch, row), all in the grid's first dimension; lanes stride along K. 65535 x (1 x 256 x 1) takes 24 us
+// here and 500 on the small tiles, 1 x 1024 x 1 3.1 and 6.7 on the pieces; 1 x 50257 x 1, a serial chain, 107 and 21.
 template <bool AVec>
 __global__ __launch_bounds__(kThreads) void rowdot_kernel(const float* __restrict__ a, const float* __restrict__ b,
                                                           float* __restrict__ out, MatmulArgs p) {
@@ -888,15 +964,16 @@ int launch_status() {
 // throughput), `end_us` the prologue and epilogue that nothing overlaps. Measured on 2^20-2^24-output
 // products with K of 256 to 50257, uniform inputs.
 struct Tiling {
-    int tm, tn, bk, per_cu;
+    int tm, tn, bk, per_cu, most_splits;
     double alone_us, crowded_us, end_us;
 };
 constexpr Tiling kTilings[] = {
-    {256, 128, 16, 1, 2.30, 2.48, 7.0},  // 8 waves of 64 x 64: the best rate (4096^3: 636 us; 128 x 128 below 662)
-    {128, 128, 16, 2, 1.35, 1.29, 5.0},  // two workgroups hide one another's ends (999 x 768 x 50257: 427 us; above 468)
-    {128, 128, 32, 1, 1.10, 1.37, 8.0},  // one workgroup per CU (2048^3: 94 us; 999 x 768 x 3072: 33)
-    {128, 64, 32, 2, 0.80, 0.76, 5.5},   // 1024 x 4096 x 256 in 8 splits: 21 us (128 x 128: 27)
-    {64, 64, 32, 3, 0.54, 0.44, 5.0},    // grids of a few hundred tiles (4096 x 256 x 256: 9.4 us; 128 x 128: 15)
+    {256, 128, 16, 1, 64, 2.30, 2.48, 7.0},  // 8 waves of 64 x 64: the best rate (4096^3: 636 us; 128 x 128 below 662)
+    {128, 128, 16, 2, 64, 1.35, 1.29, 5.0},  // two workgroups hide one another's ends (999 x 768 x 50257: 427 us; above 468)
+    {128, 128, 32, 1, 64, 1.10, 1.37, 8.0},  // one workgroup per CU (2048^3: 94 us; 999 x 768 x 3072: 33)
+    {128, 64, 32, 2, 64, 0.80, 0.76, 5.5},   // 1024 x 4096 x 256 in 8 splits: 21 us (128 x 128: 27)
+    {64, 64, 32, 3, 64, 0.54, 0.44, 5.0},    // grids of a few hundred tiles (4096 x 256 x 256: 9.4 us; 128 x 128: 15)
+    {64, 64, 16, 5, 1, 0.80, 0.52, 4.6},    // a short K over many tiles, whose ends five workgroups hide (4096 x (40 x 16 x 1024): 314 us; above 613): no splits
 };
 constexpr int kTilingCount = sizeof kTilings / sizeof kTilings[0];
 
@@ -909,7 +986,8 @@ void launch_pieces(int tiling, dim3 grid, const float* a, const float* b, float*
     case 1: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 128, 128, 4, 2, 16, 4>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
     case 2: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 128, 128, 4, 2, 32, 2>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
     case 3: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 128, 64, 4, 2, 32, 4>), grid, dim3(512), 0, s, a, b, out, p, k_split, split_o); break;
-    default: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 64, 64, 2, 2, 32, 3>), grid, dim3(256), 0, s, a, b, out, p, k_split, split_o); break;
+    case 4: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 64, 64, 2, 2, 32, 3>), grid, dim3(256), 0, s, a, b, out, p, k_split, split_o); break;
+    default: hipLaunchKernelGGL((pieces_kernel<AK, BKc, 64, 64, 2, 2, 16, 5>), grid, dim3(256), 0, s, a, b, out, p, k_split, split_o); break;
     }
 }
 
@@ -931,10 +1009,11 @@ Plan plan_pieces(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t most_
     for (int c = 0; c < kTilingCount; ++c) {
         const Tiling& tl = kTilings[c];
         const int64_t tiles = (M + tl.tm - 1) / tl.tm * ((N + tl.tn - 1) / tl.tn) * batches;
+        const int64_t most = std::min<int64_t>(most_splits, tl.most_splits);
         int64_t last_k = 0;
         for (const int want : kSplits) {
             // at least 64 deep, at most four rounds of workgroups, and partials of at most 256 MiB
-            if (want > 1 && (want > most_splits || K < want * 64 || tiles * want > 4 * cus * tl.per_cu || want * outputs > 0x1p26)) break;
+            if (want > 1 && (want > most || K < want * 64 || tiles * want > 4 * cus * tl.per_cu || want * outputs > 0x1p26)) break;
             const int64_t k_split = ((K + want - 1) / want + 31) / 32 * 32;
             if (k_split == last_k) continue;
             last_k = k_split;
@@ -995,18 +1074,7 @@ int launch_plan(const Plan& plan, const float* a, const float* b, float* out, co
     return launch_status();
 }
 
-int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
-    // the batches fold into M when they share B and lie back to back in A and the output
-    if (p.batches > 1 && p.heads == 1 && p.sb.b == 0 && p.sa.b == p.M * p.sa.r && p.so.b == p.M * p.so.r &&
-        p.M * p.batches < (int64_t{1} << 31) - 256) {
-        p.M *= p.batches;
-        p.batches = 1;
-    }
-    // A graph would hold on to partials in the shared workspace, which a later call may free to grow it, and
-    // growing it is no call to make under capture: a captured product is not split.
-    hipStreamCaptureStatus captured = hipStreamCaptureStatusNone;
-    if (stream() != nullptr) KD_HIP(hipStreamIsCapturing(stream(), &captured));
-    const Plan plan = plan_pieces(p.M, p.N, p.K, p.batches, captured == hipStreamCaptureStatusNone ? 64 : 1);
+int matmul_pieces(const float* a, const float* b, float* out, const MatmulArgs& p, const Plan& plan) {
     if (plan.splits == 1) return launch_plan(plan, a, b, out, p, 0);
     Workspace ws;  // held until the sum is enqueued
     const int64_t per = p.M * p.N;
@@ -1019,39 +1087,115 @@ int matmul_pieces(const float* a, const float* b, float* out, MatmulArgs p) {
     return launch_split_sum(static_cast<const float*>(ws.ptr), out, p, plan.splits);
 }
 
-int matmul_f32(const float* a, const float* b, float* out, const MatmulArgs& p) {
-    const int cus = compute_units();
-    if (p.batches > kGridBatches) {
-        if (p.N > kRowdotMaxN) return fail(KD_E_INVALID, "kd_matmul: too many batches");
-        const bool avec = p.sa.c == 1 && p.sa.r % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && aligned16(a);
-        const dim3 grid(static_cast<uint32_t>((p.batches * p.M + 3) / 4));
-        if (avec) hipLaunchKernelGGL((rowdot_kernel<true>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
-        else hipLaunchKernelGGL((rowdot_kernel<false>), grid, dim3(kThreads), 0, stream(), a, b, out, p);
+// ---- choosing the family ------------------------------------------------------------------------
+//
+// Estimates in us beside plan_pieces', fitted to 3300 products of 1 to 40 rows or 1 to 16 columns, 1 to 65535 batches
+// and K of 8 to 4096, each family on each of them (half of the estimates within 8 %, nine tenths within 30 %). The
+// family that they choose took at most 1.06 times the quickest's time for nine tenths of the products.
+
+// A launch, a chain of loads along K, and the waves (each a row of A and N columns of B).
+double rowdot_us(const MatmulArgs& p, bool avec) {
+    const double n = static_cast<double>(p.N), k = static_cast<double>(p.K);
+    const double rows = static_cast<double>(p.batches) * static_cast<double>(p.M);
+    const double steps = std::ceil(k / (avec ? 256 : 64));
+    double chain = p.N == 1 ? (avec ? 0.16 : 0.13) : n * 0.09;
+    if (avec && p.N > 1) chain = n * (p.sb.r == 1 ? 0.18 : 0.07 + 0.09 * std::min(rows, 4.0));  // a workgroup's waves share its loads
+    const double element = avec && p.N == 1 ? 5e-7 : n * (avec && p.sb.r == 1 ? 7e-7 : 1.2e-6);
+    return 2.7 + chain * steps + rows * (2.3e-4 + k * element);
+}
+
+// A launch, the chain of k, the workgroups' LDS sums and multiplications, and B's and the output's traffic.
+double skinny_us(const MatmulArgs& p) {
+    const double m = static_cast<double>(p.M), n = static_cast<double>(p.N), k = static_cast<double>(p.K);
+    const double batches = static_cast<double>(p.batches);
+    const double groups = batches * static_cast<double>((p.N + kSkinnyCols - 1) / kSkinnyCols);
+    return 2.5 + k * (0.029 + 0.018 * m) + groups * (1.1e-4 * (p.M <= 1 ? 1 : p.M <= 4 ? 4 : 8) + 3.1e-5 * k * (m + 1)) +
+           batches * n * (k * (p.sb.c == 1 ? 4.4e-7 : 2.2e-6) + m * 3.9e-7);
+}
+
+// Up to two tiles a CU a launch and its ends, and 0.85 us per 128 of K (16 waves of 8), 2 where a CU has two. Beyond, the
+// tiles' share of a CU and their loads and stores. Small / pieces: 512^3 6.5 / 11.4 us, 256^3 4.3 / 8.3, 128 x 64 x 784
+// 2.9 / 6.0, 64 x 784 x 128 with B transposed 7.5 / 9.2, 600^3 10.3 / 14.5; 300 x 2000 x 300 18.3 / 14.0, 128 x 2048 x 128
+// 17.3 / 10.7, 400 x 768 x 768 14.4 / 13.2; 4096 x (32 x 128 x 32) 26.5 / 36, 1000 x (24 x 64 x 24) 5.9 / 8.5.
+double small_us(const MatmulArgs& p) {
+    const double gm = static_cast<double>((p.M + kSmallTile - 1) / kSmallTile), gn = static_cast<double>((p.N + kSmallTile - 1) / kSmallTile);
+    const double batches = static_cast<double>(p.batches), tiles = gm * gn * batches, k = static_cast<double>(p.K);
+    const double m = static_cast<double>(p.M), n = static_cast<double>(p.N), cus = compute_units();
+    if (tiles <= 2 * cus) return 2.0 + static_cast<double>((p.K + 127) / 128) * (tiles <= cus ? 0.85 : 2.0);
+    return 2.2 + tiles * (2.3e-3 + 2.7e-5 * k) + batches * (1.8e-7 * k * (m * gn + n * gm) + 8.4e-7 * m * n);
+}
+
+int matmul_f32(const float* a, const float* b, float* out, MatmulArgs p) {
+    enum { kRowdot, kSkinny, kSmall, kPieces, kGeneral };
+    if (p.batches > kGridBatches && p.N > kRowdotMaxN) return fail(KD_E_INVALID, "kd_matmul: too many batches");
+    // the batches fold into M when they share B and lie back to back in A and the output
+    if (p.batches > 1 && p.heads == 1 && p.sb.b == 0 && p.sa.b == p.M * p.sa.r && p.so.b == p.M * p.so.r &&
+        p.M * p.batches < (int64_t{1} << 31) - 256) {
+        p.M *= p.batches;
+        p.batches = 1;
+    }
+    const bool avec = p.sa.c == 1 && p.sa.r % 4 == 0 && p.sa.b % 4 == 0 && p.ha % 4 == 0 && aligned16(a);
+    const int64_t gm = (p.M + kSmallTile - 1) / kSmallTile, gn = (p.N + kSmallTile - 1) / kSmallTile;
+    const bool grid = p.batches <= kGridBatches;
+    int family = kGeneral;
+    double us = 0.0;
+    const auto consider = [&](int f, double estimate) {
+        if (family == kGeneral || estimate < us) {
+            family = f;
+            us = estimate;
+        }
+    };
+    // (a launch holds fewer than 2^32 threads in its first dimension)
+    if (p.N <= kRowdotMaxN && p.batches * p.M < (int64_t{1} << 26) - 4) consider(kRowdot, rowdot_us(p, avec));
+    if (grid && p.M <= kSkinnyMaxM && p.N < (int64_t{1} << 31)) consider(kSkinny, skinny_us(p));
+    const bool pieces = pieces_addressable(p);
+    const bool fits32 = p.K * std::abs(p.sa.c) < (int64_t{1} << 31) && p.K * std::abs(p.sb.r) < (int64_t{1} << 31);
+    // (what the pieces cannot take has no estimate: beyond two tiles a CU it is the general kernel's)
+    if (grid && fits32 && gm <= 65535 && gn < (int64_t{1} << 22) && (pieces || gm * gn * p.batches <= 2 * int64_t{compute_units()}))
+        consider(kSmall, small_us(p));
+    Plan plan{};
+    // Where many tiles leave the choice close the pieces' sums have fewer roundings: small tiles if a quarter quicker.
+    if (family == kSmall && pieces && gm * gn * p.batches > 2 * int64_t{compute_units()}) us *= 1.25;
+    if (pieces && (family == kGeneral || us >= 5.3)) {  // (no plan takes less)
+        // A graph would hold on to partials in the shared workspace, which a later call may free to grow it, and
+        // growing it is no call to make under capture: a captured product is not split.
+        hipStreamCaptureStatus captured = hipStreamCaptureStatusNone;
+        if (stream() != nullptr) KD_HIP(hipStreamIsCapturing(stream(), &captured));
+        plan = plan_pieces(p.M, p.N, p.K, p.batches, captured == hipStreamCaptureStatusNone ? 64 : 1);
+        consider(kPieces, plan.us);
+    }
+    switch (family) {
+    case kRowdot: {
+        const dim3 groups(static_cast<uint32_t>((p.batches * p.M + 3) / 4));
+        if (avec) hipLaunchKernelGGL((rowdot_kernel<true>), groups, dim3(kThreads), 0, stream(), a, b, out, p);
+        else hipLaunchKernelGGL((rowdot_kernel<false>), groups, dim3(kThreads), 0, stream(), a, b, out, p);
         return launch_status();
     }
-    const bool pieces = pieces_addressable(p);
-    const int64_t gm = (p.M + kSmallTile - 1) / kSmallTile;
-    const int64_t gn = (p.N + kSmallTile - 1) / kSmallTile;
-    const bool fits32 = p.K * std::abs(p.sa.c) < (int64_t{1} << 31) && p.K * std::abs(p.sb.r) < (int64_t{1} << 31);
-    if (fits32 && gm <= 65535 && gm * gn * p.batches <= 2 * int64_t{cus}) {
-        // Small tiles where they are estimated to be quicker than the pieces' best plan: a launch and its
-        // ends, and 0.85 us per 128 of K (16 waves of 8), 2 where a CU has two tiles. Measured, small /
-        // pieces: 512^3 6.5 / 11.4 us, 256^3 4.3 / 8.3, 128 x 64 x 784 2.9 / 6.0, 64 x 784 x 128 with B
-        // transposed 7.5 / 9.2, 600^3 10.3 / 14.5; 300 x 2000 x 300 18.3 / 14.0, 128 x 2048 x 128 17.3 /
-        // 10.7, 400 x 768 x 768 14.4 / 13.2.
-        const double rounds = static_cast<double>((p.K + 127) / 128);
-        const double us = 2.0 + rounds * (gm * gn * p.batches <= cus ? 0.85 : 2.0);
-        // (no plan takes less than 5.5 us)
-        if (!pieces || us < 5.5 || us < plan_pieces(p.M, p.N, p.K, p.batches).us) {
-            const dim3 grid(static_cast<uint32_t>(gn), static_cast<uint32_t>(gm), static_cast<uint32_t>(p.batches));
-            with_k_modes(p.sa.c == 1, p.sb.r == 1, [&](auto ak, auto bk) {
-                hipLaunchKernelGGL((small_kernel<decltype(ak)::value, decltype(bk)::value>), grid, dim3(kSmallWaves * 64), 0,
-                                   stream(), a, b, out, p);
-            });
-            return launch_status();
-        }
+    case kSkinny: {
+        const dim3 groups(static_cast<uint32_t>((p.N + kSkinnyCols - 1) / kSkinnyCols), static_cast<uint32_t>(p.batches));
+        const bool bvec = p.sb.c == 1 && p.sb.r % 4 == 0 && p.sb.b % 4 == 0 && p.hb % 4 == 0 && aligned16(b);
+        const auto launch = [&](auto mt) {
+            constexpr int kRows = decltype(mt)::value;
+            if (bvec) hipLaunchKernelGGL((skinny_kernel<kRows, true>), groups, dim3(kThreads), 0, stream(), a, b, out, p);
+            else hipLaunchKernelGGL((skinny_kernel<kRows, false>), groups, dim3(kThreads), 0, stream(), a, b, out, p);
+        };
+        if (p.M <= 1) launch(std::integral_constant<int, 1>{});
+        else if (p.M <= 4) launch(std::integral_constant<int, 4>{});
+        else launch(std::integral_constant<int, kSkinnyMaxM>{});
+        return launch_status();
     }
-    if (pieces) return matmul_pieces(a, b, out, p);
+    case kSmall: {
+        const dim3 groups(static_cast<uint32_t>(gn), static_cast<uint32_t>(gm), static_cast<uint32_t>(p.batches));
+        with_k_modes(p.sa.c == 1, p.sb.r == 1, [&](auto ak, auto bk) {
+            hipLaunchKernelGGL((small_kernel<decltype(ak)::value, decltype(bk)::value>), groups, dim3(kSmallWaves * 64), 0,
+                               stream(), a, b, out, p);
+        });
+        return launch_status();
+    }
+    case kPieces: return matmul_pieces(a, b, out, p, plan);
+    default: break;
+    }
+    if (!grid) return fail(KD_E_INVALID, "kd_matmul: too many batches");
     const int64_t tiles = ((p.M + kBM - 1) / kBM) * ((p.N + kBN - 1) / kBN);
     hipLaunchKernelGGL(general_f32_kernel, dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(p.batches)), dim3(kThreads),
                        0, stream(), a, b, out, p);

@@ -133,6 +133,63 @@ def test_split_batches_of_heads(kdb):
     check(out.numpy(), a, b)
 
 
+# (batches, m, k, n): few rows (one to four columns of lanes, around K's blocks of 64), few columns, tiles of 32 and 64 that
+# a batch fills in part, with short K
+MANY = [(600, 1, 16, 1024), (600, 3, 63, 257), (300, 4, 65, 255), (600, 5, 8, 1030), (700, 8, 5, 513), (520, 1, 130, 300),
+        (5000, 1, 64, 1), (5000, 2, 257, 3), (3000, 7, 6, 4), (600, 40, 16, 130), (600, 65, 15, 70), (900, 24, 64, 24),
+        (4096, 33, 17, 9), (520, 64, 33, 64)]
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("sizes", MANY, ids=["x".join(map(str, s)) for s in MANY])
+def test_many_small_batches(kdb, sizes, layout):
+    batches, m, k, n = sizes
+    rng = np.random.default_rng(sum(sizes))
+    a, b = rng.normal(size=(batches, m, k)).astype(np.float32), rng.normal(size=(batches, k, n)).astype(np.float32)
+    at, bt = layout[0] == "t", layout[1] == "t"
+    bias = rng.normal(size=n).astype(np.float32) if layout == "nt" else None
+    got = product(kdb, np.ascontiguousarray(a.transpose(0, 2, 1)) if at else a,
+                  np.ascontiguousarray(b.transpose(0, 2, 1)) if bt else b, sizes,
+                  (m * k, 1, m) if at else (m * k, k, 1), (k * n, 1, k) if bt else (k * n, n, 1), bias=bias)
+    check(got, a, b, bias)
+
+
+def test_few_rows_by_batch_and_head(kdb):
+    """A two-level batch of one-row products against rows of one shared matrix, at odd elements."""
+    rng = np.random.default_rng(5)
+    outer, heads, k, n = 150, 4, 30, 700
+    a, b = rng.normal(size=(outer, heads, k)).astype(np.float32), rng.normal(size=(heads, k, n + 1)).astype(np.float32)
+    da, db, out = kdb.to_device(a), kdb.to_device(b), kdb.empty((outer, heads, n), np.float32)
+    kdb.call("matmul_strided_heads", kd.F32, da.ptr, ctypes.c_void_p(db.ptr + 4), out.ptr, kd.MatmulSizes(outer * heads, 1, k, n),
+             kd.MatmulStrides((heads * k, k, 1), (0, n + 1, 1), (heads * n, n, 1)), kd.MatmulHeads(heads, k, k * (n + 1), n))
+    check(out.numpy()[:, :, None], a[:, :, None], np.broadcast_to(b[None, :, :, 1:], (outer, heads, k, n)))
+
+
+# The time that such products must not exceed, us: about three times what they take, which is their traffic or the launch
+# rate of their workgroups; a 64x64 tile a batch took 500, 235, 258 and 275.
+@pytest.mark.parametrize("sizes,limit", [((65535, 1, 256, 1), 80), ((65535, 2, 64, 1), 120), ((4096, 1, 16, 1024), 130),
+                                         ((65535, 1, 16, 16), 210)], ids=str)
+def test_small_batches_pay_for_no_tile(kdb, sizes, limit):
+    batches, m, k, n = sizes
+    a, b = np.ones((batches, m, k), np.float32), np.ones((batches, k, n), np.float32)
+    da, db, out = kdb.to_device(a), kdb.to_device(b), kdb.empty((batches, m, n), np.float32)
+    events = [ctypes.c_void_p(), ctypes.c_void_p()]
+    for e in events:
+        kdb.call("event_create", ctypes.byref(e))
+    ms, best = ctypes.c_float(), np.inf
+    for _ in range(10):
+        kdb.call("event_record", events[0])
+        for _ in range(10):
+            kdb.call("matmul", kd.F32, da.ptr, db.ptr, out.ptr, kd.MatmulSizes(*sizes))
+        kdb.call("event_record", events[1])
+        kdb.call("event_elapsed_ms", ctypes.byref(ms), *events)
+        best = min(best, ms.value * 100)
+    for e in events:
+        kdb.call("event_destroy", e)
+    assert (out.numpy() == k).all()
+    assert best < limit
+
+
 @pytest.mark.parametrize("n", [1, 3, 4])
 @pytest.mark.parametrize("k", [6, 64])
 def test_few_columns_over_more_batches_than_a_grid_dimension(kdb, k, n):
