@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
 // The next block's split runs between the MFMAs of the scores: 105 -> 100 us, alone 77 -> 62. Error of the
 // output against 64 bits 2.0e-7 -> 1.4e-7.
 //
-// A workgroup that meets a value above 1e18, an infinity or a NaN (pieces or their products may be infinite)
+// A workgroup that meets a value above 2^40 = 1e12, an infinity or a NaN (pieces or their products may be infinite)
 // starts again on the f32 matrix cores, straight from memory.
 constexpr int kWide = 128;                             // queries of a workgroup
 constexpr int kKeyGroup = kBlock * 16 + 32;            // bytes of 8 features of the keys; 32 against bank conflicts
@@ -376,7 +376,7 @@ constexpr int kKeyPiece = kD / 8 * kKeyGroup;
 constexpr int kValueGroup = kD * 16;                   // bytes of 8 keys of the features
 constexpr int kValuePiece = kBlock / 8 * kValueGroup;
 constexpr int kStage = 3 * (kKeyPiece + kValuePiece);
-constexpr float kPieceLimit = 1e18f;
+constexpr float kPieceLimit = 0x1p40f;  // 64 products of scaled pieces stay finite
 
 __device__ __forceinline__ bool past_limit(const float (&x)[8]) {
     float sum = 0.f;
@@ -495,17 +495,18 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
         load(kb + 2);
         if (mine) {
             // scale and mask; the scores are finite, and every query has a key in block 0
+            const float scale = sh.inv_scale * kUnscale;
             float bmax = -INFINITY;
             if (kb == last) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    s[r] = block_row(r, lh) > li ? -INFINITY : s[r] * sh.inv_scale;
+                    s[r] = block_row(r, lh) > li ? -INFINITY : s[r] * scale;
                     bmax = fmaxf(bmax, s[r]);
                 }
             } else {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    s[r] *= sh.inv_scale;
+                    s[r] *= scale;
                     bmax = fmaxf(bmax, s[r]);
                 }
             }
@@ -591,7 +592,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
     }
     // o[dt][r] = O^T[32 dt + block_row(r, lh)][query li]
     if (query < sh.length) {
-        const float inv = 1.f / l;
+        const float inv = (redo ? 1.f : kUnscale) / l;
         float* dst = out + (static_cast<int64_t>(b) * sh.length + query) * sh.out_row + h * kD;
 #pragma unroll
         for (int dt = 0; dt < 2; ++dt)

@@ -88,9 +88,8 @@ __device__ __forceinline__ void tile_of(int64_t id, int64_t tiles_m, int64_t til
 
 // ---- pieces family (f32 on the bf16 matrix cores) ---------------------------------------------
 //
-// An f32 value is the exact sum of three bf16 values (8 + 8 + 8 significant bits, each piece the
-// remainder rounded to nearest), so a product of two f32 values is the sum of nine bf16 products, of
-// which the six above 2^-27 of it are taken: hi.hi on one accumulator, and lo.hi, hi.lo, mid.mid,
+// An f32 value, scaled by 2^16, is the exact sum of three bf16 values (kd_pieces.h), so a product of
+// two f32 values is 2^-32 times the sum of nine bf16 products, of which the six above 2^-27 of it are taken: hi.hi on one accumulator, and lo.hi, hi.lo, mid.mid,
 // mid.hi, hi.mid on a second, both in f32 by v_mfma_f32_32x32x16_bf16, added at the end. The dropped
 // three are below half an f32 rounding of the product; what bounds the error is the rounding of the
 // running sum, and hi.hi's takes two roundings per 16 K where v_mfma_f32_32x32x2f32 takes sixteen.
@@ -98,17 +97,18 @@ __device__ __forceinline__ void tile_of(int64_t id, int64_t tiles_m, int64_t til
 // 256 8.9e-8 (2.1e-7), 2048 2.7e-7 (8.1e-7), 4096 1.9e-7 in splits (5.7e-7); of the column sums of
 // the result likewise, which the second accumulator is for: the bf16 instructions cut the low bits
 // of what they align below the accumulator towards minus infinity, and six products on one
-// accumulator leave a bias (2048: column sums 4.9e-6). bf16 has f32's exponents and the matrix cores
-// keep its subnormals, so any magnitude splits; infinities and NaN do not (inf - inf), see the end.
+// accumulator leave a bias (2048: column sums 4.9e-6). The matrix cores keep bf16 subnormals, so with the
+// scale every value below 2^112 splits; larger ones, infinities and NaN, and sums from 2^96 on, see the end.
 //
 // The rate: 2.5 PFLOP/s / 6 = 417 TFLOP/s of f32 products against 157 on the f32 matrix cores.
-// Measured at 4096^3: 636 us (216 TFLOP/s: 1.30 PFLOP/s of bf16 products, where the vendor's bf16
-// product reaches 1.13 at this size and 1.36 at 8192^3; the clock falls to ~2.1 GHz under either)
-// against 966 us (142 TFLOP/s) on the f32 matrix cores.
+// Measured at 4096^3: 662 us (208 TFLOP/s: 1.25 PFLOP/s of bf16 products, where the vendor's bf16
+// product reaches 1.13 at this size and 1.36 at 8192^3; the clock falls to ~2.1 GHz under either, and the scaling
+// of the operands, one operation in 6.5 of the split, costs 3.5 %) against 966 us (142 TFLOP/s) on the f32
+// matrix cores.
 //
 // A workgroup owns a TM x TN tile and stages both operands through LDS as pieces: each 8-deep K group
 // of a row is one 16-byte unit per piece, [piece][group][row], so that a lane's MFMA operand is one
-// conflict-free 16-byte read. The split into pieces (5.5 VALU operations per element) runs between
+// conflict-free 16-byte read. The split into pieces (6.5 VALU operations per element) runs between
 // the MFMAs of the step before. Global loads run two steps ahead (one step: 4096 x 256 x 768 on
 // 128 x 128 tiles 24 us, two 17). A partial K step comes first, with guarded loads; rows past M or N
 // repeat the last one and are not stored, so ragged sizes cost no tests in the loop. Element
@@ -297,12 +297,12 @@ __global__ __launch_bounds__(WM * WN * 64, Occ) void pieces_kernel(const float* 
         }
     };
     // The end of a step in which the next stage was also split and stored: its VALU work between the
-    // MFMAs, four operations after each.
+    // MFMAs, six operations after each (999 x 768 x 3072: 34.4 us; four 37.5).
     const auto mix = [&]() {
 #pragma unroll
         for (int q = 0; q < IM * JN * 6 * (BK / 16); ++q) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
         }
         __syncthreads();
     };
@@ -346,9 +346,9 @@ __global__ __launch_bounds__(WM * WN * 64, Occ) void pieces_kernel(const float* 
     }
 
     const int row0 = m0 + wm * IM * 32, col0 = n0 + wn * JN * 32;
-    // A sum that is not finite means an infinity or a NaN among the inputs, or an overflow. Pieces give
-    // NaN where the f32 product of an infinity is one, so the wave's outputs are computed again from
-    // the f32 operands on the f32 matrix cores. With finite inputs and sums this is never taken.
+    // A sum that is not finite means an infinity or a NaN among the inputs, or an overflow of the scaled sum or
+    // of a piece (values from 2^112 = 5e33 on, sums from 2^96 = 8e28 on). The wave's outputs are then computed
+    // again from the f32 operands on the f32 matrix cores.
     bool odd = false;
 #pragma unroll
     for (int i = 0; i < IM; ++i)
@@ -358,6 +358,7 @@ __global__ __launch_bounds__(WM * WN * 64, Occ) void pieces_kernel(const float* 
             for (int r = 0; r < 16; ++r) {
                 acc[i][j][r] += small[i][j][r];
                 odd |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+                acc[i][j][r] *= kUnscale;
             }
     if (__any(odd)) {
 #pragma unroll
@@ -968,7 +969,7 @@ struct Tiling {
     double alone_us, crowded_us, end_us;
 };
 constexpr Tiling kTilings[] = {
-    {256, 128, 16, 1, 64, 2.30, 2.48, 7.0},  // 8 waves of 64 x 64: the best rate (4096^3: 636 us; 128 x 128 below 662)
+    {256, 128, 16, 1, 64, 2.30, 2.48, 7.0},  // 8 waves of 64 x 64: the best rate (4096^3: 662 us; 128 x 128 below 690)
     {128, 128, 16, 2, 64, 1.35, 1.29, 5.0},  // two workgroups hide one another's ends (999 x 768 x 50257: 427 us; above 468)
     {128, 128, 32, 1, 64, 1.10, 1.37, 8.0},  // one workgroup per CU (2048^3: 94 us; 999 x 768 x 3072: 33)
     {128, 64, 32, 2, 64, 0.80, 0.76, 5.5},   // 1024 x 4096 x 256 in 8 splits: 21 us (128 x 128: 27)

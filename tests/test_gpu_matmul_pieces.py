@@ -5,6 +5,11 @@ Tolerance per element, from the arithmetic: every product keeps six of the nine 
 operands' pieces (the dropped three are below 3 * 2^-27 of it), and the running sums round at most
 twice per 8 of K and once per split; each rounding is at most 2^-24 of a partial sum, which is at most
 sum |a||b|. The same bound covers the small tiles and the general kernel (one rounding per K).
+
+That bound grows with K while a lost term's error averages out, so for random operands of one size the 2-norm of the
+error is bounded as well: roundings of rms 2^-24 / sqrt(3) at K / 8 partial sums that grow to the result make
+2^-24 sqrt(K / 48) = 3.5e-8 sqrt(K / 16) of it, and the last few and the dropped products two more. A third piece or
+the product of the second pieces left out makes 1e-6 and more at any K.
 """
 import ctypes
 
@@ -37,6 +42,7 @@ def check(got, a, b, bias=None):
         want, size = want + bias, size + np.abs(bias)
     err = np.abs(got.reshape(want.shape) - want)
     assert (err <= (k + 72) * 2.0 ** -24 * size).all(), (err / size).max() * 2 ** 24
+    return np.linalg.norm(err) / np.linalg.norm(want)
 
 
 # (m, k, n): around the tiles of 64, 128 and 256 and the K steps of 16 and 32, one short K step, long K
@@ -54,7 +60,25 @@ def test_ragged_products(kdb, m, k, n, layout):
     bias = rng.normal(size=n).astype(np.float32) if layout == "nt" else None
     got = product(kdb, a.T.copy() if at else a, b.T.copy() if bt else b, (1, m, k, n), (0, 1, m) if at else (0, k, 1),
                   (0, 1, k) if bt else (0, n, 1), bias=bias)
-    check(got, a, b, bias)
+    assert check(got, a, b, bias) <= 3.5e-8 * ((k / 16) ** 0.5 + 2)
+
+
+@pytest.mark.parametrize("small_b", [False, True])
+@pytest.mark.parametrize("k", [1, 8, 40])
+@pytest.mark.parametrize("exponent", [-149, -140, -127, -126, -120, -115, -112, -110, -100, 95, 105, 111, 112, 127])
+def test_operands_of_any_size_keep_their_bits(kdb, exponent, k, small_b):
+    """One operand's values from the smallest subnormals to the largest, the other's such that products are near 1 (or as
+    near as f32 goes): a short K, so that nothing averages out. Six products' dropped terms and a rounding per product."""
+    rng = np.random.default_rng(k + 200 - exponent)
+    m, n = 2000, 1030  # beyond the small tiles
+    a = np.ldexp(rng.uniform(1, 2, (m, k)), exponent).astype(np.float32)  # (rounded to the subnormals' grid)
+    b = np.ldexp(rng.uniform(1, 2, (k, n)), int(np.clip(-exponent, -126, 120))).astype(np.float32)
+    if small_b:
+        a, b, m, n = b.T.copy(), a.T.copy(), n, m
+    got = product(kdb, a, b, (1, m, k, n), (0, k, 1), (0, n, 1)).reshape(m, n)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - want) <= (k + 3) * 2.0 ** -24 * want + 2.0 ** -149).all()
 
 
 def test_magnitudes_that_one_bf16_cannot_hold(kdb):
