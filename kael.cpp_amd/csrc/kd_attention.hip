@@ -220,6 +220,17 @@ __device__ __forceinline__ v16f dot_rows(const float (&a)[32], const float (&b)[
     return s0 + s1;
 }
 
+// The same from the rows in memory (lane li's of each side).
+__device__ __forceinline__ v16f dot_memory(const float* __restrict__ a, const float* __restrict__ b, int lh) {
+    v16f s0 = zero16(), s1 = zero16();
+#pragma unroll 1
+    for (int t = 0; t < 32; t += 2) {
+        s0 = mfma(a[32 * lh + t], b[32 * lh + t], s0);
+        s1 = mfma(a[32 * lh + t + 1], b[32 * lh + t + 1], s1);
+    }
+    return s0 + s1;
+}
+
 // ---- forward -----------------------------------------------------------------------------
 
 // Where the forward's heads lie: elements between batches, heads and rows of q, and of k and v.
@@ -363,13 +374,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
 // features, V by the 8 keys that a lane's score registers hold, so that P is an operand as it stands.
 // Every query's keys pass through one wave, which needs no merge.
 //
-// 8 x 1024 tokens, 12 heads: 154 -> 100 us (129 TFLOP/s). A step of a workgroup alone takes 1.8 us, 0.7 of
+// 8 x 1024 tokens, 12 heads: 154 -> 104 us (124 TFLOP/s). A step of a workgroup alone takes 1.8 us, 0.7 of
 // it MFMAs; two workgroups of a CU overlap, and the VALU work (the split, the exponentials) is what is left.
 // The next block's split runs between the MFMAs of the scores: 105 -> 100 us, alone 77 -> 62. Error of the
 // output against 64 bits 2.0e-7 -> 1.4e-7.
 //
 // A workgroup that meets a value above 2^40 = 1e12, an infinity or a NaN (pieces or their products may be infinite)
-// starts again on the f32 matrix cores, straight from memory.
+// starts again straight from memory, with P . V on the f32 matrix cores and the scores on pieces as far as they are
+// finite, block pair by block pair. The backward takes the scores by the same rule: exp(S - L) has to see the S that
+// went into L, or P would be off by the difference of two roundings of S (3e-7 of it), where a key that alone makes up
+// its row must have P = 1 whatever its score.
 constexpr int kWide = 128;                             // queries of a workgroup
 constexpr int kKeyGroup = kBlock * 16 + 32;            // bytes of 8 features of the keys; 32 against bank conflicts
 constexpr int kKeyPiece = kD / 8 * kKeyGroup;
@@ -393,12 +407,52 @@ __device__ __forceinline__ void store_pieces(char* unit, int piece, const float 
     *reinterpret_cast<bf8*>(unit + 2 * piece) = lo;
 }
 
-// hi and small accumulate one 16-deep product of pieces.
+// hi and small accumulate one 16-deep product of pieces; Swapped: a and b stand in each other's place, term for term.
+template <bool Swapped = false>
 __device__ __forceinline__ void multiply_pieces(const bf8 (&a)[3], const bf8 (&b)[3], v16f& hi, v16f& small) {
     constexpr int kA[5] = {2, 0, 1, 1, 0}, kB[5] = {0, 2, 1, 0, 1};
 #pragma unroll
-    for (int q = 0; q < 5; ++q) small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kA[q]], b[kB[q]], small, 0, 0, 0);
+    for (int q = 0; q < 5; ++q)
+        small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[Swapped ? kB[q] : kA[q]], b[Swapped ? kA[q] : kB[q]], small, 0, 0, 0);
     hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], hi, 0, 0, 0);
+}
+
+// Pieces of a row's features 16 g + 8 lh .. + 7, from memory or a padded LDS row.
+__device__ __forceinline__ void row_pieces(bf8 (&p)[3], const float* __restrict__ row, int g, int lh) {
+    const v4f a = *reinterpret_cast<const v4f*>(row + 16 * g + 8 * lh);
+    const v4f c = *reinterpret_cast<const v4f*>(row + 16 * g + 8 * lh + 4);
+    const float x[8] = {a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+    split_pieces(x, p[0], p[1], p[2]);
+}
+
+// A block pair's scores on pieces (times 2^32), one side's rows at `row` (lane li's, the product's A), the other's pieces
+// from `other(g, pieces)`. The same for every kernel that computes them, bit for bit, whichever side is A.
+template <bool Swapped, class Other> __device__ __forceinline__ v16f piece_scores(const float* __restrict__ row, int lh, const Other& other) {
+    v16f s = zero16(), small = zero16();
+#pragma unroll
+    for (int g = 0; g < kD / 16; ++g) {
+        bf8 mine[3], theirs[3];
+        row_pieces(mine, row, g, lh);
+        other(g, theirs);
+        multiply_pieces<Swapped>(mine, theirs, s, small);
+    }
+    return s + small;
+}
+
+// The same with the pieces in registers.
+template <bool Swapped> __device__ __forceinline__ v16f piece_scores(const float* __restrict__ row, int lh, const bf8 (&other)[kD / 16][3]) {
+    return piece_scores<Swapped>(row, lh, [&](int g, bf8 (&p)[3]) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w) p[w] = other[g][w];
+    });
+}
+
+// Whether a block pair's scores have to be computed in f32: pieces overflowed, or met an infinity or a NaN.
+__device__ __forceinline__ bool scores_overflowed(const v16f& s) {
+    bool odd = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) odd |= !(fabsf(s[r]) < INFINITY);
+    return __any(odd);
 }
 
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kernel(float* __restrict__ out, float* __restrict__ lse,
@@ -557,14 +611,17 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
         for (int kb = 0; kb <= min(last, blocks - 1); ++kb) {
             const int j0 = kb * kBlock;
             const float* krow = k + static_cast<int64_t>(min(j0 + li, sh.length - 1)) * in.kv_row;
-            v16f s = zero16();
-#pragma unroll 1
-            for (int f = 0; f < 32; ++f) s = mfma(krow[32 * lh + f], qrow[32 * lh + f], s);
+            v16f s = piece_scores<false>(krow, lh, qp);
+            float scale = sh.inv_scale * kUnscale;
+            if (scores_overflowed(s)) {
+                scale = sh.inv_scale;
+                s = dot_memory(krow, qrow, lh);
+            }
             float bmax = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int j = j0 + block_row(r, lh);
-                s[r] = (j > query || j >= sh.length) ? -INFINITY : s[r] * sh.inv_scale;
+                s[r] = (j > query || j >= sh.length) ? -INFINITY : s[r] * scale;
                 bmax = fmaxf(bmax, s[r]);
             }
             const float mnew = fmaxf(m, halves_max(bmax));
@@ -621,12 +678,40 @@ __device__ __forceinline__ float row_delta(const float (&g)[32], const float (&o
     return halves_sum(part);
 }
 
-// P from a row's log-sum-exp. The score and the log-sum-exp take the same steps (1 / 8 is exact), so that the exponent
-// is 0 and P exactly 1 for a key that alone makes up its row, whatever the score's size: a constant's rounding on one
-// side of the difference alone would grow with it.
-__device__ __forceinline__ float row_probability(float s, float inv_scale, float lse) { return __expf(s * inv_scale - lse); }
+// P = exp(S - L) of a row's log-sum-exp L. The score is the forward's, bit for bit, and P must be 1 for a key that alone
+// makes up its row, whatever the score's size. Near: exp2(S log2(e) - at) times `factor`, which holds what L log2(e)
+// rounded off: one rounding of the exponent where exp(S - L) has two, with as many operations. Both sides take the f32
+// constant, as its error on one side alone is 1.3e-8 L of P; below 8, where that is less than P's last bit, the factor
+// holds it for L, so that a flat row (S near 0) has none. What is rounded off has to stay an exponent of 2: beyond kNear
+// the steps are those of the log-sum-exp (`scale` is a power of two, so that S - L is 0).
+constexpr float kLog2e = 1.44269504088896341f;
+constexpr float kLog2eRest = 1.92596299e-8f;  // log2(e) - kLog2e
+constexpr float kNear = 1048576.f, kSmall = 8.f;
 
-// The dQ group `group`: lds holds 7 tiles.
+// A block of rows that are all near or not: P = exp2(S first - at) factor, or exp(S first - at).
+struct BlockScale {
+    bool near;
+    float first;
+
+    __device__ __forceinline__ explicit BlockScale(float lse) : near(__all(fabsf(lse) < kNear)) {}
+    __device__ __forceinline__ void set_scale(float scale) {
+        first = near ? scale * kLog2e : scale;
+    }
+    __device__ __forceinline__ void row(float lse, float& at, float& factor) const {
+        const float product = lse * kLog2e, rest = fmaf(lse, kLog2e, -product);
+        at = near ? product : lse;
+        factor = near ? __builtin_amdgcn_exp2f(-(fabsf(lse) < kSmall ? fmaf(lse, kLog2eRest, rest) : rest)) : 1.f;
+    }
+    __device__ __forceinline__ float probability(float s, float at) const {  // without the factor
+        float x = fmaf(s, first, -at);
+        if (!near) x *= kLog2e;
+        return __builtin_amdgcn_exp2f(x);
+    }
+};
+
+// The dQ group `group`: lds holds 7 tiles and the query block's pieces. Pieces: the scores as
+// attention_forward_pieces_kernel has them.
+template <bool Pieces>
 __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, float* __restrict__ dqkv,
                                          const float* __restrict__ dout, const float* __restrict__ qkv,
                                          const float* __restrict__ out, const float* __restrict__ lse,
@@ -656,6 +741,10 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     part_load(gpart, go, i0, sh.length, sh.out_row, wave, lane);
     part_load(opart, o, i0, sh.length, sh.out_row, wave, lane);
     const float row_lse = query < sh.length ? lse[static_cast<int64_t>(bh) * sh.length + query] : 0.f;
+    BlockScale rows_scale(row_lse);
+    float at, factor;
+    rows_scale.row(row_lse, at, factor);
+    factor *= sh.inv_scale;
     if (wave <= qb) {
         tile_load(kload, k, wave * kBlock, sh.length, sh.row, lane);
         tile_load(vload, v, wave * kBlock, sh.length, sh.row, lane);
@@ -665,7 +754,17 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     part_store(rows[2], opart, wave, lane);
     __syncthreads();
     float qreg[32], doreg[32];
-    lds_half_row(qreg, rows[0], li, lh);
+    char* qpieces = reinterpret_cast<char*>(lds + (kWaves + 3) * kTile);  // as a key stage of the forward
+    if constexpr (Pieces) {
+        const int row = threadIdx.x / 8, unit = threadIdx.x % 8;
+        bf8 qp[3];
+        row_pieces(qp, rows[0] + row * kLd, unit / 2, unit % 2);
+#pragma unroll
+        for (int w = 0; w < 3; ++w) *reinterpret_cast<bf8*>(qpieces + w * kKeyPiece + unit * kKeyGroup + row * 16) = qp[w];
+        __syncthreads();
+    } else {
+        lds_half_row(qreg, rows[0], li, lh);
+    }
     lds_half_row(doreg, rows[1], li, lh);
     float dl;
     {
@@ -688,7 +787,15 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
             wave_sync();
             dp = dot_rows(vreg, doreg);
         }
-        {
+        float scale = sh.inv_scale;
+        if constexpr (Pieces) {
+            s = piece_scores<false>(tile + li * kLd, lh, [&](int g, bf8 (&p)[3]) {
+#pragma unroll
+                for (int w = 0; w < 3; ++w) p[w] = *reinterpret_cast<const bf8*>(qpieces + w * kKeyPiece + (2 * g + lh) * kKeyGroup + li * 16);
+            });
+            if (scores_overflowed(s)) s = dot_memory(tile + li * kLd, rows[0] + li * kLd, lh);
+            else scale *= kUnscale;
+        } else {
             float kreg[32];
             lds_half_row(kreg, tile, li, lh);
             s = dot_rows(kreg, qreg);
@@ -698,12 +805,13 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
             tile_load(vload, v, j0 + kWaves * kBlock, sh.length, sh.row, lane);
         }
         // s[r] = S[query][key], dp[r] = dP[query][key] for key j0 + block_row(r, lh)
+        rows_scale.set_scale(scale);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int key = j0 + block_row(r, lh);
             const bool live = key <= query && key < sh.length && query < sh.length;
-            const float p = live ? row_probability(s[r], sh.inv_scale, row_lse) : 0.f;
-            s[r] = p * (dp[r] - dl) * sh.inv_scale;
+            const float p = live ? rows_scale.probability(s[r], at) : 0.f;
+            s[r] = p * (dp[r] - dl) * factor;
         }
         // dQ[i][d] += sum_j dS[i][j] K[j][d]: A = dS (lane li: query li), B = K (feature 32 dt + li)
 #pragma unroll
@@ -720,15 +828,16 @@ __device__ __forceinline__ void dq_group(int group, float* __restrict__ lds, flo
     store_tile_sum(dqkv + tok0 * sh.row + h * kD, tiles, i0, sh.length, sh.row, wave, lane);
 }
 
-// The dK / dV group `group`: lds holds 9 tiles and 2 x 4 rows of 32.
+// The dK / dV group `group`: lds holds 9 tiles and 3 numbers of 4 x 32 rows. Pieces: as for dq_group.
+template <bool Pieces>
 __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, float* __restrict__ dqkv,
                                           const float* __restrict__ dout, const float* __restrict__ qkv,
                                           const float* __restrict__ out, const float* __restrict__ lse,
                                           const AttentionShape& sh) {
     float* tiles = lds;                        // each wave's Q (O first) and dO tiles; the first holds K at the start
     float* vtile = lds + 2 * kWaves * kTile;   // the key block's V
-    float (*lses)[kBlock] = reinterpret_cast<float (*)[kBlock]>(vtile + kTile);
-    float (*deltas)[kBlock] = lses + kWaves;
+    f2v (*rows)[kBlock] = reinterpret_cast<f2v (*)[kBlock]>(vtile + kTile);  // of each wave: at, factor (BlockScale)
+    float (*deltas)[kBlock] = reinterpret_cast<float (*)[kBlock]>(rows + kWaves);
     const int blocks = (sh.length + kBlock - 1) / kBlock;
     const int units = sh.batch * sh.heads;
     const int bh = group % units;
@@ -766,27 +875,45 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     part_store(vtile, vpart, wave, lane);
     __syncthreads();
     float kreg[32];
-    lds_half_row(kreg, tiles, li, lh);
+    bf8 kp[kD / 16][3];
+    if constexpr (Pieces) {
+#pragma unroll
+        for (int g = 0; g < kD / 16; ++g) row_pieces(kp[g], tiles + li * kLd, g, lh);
+    } else {
+        lds_half_row(kreg, tiles, li, lh);
+    }
     __syncthreads();
 
     v16f dk[2] = {zero16(), zero16()}, dv[2] = {zero16(), zero16()};
     const auto block_products = [&](int i0) {
         tile_store(qtile, oload, lane);  // O first, for the rows' delta (the previous block's reads are done)
         tile_store(gtile, gload, lane);
-        if (lane < kBlock) lses[wave][lane] = lload;
+        BlockScale rows_scale(lload);  // (0 in the upper lanes)
         wave_sync();
         {
             float greg[32], oreg[32];
             lds_half_row(greg, gtile, li, lh);
             lds_half_row(oreg, qtile, li, lh);
             const float dl = row_delta(greg, oreg);
-            if (lh == 0) deltas[wave][li] = dl;
+            if (lh == 0) {
+                float at, factor;
+                rows_scale.row(lload, at, factor);
+                rows[wave][li] = f2v{at, factor};
+                deltas[wave][li] = dl;
+            }
         }
         wave_sync();
         tile_store(qtile, qload, lane);  // then Q in its place: a wave's LDS operations run in issue order
         wave_sync();
         v16f s, dp;
-        {
+        float scale = sh.inv_scale;
+        if constexpr (Pieces) {
+            s = piece_scores<true>(qtile + li * kLd, lh, kp);
+            // (K's rows from memory: its tile has been written over)
+            if (scores_overflowed(s))
+                s = dot_memory(qtile + li * kLd, k + static_cast<int64_t>(min(key, sh.length - 1)) * sh.row, lh);
+            else scale *= kUnscale;
+        } else {
             float qreg[32];
             lds_half_row(qreg, qtile, li, lh);
             s = dot_rows(qreg, kreg);
@@ -799,12 +926,14 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
         }
         // s[r] = S[query][key], dp[r] = dP[query][key] for query i0 + block_row(r, lh), key li
         float p[16];
+        rows_scale.set_scale(scale);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int local = block_row(r, lh);
             const int query = i0 + local;
             const bool live = key <= query && query < sh.length && key < sh.length;
-            p[r] = live ? row_probability(s[r], sh.inv_scale, lses[wave][local]) : 0.f;
+            const f2v row = rows[wave][local];
+            p[r] = live ? rows_scale.probability(s[r], row[0]) * row[1] : 0.f;
             s[r] = p[r] * (dp[r] - deltas[wave][local]) * sh.inv_scale;
         }
         // dV[j][d] += sum_i P[i][j] dO[i][d], dK[j][d] += sum_i dS[i][j] Q[i][d]:
@@ -837,21 +966,23 @@ __device__ __forceinline__ void dkv_group(int group, float* __restrict__ lds, fl
     store_tile_sum(dstk + sh.heads * kD, tiles + kWaves * kTile, j0, sh.length, sh.row, wave, lane);
 }
 
-constexpr int kBackwardLds = (2 * kWaves + 1) * kTile + 2 * kWaves * kBlock;  // the dK / dV group's, the larger
+constexpr int kBackwardLds = (2 * kWaves + 1) * kTile + 3 * kWaves * kBlock;  // the dK / dV group's, the larger
+static_assert(4 * kBackwardLds >= 4 * (kWaves + 3) * kTile + 3 * kKeyPiece);
 
+template <bool Pieces>
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_backward_kernel(float* __restrict__ dqkv,
                                                                             const float* __restrict__ dout,
                                                                             const float* __restrict__ qkv,
                                                                             const float* __restrict__ out,
                                                                             const float* __restrict__ lse,
                                                                             AttentionShape sh) {
-    __shared__ float lds[kBackwardLds];
+    __shared__ __attribute__((aligned(16))) float lds[kBackwardLds];
     const int groups = sh.batch * sh.heads * ((sh.length + kBlock - 1) / kBlock);
     const int i = static_cast<int>(blockIdx.x);
     if (i < groups)
-        dkv_group(i, lds, dqkv, dout, qkv, out, lse, sh);
+        dkv_group<Pieces>(i, lds, dqkv, dout, qkv, out, lse, sh);
     else
-        dq_group(i - groups, lds, dqkv, dout, qkv, out, lse, sh);
+        dq_group<Pieces>(i - groups, lds, dqkv, dout, qkv, out, lse, sh);
 }
 
 // ---- attention of new queries against a KV cache -------------------------------------------------
@@ -981,17 +1112,20 @@ int check_shape(int dtype, int64_t batch, int64_t length, int64_t heads, int64_t
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+// Whether the forward of this shape runs on pieces, and so the backward's scores. One of those workgroups is a longer
+// chain (1.8 us a key block, where the four waves of the f32 kernel share a query block's keys), so they need more than
+// one a CU, and more queries than the f32 kernel's block. f32 / pieces, us, and workgroups of the latter: 8 x 1024 x 12
+// 154 / 104 (768), 16 x 300 x 16 63 / 45 (768), 8 x 512 x 12 48 / 40 (384), 128 x 33 x 8 27 / 20 (1024), 3 x 1024 x 12
+// 65 / 68 (288, with the backward 252 / 251); 4 x 1024 x 8 58 / 62 (256), 8 x 250 x 8 12 / 20 (128), 32 x 128 x 4 9.0 / 12.8 (128), 256 x 32 x 8
+// 26.6 / 28.2 (2048).
+int64_t wide_groups(const AttentionShape& sh) { return int64_t{sh.batch} * sh.heads * ((sh.length + kWide - 1) / kWide); }
+bool on_pieces(const AttentionShape& sh) { return sh.length > kBlock && wide_groups(sh) > compute_units(); }
+
 template <bool Exact> int launch_forward(float* out, float* lse, const HeadViews& in, const AttentionShape& sh) {
     if constexpr (!Exact) {
-        // One of these workgroups is a longer chain (1.8 us a key block, where the four waves of the f32 kernel share
-        // a query block's keys), so they need more than one a CU, and more queries than the f32 kernel's block. f32 /
-        // pieces, us, and workgroups of the latter: 8 x 1024 x 12 154 / 100 (768), 16 x 300 x 16 63 / 41 (768),
-        // 8 x 512 x 12 48 / 38 (384), 128 x 33 x 8 27 / 20 (1024), 3 x 1024 x 12 65 / 64 (288); 4 x 1024 x 8
-        // 58 / 62 (256), 8 x 250 x 8 12 / 20 (128), 32 x 128 x 4 9.0 / 12.8 (128), 256 x 32 x 8 26.6 / 28.2 (2048).
-        const int64_t wide = int64_t{sh.batch} * sh.heads * ((sh.length + kWide - 1) / kWide);
-        if (sh.length > kBlock && wide > compute_units()) {
-            hipLaunchKernelGGL(attention_forward_pieces_kernel, dim3(static_cast<uint32_t>(wide)), dim3(kWaves * 64), 0, stream(),
-                               out, lse, in, sh);
+        if (on_pieces(sh)) {
+            hipLaunchKernelGGL(attention_forward_pieces_kernel, dim3(static_cast<uint32_t>(wide_groups(sh))), dim3(kWaves * 64), 0,
+                               stream(), out, lse, in, sh);
             KD_LAUNCH_CHECK();
             return KD_OK;
         }
@@ -1039,10 +1173,13 @@ extern "C" int kd_causal_attention_backward(int dtype, void* dqkv, const void* d
         return fail(KD_E_INVALID, "kd_causal_attention_backward: every operand must be given, 16-byte aligned");
     if (int rc = ensure_device()) return rc;
     const int64_t blocks = (length + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(attention_backward_kernel, dim3(static_cast<uint32_t>(2 * batch * heads * blocks)),
-                       dim3(kWaves * 64), 0, stream(), static_cast<float*>(dqkv), static_cast<const float*>(dout),
-                       static_cast<const float*>(qkv), static_cast<const float*>(out), static_cast<const float*>(lse),
-                       sh);
+    const auto launch = [&](auto pieces) {
+        hipLaunchKernelGGL(attention_backward_kernel<decltype(pieces)::value>, dim3(static_cast<uint32_t>(2 * batch * heads * blocks)),
+                           dim3(kWaves * 64), 0, stream(), static_cast<float*>(dqkv), static_cast<const float*>(dout),
+                           static_cast<const float*>(qkv), static_cast<const float*>(out), static_cast<const float*>(lse), sh);
+    };
+    if (on_pieces(sh)) launch(std::true_type{});
+    else launch(std::false_type{});
     KD_LAUNCH_CHECK();
     return KD_OK;
 }

@@ -123,10 +123,25 @@ def check_large_scores(kdb, qkv, dout, size):
 
 
 @pytest.mark.parametrize("size", [10, 100, -100, 1.2e3, -1.2e4, 1.2e6, -1.2e6, 1.2e8, -1.2e9, 1.2e10, 1e12, -1e12])
-@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 37, 3), (1, 300, 1)], ids=["1x1x1", "2x37x3", "1x300x1"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 37, 3), (1, 300, 1), (33, 33, 8), (3, 300, 30)],
+                         ids=["1x1x1", "2x37x3", "1x300x1", "33x33x8", "3x300x30"])
 def test_gradients_at_large_scores(kdb, shape, size):
-    """P is exactly 1 where one key makes up the row (row 0 of every sequence, one dominating key), at any score."""
+    """P is exactly 1 where one key makes up the row (row 0 of every sequence, one dominating key), at any score: the
+    last two shapes have their products in bf16 pieces, forward and scores of the backward."""
     check_large_scores(kdb, *scores_of_size(*shape, size), size)
+
+
+@pytest.mark.parametrize("q_size", [1e8, 1e13, 1e20, 1e30])
+def test_gradients_where_pieces_overflow(kdb, q_size):
+    """Queries of one block of 32 past what pieces hold (with small keys, so that the scores stay at 1e6) among ordinary
+    ones; some values of V too. Forward and backward have to take the same blocks in f32."""
+    size, (b, t, h) = 1e6, (3, 300, 30)
+    qkv, dout = scores_of_size(b, t, h, size)
+    qkv[1, :, 1, :10] /= np.float32(q_size)
+    qkv[1, 40:70, 0, :10] *= np.float32(q_size)
+    qkv[2, 200, 2, 3, 5], qkv[2, 10, 2, 4, 9] = 3e15, -2e14
+    dout[2] *= np.float32(1e-3)
+    check_large_scores(kdb, qkv, dout, size)
 
 
 def test_attention_rejects_unsupported_shapes(kdb):
