@@ -233,18 +233,37 @@ __device__ __forceinline__ v16f dot_memory(const float* __restrict__ a, const fl
 
 // ---- forward -----------------------------------------------------------------------------
 
-// Where the forward's heads lie: elements between batches, heads and rows of q, and of k and v.
+// Where the forward's heads lie. A head's rows of q, k and v in the fused projection, with everything from the shape:
+// six strides more to load and multiply out are a few per cent of a short launch (1 x 64 x 1 5.52 us against 5.70).
+struct FusedViews {
+    const float* qkv;
+
+    __device__ __forceinline__ const float* q(const AttentionShape& sh, int b, int h) const {
+        return qkv + static_cast<int64_t>(b) * sh.length * sh.row + h * kD;
+    }
+    __device__ __forceinline__ const float* k(const AttentionShape& sh, int b, int h) const { return q(sh, b, h) + sh.heads * kD; }
+    __device__ __forceinline__ const float* v(const AttentionShape& sh, int b, int h) const { return k(sh, b, h) + sh.heads * kD; }
+    __device__ __forceinline__ int64_t q_row(const AttentionShape& sh) const { return sh.row; }
+    __device__ __forceinline__ int64_t kv_row(const AttentionShape& sh) const { return sh.row; }
+};
+
+// One sequence whose heads lie apart.
 struct HeadViews {
-    const float *q, *k, *v;
-    int64_t q_batch, q_head, q_row;
-    int64_t kv_batch, kv_head, kv_row;
+    const float *q_, *k_, *v_;
+    int64_t q_stride, kv_head;
+
+    __device__ __forceinline__ const float* q(const AttentionShape&, int, int h) const { return q_ + h * kD; }
+    __device__ __forceinline__ const float* k(const AttentionShape&, int, int h) const { return k_ + h * kv_head; }
+    __device__ __forceinline__ const float* v(const AttentionShape&, int, int h) const { return v_ + h * kv_head; }
+    __device__ __forceinline__ int64_t q_row(const AttentionShape&) const { return q_stride; }
+    __device__ __forceinline__ int64_t kv_row(const AttentionShape&) const { return kD; }
 };
 
 // Exact: exponentials by expf and the softmax's sum in double, as the GPT-2 engine's decode step has
 // them; otherwise the hardware exp2 and an f32 sum.
-template <bool Exact>
+template <bool Exact, class Views>
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float* __restrict__ out, float* __restrict__ lse,
-                                                                           HeadViews in, AttentionShape sh) {
+                                                                           Views in, AttentionShape sh) {
     __shared__ float tiles[kWaves * kTile];  // each wave's K, then V, tile of its current key block
     __shared__ float qtile[kTile];           // the query block
     typedef std::conditional_t<Exact, double, float> Sum;
@@ -257,18 +276,18 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
     const int qb = blocks - 1 - static_cast<int>(blockIdx.x / units);  // longest rows first, all heads interleaved
     const int b = bh / sh.heads, h = bh % sh.heads;
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 32, lh = lane / 32;
-    const float* __restrict__ q = in.q + b * in.q_batch + h * in.q_head;
-    const float* __restrict__ k = in.k + b * in.kv_batch + h * in.kv_head;
-    const float* __restrict__ v = in.v + b * in.kv_batch + h * in.kv_head;
+    const float* __restrict__ q = in.q(sh, b, h);
+    const float* __restrict__ k = in.k(sh, b, h);
+    const float* __restrict__ v = in.v(sh, b, h);
     float* tile = tiles + wave * kTile;
     const int query = qb * kBlock + li;
 
     // every load in flight together: the wave's quarter of the query block, its first K and V tiles
     v4f qpart[kPartVec], kload[kTileVec], vload[kTileVec];
-    part_load(qpart, q, qb * kBlock, sh.length, in.q_row, wave, lane);
+    part_load(qpart, q, qb * kBlock, sh.length, in.q_row(sh), wave, lane);
     if (wave <= qb) {
-        tile_load(kload, k, wave * kBlock, sh.length, in.kv_row, lane);
-        tile_load(vload, v, wave * kBlock, sh.length, in.kv_row, lane);
+        tile_load(kload, k, wave * kBlock, sh.length, in.kv_row(sh), lane);
+        tile_load(vload, v, wave * kBlock, sh.length, in.kv_row(sh), lane);
     }
     part_store(qtile, qpart, wave, lane);
     __syncthreads();
@@ -288,8 +307,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_kernel(float
         wave_sync();
         const bool more = kb + kWaves <= qb;
         if (more) {  // the next block's loads run while this block computes
-            tile_load(kload, k, j0 + kWaves * kBlock, sh.length, in.kv_row, lane);
-            tile_load(vload, v, j0 + kWaves * kBlock, sh.length, in.kv_row, lane);
+            tile_load(kload, k, j0 + kWaves * kBlock, sh.length, in.kv_row(sh), lane);
+            tile_load(vload, v, j0 + kWaves * kBlock, sh.length, in.kv_row(sh), lane);
         }
         v16f s = dot_rows(kreg, qreg);
         // scale, mask, block max of this query's scores (16 here, 16 in lane li + 32)
@@ -456,7 +475,7 @@ __device__ __forceinline__ bool scores_overflowed(const v16f& s) {
 }
 
 __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kernel(float* __restrict__ out, float* __restrict__ lse,
-                                                                                  HeadViews in, AttentionShape sh) {
+                                                                                  FusedViews in, AttentionShape sh) {
     __shared__ __attribute__((aligned(16))) char stages[2][kStage];
     __shared__ int bad[2];  // the last block (+ 1) of each stage that pieces cannot hold
     const int tiles = (sh.length + kWide - 1) / kWide;
@@ -465,9 +484,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
     const int q0 = (tiles - 1 - static_cast<int>(blockIdx.x / units)) * kWide;  // longest rows first, all heads interleaved
     const int b = bh / sh.heads, h = bh % sh.heads;
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, li = lane % 32, lh = lane / 32;
-    const float* __restrict__ q = in.q + b * in.q_batch + h * in.q_head;
-    const float* __restrict__ k = in.k + b * in.kv_batch + h * in.kv_head;
-    const float* __restrict__ v = in.v + b * in.kv_batch + h * in.kv_head;
+    const float* __restrict__ q = in.q(sh, b, h);
+    const float* __restrict__ k = in.k(sh, b, h);
+    const float* __restrict__ v = in.v(sh, b, h);
     const int query = q0 + wave * kBlock + li;
     const int blocks = min(q0 + kWide, sh.length - 1 + kBlock) / kBlock;  // of keys, up to the workgroup's last query
     const int last = q0 / kBlock + wave;                                  // this wave's last block
@@ -477,8 +496,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
     float kx[8], vx[8];
     const auto load = [&](int kb) {
         const int j0 = kb * kBlock;
-        const v4f a = row_piece(k, j0 + key, sh.length, in.kv_row, feature / 4);
-        const v4f c = row_piece(k, j0 + key, sh.length, in.kv_row, feature / 4 + 1);
+        const v4f a = row_piece(k, j0 + key, sh.length, in.kv_row(sh), feature / 4);
+        const v4f c = row_piece(k, j0 + key, sh.length, in.kv_row(sh), feature / 4 + 1);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             kx[e] = a[e];
@@ -487,7 +506,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int row = j0 + block_row(8 * (wave / 2) + e, wave % 2);
-            const float x = v[static_cast<int64_t>(min(row, sh.length - 1)) * in.kv_row + lane];
+            const float x = v[static_cast<int64_t>(min(row, sh.length - 1)) * in.kv_row(sh) + lane];
             vx[e] = row < sh.length ? x : 0.f;
         }
     };
@@ -502,7 +521,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
     load(0);
     bf8 qp[kD / 16][3];
     bool far = false;
-    const float* qrow = q + static_cast<int64_t>(min(query, sh.length - 1)) * in.q_row;
+    const float* qrow = q + static_cast<int64_t>(min(query, sh.length - 1)) * in.q_row(sh);
 #pragma unroll
     for (int s = 0; s < kD / 16; ++s) {
         const v4f a = *reinterpret_cast<const v4f*>(qrow + 16 * s + 8 * lh);
@@ -610,7 +629,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
 #pragma unroll 1
         for (int kb = 0; kb <= min(last, blocks - 1); ++kb) {
             const int j0 = kb * kBlock;
-            const float* krow = k + static_cast<int64_t>(min(j0 + li, sh.length - 1)) * in.kv_row;
+            const float* krow = k + static_cast<int64_t>(min(j0 + li, sh.length - 1)) * in.kv_row(sh);
             v16f s = piece_scores<false>(krow, lh, qp);
             float scale = sh.inv_scale * kUnscale;
             if (scores_overflowed(s)) {
@@ -641,7 +660,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attention_forward_pieces_kerne
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
                 const int row = j0 + block_row(t, lh);
-                const float* vrow = v + static_cast<int64_t>(min(row, sh.length - 1)) * in.kv_row + li;
+                const float* vrow = v + static_cast<int64_t>(min(row, sh.length - 1)) * in.kv_row(sh) + li;
                 o[0] = mfma(row < sh.length ? vrow[0] : 0.f, s[t], o[0]);
                 o[1] = mfma(row < sh.length ? vrow[32] : 0.f, s[t], o[1]);
             }
@@ -1121,18 +1140,10 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 int64_t wide_groups(const AttentionShape& sh) { return int64_t{sh.batch} * sh.heads * ((sh.length + kWide - 1) / kWide); }
 bool on_pieces(const AttentionShape& sh) { return sh.length > kBlock && wide_groups(sh) > compute_units(); }
 
-template <bool Exact> int launch_forward(float* out, float* lse, const HeadViews& in, const AttentionShape& sh) {
-    if constexpr (!Exact) {
-        if (on_pieces(sh)) {
-            hipLaunchKernelGGL(attention_forward_pieces_kernel, dim3(static_cast<uint32_t>(wide_groups(sh))), dim3(kWaves * 64), 0,
-                               stream(), out, lse, in, sh);
-            KD_LAUNCH_CHECK();
-            return KD_OK;
-        }
-    }
+template <bool Exact, class Views> int launch_forward(float* out, float* lse, const Views& in, const AttentionShape& sh) {
     const int64_t blocks = (sh.length + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(attention_forward_kernel<Exact>, dim3(static_cast<uint32_t>(sh.batch * sh.heads * blocks)), dim3(kWaves * 64),
-                       0, stream(), out, lse, in, sh);
+    hipLaunchKernelGGL((attention_forward_kernel<Exact, Views>), dim3(static_cast<uint32_t>(sh.batch * sh.heads * blocks)),
+                       dim3(kWaves * 64), 0, stream(), out, lse, in, sh);
     KD_LAUNCH_CHECK();
     return KD_OK;
 }
@@ -1143,7 +1154,7 @@ int causal_attention_heads(float* out, const float* q, int64_t q_row, const floa
                            int64_t length, int64_t heads) {
     AttentionShape sh;
     if (int rc = check_shape(KD_F32, 1, length, heads, kD, sh, "causal_attention_heads")) return rc;
-    return launch_forward<true>(out, nullptr, HeadViews{q, k, v, 0, kD, q_row, 0, kv_head, kD}, sh);
+    return launch_forward<true>(out, nullptr, HeadViews{q, k, v, q_row, kv_head}, sh);
 }
 
 } // namespace kd
@@ -1157,10 +1168,12 @@ extern "C" int kd_causal_attention(int dtype, void* out, void* lse, const void* 
     if (out == nullptr || qkv == nullptr || lse == nullptr || !aligned16(out) || !aligned16(qkv))
         return fail(KD_E_INVALID, "kd_causal_attention: out, lse and qkv must be given, out and qkv 16-byte aligned");
     if (int rc = ensure_device()) return rc;
-    const float* q = static_cast<const float*>(qkv);
-    const int64_t width = heads * kD, tokens = length * sh.row;
-    return launch_forward<false>(static_cast<float*>(out), static_cast<float*>(lse),
-                          HeadViews{q, q + width, q + 2 * width, tokens, kD, sh.row, tokens, kD, sh.row}, sh);
+    const FusedViews in{static_cast<const float*>(qkv)};
+    if (!on_pieces(sh)) return launch_forward<false>(static_cast<float*>(out), static_cast<float*>(lse), in, sh);
+    hipLaunchKernelGGL(attention_forward_pieces_kernel, dim3(static_cast<uint32_t>(wide_groups(sh))), dim3(kWaves * 64), 0,
+                       stream(), static_cast<float*>(out), static_cast<float*>(lse), in, sh);
+    KD_LAUNCH_CHECK();
+    return KD_OK;
 }
 
 extern "C" int kd_causal_attention_backward(int dtype, void* dqkv, const void* dout, const void* qkv, const void* out,
