@@ -35,7 +35,8 @@
 // chain starts from are sums of about 10^4 of them, taken by 16 workgroups a chain that each add
 // the words of a range of coefficients (exclusive or: any order gives the same); then a workgroup
 // per chain walks its own 64 blocks. 2^20 draws: 1.26 ms on one chain, 0.13 ms so, of which the three
-// kernels take 20, 50 (LDS reads: 17 MB a chain) and 39 us. At 300 blocks the two are even (0.10 ms).
+// kernels take 20, 50 (LDS reads: 17 MB a chain) and 39 us. At 300 blocks the two are even (0.10 ms). A process's
+// first such call also computes and copies the polynomials: 1.37 ms.
 #include "kd_mt_jump.h"
 
 #include <algorithm>
@@ -275,14 +276,20 @@ __global__ __launch_bounds__(kChainThreads) void chain_kernel(RngArgs a, T keep_
     else if (chain == kJumpChains - 1 && t < kWords) after[t] = mt[cur][t];
 }
 
-// The polynomials on the device, copied once (a first call per device; kd_dropout and kd_bernoulli block).
-int ensure_jump(const uint64_t* polynomials) {
+// At least `count` polynomials on the device (the backend has one device a process): each computed and copied once, by
+// the first call that draws as many chains (kd_dropout and kd_bernoulli block).
+int ensure_jump(int count) {
     static std::mutex mutex;
-    static bool ready = false;
+    static int ready = 0;
     std::lock_guard<std::mutex> lock(mutex);
-    if (ready) return KD_OK;
-    KD_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_jump), polynomials, sizeof g_jump, 0, hipMemcpyHostToDevice));
-    ready = true;
+    if (ready >= count) return KD_OK;
+    constexpr size_t kBytes = kWords * sizeof(uint64_t);
+    const uint64_t* polynomials = mt_jump_polynomials(count);
+    while (ready < count) {  // 10 KB at a time: a process's first copy of more than 16 KB takes 5 to 10 ms
+        const int n = std::min(count - ready, 4);
+        KD_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_jump), polynomials + ready * kWords, n * kBytes, ready * kBytes, hipMemcpyHostToDevice));
+        ready += n;
+    }
     return KD_OK;
 }
 
@@ -297,12 +304,12 @@ int run_rng(void* out, void* mask, const void* in, int64_t count, double p, uint
     a.first = std::min<int64_t>(kWords - pos, count);
     a.blocks = 1 + (count - a.first + kWords - 1) / kWords;
     a.p = p;
-    const uint64_t* polynomials = a.blocks > kSerialBlocks ? mt_jump_polynomials() : nullptr;
-    if (polynomials != nullptr)
-        if (int rc = ensure_jump(polynomials)) return rc;
+    const bool rounds = a.blocks > kSerialBlocks;
+    if (rounds)
+        if (int rc = ensure_jump(static_cast<int>((std::min(a.blocks, kRoundBlocks) + kJumpBlocks - 1) / kJumpBlocks) - 1)) return rc;
     // the state, the state after, then (for rounds) a round's words, its chains' starts, and its last words
     constexpr int64_t kRoundWords = int64_t{kJumpBlocks + 1} * kWords;
-    const int64_t words = 2 * (kWords + 1) + (polynomials != nullptr ? kRoundWords + int64_t{kJumpChains} * kWords : 0);
+    const int64_t words = 2 * (kWords + 1) + (rounds ? kRoundWords + int64_t{kJumpChains} * kWords : 0);
     Workspace lease;
     if (int rc = workspace(lease, static_cast<size_t>(words) * sizeof(uint64_t))) return rc;
     uint64_t* dev_state = static_cast<uint64_t*>(lease.ptr);
@@ -310,7 +317,7 @@ int run_rng(void* out, void* mask, const void* in, int64_t count, double p, uint
     a.next = dev_state + kWords + 1;
     hipStream_t s = stream();
     KD_HIP(hipMemcpyAsync(dev_state, host_state, (kWords + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, s));
-    if (polynomials != nullptr) {
+    if (rounds) {
         uint64_t* round_words = dev_state + 2 * (kWords + 1);
         uint64_t* starts = round_words + kRoundWords;
         uint64_t* after = starts + (kJumpChains - 1) * kWords;
