@@ -2031,7 +2031,9 @@ struct Engine {
     }
 
     // Prompts of at most kShortPrompt positions: the products split over K (at most one 64x64-tile
-    // workgroup per CU, or one whole product). (256: the same at 129 to 256 positions.)
+    // workgroup per CU, or one whole product). (256: the same at 129 to 256 positions.) The three lines are GPT-2
+    // small's; at 4 layers of widths 256, 384 and 1024 (heads of 64 and of 32), no prompt length of 1 to 1000 took
+    // longer than with every product whole and rows padded, but 129 and 400 positions at 256, by 3 to 5 %.
     static constexpr int64_t kShortPrompt = 128;
     // Up to so many, longer prompts leave their partials to the epilogue as well (129 positions 1.03 ms, 1.10
     // with a sum of its own); beyond, the epilogues, a workgroup per row, take longer over the partials

@@ -60,8 +60,8 @@ int workspace(Workspace& lease, size_t bytes);
 int matmul_split_parts(const float* a, const float* b, float* parts, int64_t M, int64_t N, int64_t K, int64_t lda,
                        int64_t ldb, int64_t splits);
 
-// The same for longer operands, on the tiles and splits that kd_matmul's main family would take, as far as
-// `capacity` floats hold the partials (at least M * N); *splits says how many there are.
+// The same for longer operands, on the tiles and splits that kd_matmul would take, as far as `capacity` floats
+// hold the partials (at least M * N); *splits says how many there are.
 int matmul_linear_parts(const float* a, const float* b, float* parts, int64_t capacity, int64_t M, int64_t N, int64_t K,
                         int64_t* splits);
 

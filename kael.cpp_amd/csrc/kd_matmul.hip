@@ -1126,6 +1126,16 @@ double small_us(const MatmulArgs& p) {
     return 2.2 + tiles * (2.3e-3 + 2.7e-5 * k) + batches * (1.8e-7 * k * (m * gn + n * gm) + 8.4e-7 * m * n);
 }
 
+int launch_small(const float* a, const float* b, float* out, const MatmulArgs& p) {
+    const dim3 grid(static_cast<uint32_t>((p.N + kSmallTile - 1) / kSmallTile), static_cast<uint32_t>((p.M + kSmallTile - 1) / kSmallTile),
+                    static_cast<uint32_t>(p.batches));
+    with_k_modes(p.sa.c == 1, p.sb.r == 1, [&](auto ak, auto bk) {
+        hipLaunchKernelGGL((small_kernel<decltype(ak)::value, decltype(bk)::value>), grid, dim3(kSmallWaves * 64), 0, stream(), a, b,
+                           out, p);
+    });
+    return launch_status();
+}
+
 int matmul_f32(const float* a, const float* b, float* out, MatmulArgs p) {
     enum { kRowdot, kSkinny, kSmall, kPieces, kGeneral };
     if (p.batches > kGridBatches && p.N > kRowdotMaxN) return fail(KD_E_INVALID, "kd_matmul: too many batches");
@@ -1185,14 +1195,7 @@ int matmul_f32(const float* a, const float* b, float* out, MatmulArgs p) {
         else launch(std::integral_constant<int, kSkinnyMaxM>{});
         return launch_status();
     }
-    case kSmall: {
-        const dim3 groups(static_cast<uint32_t>(gn), static_cast<uint32_t>(gm), static_cast<uint32_t>(p.batches));
-        with_k_modes(p.sa.c == 1, p.sb.r == 1, [&](auto ak, auto bk) {
-            hipLaunchKernelGGL((small_kernel<decltype(ak)::value, decltype(bk)::value>), groups, dim3(kSmallWaves * 64), 0,
-                               stream(), a, b, out, p);
-        });
-        return launch_status();
-    }
+    case kSmall: return launch_small(a, b, out, p);
     case kPieces: return matmul_pieces(a, b, out, p, plan);
     default: break;
     }
@@ -1408,6 +1411,11 @@ int matmul_linear_parts(const float* a, const float* b, float* parts, int64_t ca
     if (M <= 0 || N <= 0 || K <= 0 || capacity < M * N || !pieces_addressable(p))
         return fail(KD_E_INVALID, "matmul_linear_parts: operands outside the product's bounds");
     const Plan plan = plan_pieces(M, N, K, 1, capacity / (M * N));
+    const int64_t small_tiles = (M + kSmallTile - 1) / kSmallTile * ((N + kSmallTile - 1) / kSmallTile);
+    if (small_tiles <= 2 * int64_t{compute_units()} && small_us(p) < plan.us) {
+        *splits = 1;
+        return launch_small(a, b, parts, p);
+    }
     *splits = plan.splits;
     return launch_plan(plan, a, b, parts, p, M * N);
 }

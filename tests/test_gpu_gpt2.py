@@ -201,6 +201,37 @@ def test_small_model_batched_prefill(kdb, refdev, prompt_len):
         ref.ref_gpt_destroy(h)
 
 
+@pytest.mark.parametrize("width,heads", [(256, 4), (96, 3), (384, 6)])
+def test_batched_prefill_against_steps(kdb, width, heads):
+    """Prompts around the lengths where the products' and the attention's kernels change, against the same engine's token
+    by token prefill: the logits of the last position, at kael's device tolerance of 1e-4 (reference
+    tests/test_cuda.cpp:40-43) of logits of order 1, and the cache by one more token."""
+    vocab, positions = 300, 300
+    rng = np.random.default_rng(width)
+    weights = {}
+    for name, shape in kd.gpt2_parameter_shapes(vocab, positions, 2, width):
+        weights[name] = (np.full(shape, float(name.endswith("weight")), np.float32) if ".ln" in name or name.startswith("ln")
+                         else rng.normal(0, 0.05, shape).astype(np.float32))
+    engines = [kd.Gpt(kdb, vocab, positions, 2, heads, width, True, stepwise_prefill=s) for s in (False, True)]
+    for g in engines:
+        for name, w in weights.items():
+            g.load(name, w)
+    for length in (1, 31, 32, 33, 64, 65, 128, 129, 200, 256, 257, 299):
+        prompt = rng.integers(0, vocab, length)
+        logits = []
+        for g in engines:
+            g.prefill(prompt)
+            first = g.logits()
+            g.decode(1)
+            logits.append((first, g.logits()))
+        if engines[0].sequence()[length] != engines[1].sequence()[length]:  # (a tie within the tolerance)
+            top = np.sort(logits[1][0])[-2:]
+            assert top[1] - top[0] < 2e-4
+            logits = [l[:1] for l in logits]
+        for got, want in zip(*logits):
+            np.testing.assert_allclose(got, want, rtol=1e-4, atol=1e-4)
+
+
 def test_gpt2_small_batched_prefill(kdb, refdev):
     """Config C5 with prompts of 1, 64 and 100 positions (split-K partial products on 64-row
     tiles, one and two of them), 129, 300 (128-row tiles) and 600 positions (decode steps past
