@@ -137,12 +137,11 @@ def _strided_product(kdb, a_store, b_store, batches, m, k, n, sa, sb):
 
 @pytest.mark.parametrize("a_t,b_t", [(True, False), (False, True), (True, True)], ids=["aT", "bT", "both"])
 def test_transposed_whole_tiles_equal_row_major(kdb, a_t, b_t):
-    """A and/or B read in place through transposed views, whole 128x128 tiles and enough of them
-    to skip the small-product path (3 x 1024x256x1024): the product runs on the kernel that loads
-    a transposed operand as 4x4 blocks and writes them transposed into the same LDS tiles the
-    row-major kernel fills, with the same MFMA order, so it must equal bit for bit the row-major
-    product of the materialized operands (reference src/autograd/functions_linalg.cpp:37,44 and
-    src/nn/layers.cpp:43 issue X^T . g and x . W^T)."""
+    """A and/or B read in place through transposed views, whole tiles of every size and enough of
+    them to skip the small tiles (3 x 1024x256x1024): a transposed operand is loaded in another
+    order but makes the same LDS tiles of pieces, multiplied in the same order, so the product must
+    equal bit for bit the row-major product of the materialized operands (reference
+    src/autograd/functions_linalg.cpp:37,44 and src/nn/layers.cpp:43 issue X^T . g and x . W^T)."""
     batches, m, k, n = 3, 1024, 256, 1024
     rng = np.random.default_rng(44 + 2 * a_t + b_t)
     a = rng.uniform(-1, 1, (batches, m, k)).astype(np.float32)
@@ -160,7 +159,7 @@ def test_transposed_whole_tiles_equal_row_major(kdb, a_t, b_t):
 
 def test_weight_gradient_shape_of_c4(kdb):
     """C4's Linear weight gradient X^T . g with X [4096 tokens, 256] and g [4096, 768] read in
-    place (M 256, K 4096, N 768: whole tiles, K too long for the small-product path). At K = 4096
+    place (M 256, K 4096, N 768: whole tiles, K too long for the small tiles). At K = 4096
     an element's f32 error scales with its sum of |a||b|, so the check is the GPT-2 logits rule:
     within 1e-4 of the largest |element| of the float64 product."""
     m, k, n = 256, 4096, 768
@@ -176,8 +175,8 @@ def test_weight_gradient_shape_of_c4(kdb):
                          ids=["proj-WT", "fc2-WT", "fc2-W", "flat-WT"])
 def test_linear_forward_shapes_of_c4(kdb, batches, k, b_t):
     """kael's Linear forward x . W^T at C4's narrow outputs (x [32, 128, K], W [256, K] shared by
-    every batch item, reference src/nn/layers.cpp:43): 64 output tiles, so the batch folds into M
-    and K is split over the device, the partial products added in split order. Checked against the
+    every batch item, reference src/nn/layers.cpp:43): the batch folds into M, and where few tiles
+    are left K is split over the device, the partial products added in split order. Checked against the
     float64 product within 1e-4 of its largest |element| (the GPT-2 logits rule), and run twice to
     check that the result is deterministic."""
     m, n = 128 * 32 // batches, 256
@@ -194,10 +193,10 @@ def test_linear_forward_shapes_of_c4(kdb, batches, k, b_t):
 
 
 def test_64_tiles_equal_128_tiles(kdb):
-    """3 batches of 1024 x 256 x 1024 have 192 128x128 tiles, fewer than the 256 CUs, and run on
-    64x64 tiles; 4 batches have 256 and stay on 128x128 tiles. Each batch item's product is the same
-    computation either way: the same (k, k + 4) MFMA pairs in the same K order, so the first three
-    items must agree bit for bit."""
+    """3 and 4 batches of 1024 x 256 x 1024, which may take tiles of different sizes and K steps (192
+    and 256 tiles of 128x128 on 256 CUs): each batch item's product is the same computation on every
+    tiling, the same pieces multiplied in the same K order, so the first three items must agree bit
+    for bit."""
     m, k, n = 1024, 256, 1024
     rng = np.random.default_rng(51)
     a = rng.uniform(-1, 1, (4, m, k)).astype(np.float32)
@@ -218,8 +217,8 @@ ATTENTION = [(128, 128, 128, 64), (128, 128, 64, 128), (128, 64, 128, 128), (8, 
 @pytest.mark.parametrize("batches,m,k,n", ATTENTION, ids=[f"{b}x{m}x{k}x{n}" for b, m, k, n in ATTENTION])
 def test_attention_shaped_batches(kdb, batches, m, k, n):
     """The batched products of C4's attention (32 x 4 heads: Q.K^T with K = head_dim 64, P.V with
-    N = 64, and their gradients, reference src/nn/transformer.cpp:103-139) on 64x64 tiles, and the
-    smallest whole case (64 x 32 x 64)."""
+    N = 64, and their gradients, reference src/nn/transformer.cpp:103-139), and the smallest with
+    whole 64x64 tiles (64 x 32 x 64)."""
     rng = np.random.default_rng(52 + m + k + n)
     a = rng.uniform(-1, 1, (batches, m, k)).astype(np.float32)
     b = rng.uniform(-1, 1, (batches, k, n)).astype(np.float32)
@@ -231,10 +230,9 @@ def test_attention_shaped_batches(kdb, batches, m, k, n):
 @pytest.mark.parametrize("a_t,b_t", [(False, False), (True, False), (False, True), (True, True)],
                          ids=["rows", "aT", "bT", "both"])
 def test_64_tiles_with_transposed_operands(kdb, a_t, b_t):
-    """M and N multiples of 64 but not of 128 (192 x 96 x 320, 4 batches), every operand layout:
-    the 64x64 kernel's loaders (coalesced along each stored operand's contiguous dim, A^T written
-    transposed into a swizzled tile) against the float64 product; all four layouts equal bit for
-    bit (the same tiles, MFMA pairs and order)."""
+    """M and N multiples of 64 but not of 128 (192 x 96 x 320, 4 batches), every operand layout, each
+    read along its contiguous dimension, against the float64 product; all four layouts equal bit
+    for bit (the same tiles, products and order)."""
     batches, m, k, n = 4, 192, 96, 320
     rng = np.random.default_rng(53)
     a = rng.uniform(-1, 1, (batches, m, k)).astype(np.float32)
@@ -251,7 +249,7 @@ def test_64_tiles_with_transposed_operands(kdb, a_t, b_t):
 
 def test_split_k_on_64_tiles(kdb):
     """C4's narrowest weight gradient X^T . g (M = N = 256, K = 4096: 16 tiles of 64x64) splits K
-    16 ways over the device and adds the partial products in split order: within 1e-4 of the
+    over the device and adds the partial products in split order: within 1e-4 of the
     largest |element| of the float64 product, and the same bits on a second run."""
     m, k, n = 256, 4096, 256
     rng = np.random.default_rng(54)
@@ -266,7 +264,7 @@ def test_split_k_on_64_tiles(kdb):
 
 @pytest.mark.parametrize("m, k, n, sa, sb", [
     (96, 4096, 256, (0, 1, 96), (0, 256, 1)),       # kael's tied LM-head weight gradient (A read transposed)
-    (100, 1024, 128, (0, 1024, 1), (0, 128, 1)),    # ragged M on 64x64 tiles, A row-major
+    (100, 1024, 128, (0, 1024, 1), (0, 128, 1)),    # ragged M, A row-major
     (36, 2048, 64, (0, 1, 36), (0, 64, 1)),         # one ragged tile row, A read transposed
     (68, 96, 192, (0, 96, 1), (0, 1, 96)),          # ragged M, short K (no split), B read transposed
     (130, 3072, 70, (0, 3072, 1), (0, 1, 3072)),    # ragged M and N, B read transposed
@@ -274,11 +272,10 @@ def test_split_k_on_64_tiles(kdb):
 ], ids=["head_96x4096x256", "ragged_100x1024x128", "ragged_36x2048x64", "ragged_68x96x192", "ragged_130x3072x70",
         "generic_33x2560x200"])
 def test_split_k_on_ragged_tiles(kdb, m, k, n, sa, sb):
-    """Few ragged tiles with a long K: K split over the device (the splits in the kernel's batch
-    slot; 64x64 tiles whose last tile row loads zeros past M and stores only rows below it when M
-    is a multiple of 4 and N of 64, else the general kernel) and split_sum_kernel adding the
-    partials in split order: within 1e-4 of the largest |element| of the float64 product, and the
-    same bits on a second run."""
+    """Few ragged tiles with a long K: K split over the device (the last tile row and column repeat
+    the last element's operands and store nothing past it) and the partials added in split order, or
+    the small tiles, which split K over a workgroup's waves: within 1e-4 of the largest |element| of
+    the float64 product, and the same bits on a second run."""
     rng = np.random.default_rng(m + k + n)
 
     def extent(shape, st):
@@ -296,14 +293,14 @@ def test_split_k_on_ragged_tiles(kdb, m, k, n, sa, sb):
 
 
 def test_headline_4096_cubed(kdb, refdev, oracle):
-    """The benchmark's headline product (row-major MFMA kernel, whole tiles) at its full size,
-    inputs as bench.py draws them. At K = 4096 an element's f32 rounding error scales with its
-    dot product's sum of |a||b| (~1024 here), not with the element itself, so elements near
+    """The benchmark's headline product (256x128 tiles of pieces) at its full size, inputs as
+    bench.py draws them. At K = 4096 an element's f32 rounding error scales with its dot product's sum of |a||b| (~1024 here), not with the element itself, so elements near
     zero miss the small-shape rule 1e-4 + 1e-4 |y| by a few ulps of that sum in any f32
     product. Checks: within 1e-4 of the largest |element| of the float64 product (the rule of
     the GPT-2 logits), and within 8x the worst error of kael's own f32 CPU product of the same
-    inputs (reference matmul_versions v6). Measured: device worst 3.6e-4 (one running f32 MFMA
-    sum over K), kael CPU 6.6e-5 (its K blocking shortens the running sums), scale ~1e2."""
+    inputs (reference matmul_versions v6). Measured on the f32 matrix cores: device worst 3.6e-4
+    (one running f32 MFMA sum over K; on pieces two thirds of the 2-norm), kael CPU 6.6e-5 (its K
+    blocking shortens the running sums), scale ~1e2."""
     rng = np.random.default_rng(0)
     a = rng.uniform(-1, 1, (4096, 4096)).astype(np.float32)
     b = rng.uniform(-1, 1, (4096, 4096)).astype(np.float32)
@@ -320,7 +317,7 @@ def test_headline_4096_cubed(kdb, refdev, oracle):
     assert err.max() <= 1e-4 * np.abs(want).max(), f"worst {err.max()} vs scale {np.abs(want).max()}"
     assert err.max() <= 8 * err_cpu.max(), f"device worst {err.max()}, kael CPU worst {err_cpu.max()}"
     # The reference's device kernel (src/cuda/kernels.inl:136-177) keeps one running f32 sum per
-    # element over k = 0 .. K-1, as this backend's MFMA accumulators do: on 64 sampled rows the
+    # element over k = 0 .. K-1, as each of this backend's accumulators does: on 64 sampled rows the
     # device's error must not exceed that order's (the oracle's restatement) by more than 1.5x.
     rows = np.random.default_rng(1).choice(4096, 64, replace=False)
     a_rows = np.ascontiguousarray(a[rows])
@@ -338,8 +335,8 @@ def test_headline_4096_cubed(kdb, refdev, oracle):
 
 @pytest.mark.parametrize("batches,m,k,n", [(2, 384, 256, 512), (3, 128, 1024, 128)])
 def test_batched_whole_tiles_with_split_k(kdb, batches, m, k, n):
-    """Batched row-major products with few tiles: the row-major kernel splits K and sums the
-    partials per batch."""
+    """Batched row-major products with few tiles: K may be split, with the partials summed per
+    batch."""
     rng = np.random.default_rng(m + k + n)
     a = rng.uniform(-1, 1, (batches, m, k)).astype(np.float32)
     b = rng.uniform(-1, 1, (batches, k, n)).astype(np.float32)
@@ -501,15 +498,15 @@ def test_two_level_batches_reject_bad_heads(kdb):
 
 
 BIAS_CASES = [  # batches, m, k, n, a strides, b strides: kael's x . W^T shapes and every kernel family
-    (32, 128, 256, 768, (128 * 256, 256, 1), (0, 1, 256)),      # t64 folded (C4 qkv)
-    (32, 128, 256, 1024, (128 * 256, 256, 1), (0, 1, 256)),     # 128x128 transposed-B kernel (C4 fc1)
+    (32, 128, 256, 768, (128 * 256, 256, 1), (0, 1, 256)),      # the batch folded into M (C4 qkv)
+    (32, 128, 256, 1024, (128 * 256, 256, 1), (0, 1, 256)),     # the batch folded into M (C4 fc1)
     (1, 4096, 4096, 256, (0, 4096, 1), (0, 1, 4096)),           # split K
-    (1, 512, 512, 512, (0, 512, 1), (0, 512, 1)),               # row-major whole tiles / small kernel
-    (1, 3, 768, 2304, (0, 768, 1), (0, 1, 768)),                # skinny (decode-shaped)
+    (1, 512, 512, 512, (0, 512, 1), (0, 512, 1)),               # small tiles
+    (1, 3, 768, 2304, (0, 768, 1), (0, 1, 768)),                # three rows (decode-shaped)
     (1, 64, 784, 128, (0, 784, 1), (0, 1, 784)),                # C3's first Linear
     (2, 33, 17, 3, (17 * 33, 17, 1), (0, 1, 17)),               # row-dot
-    (2, 130, 70, 200, (130 * 70, 70, 1), (0, 1, 70)),           # ragged tiles, general kernel
-    (1, 96, 4096, 256, (0, 1, 96), (0, 256, 1)),                # ragged tiles, general kernel split K
+    (2, 130, 70, 200, (130 * 70, 70, 1), (0, 1, 70)),           # ragged tiles in batches
+    (1, 96, 4096, 256, (0, 1, 96), (0, 256, 1)),                # ragged tiles, split K or small tiles
 ]
 
 

@@ -114,8 +114,8 @@ def test_infinities_and_nan_as_an_f32_product_has_them(kdb, k):
 
 @pytest.mark.parametrize("case", ["steps", "broadcast", "reversed", "output", "unaligned"])
 def test_strides_that_are_no_plain_matrix(kdb, case):
-    """Both strides of an operand above 1, rows that repeat, negative strides (the general kernel), an
-    output of strided columns, and operands that start and step at odd elements."""
+    """Both strides of an operand above 1, rows that repeat, negative strides, an output of strided columns, and
+    operands that start and step at odd elements."""
     rng = np.random.default_rng(11)
     m, k, n = 150, 900, 140
     store = rng.normal(size=2_000_000).astype(np.float32)
@@ -141,6 +141,30 @@ def test_strides_that_are_no_plain_matrix(kdb, case):
         assert (got.reshape(m, n, 3)[:, :, 1:] == 0).all()
         got = got.reshape(m, n, 3)[:, :, 0]
     check(got, store[index], b)
+
+
+@pytest.mark.parametrize("heads,bias", [(0, False), (0, True), (3, False)])
+@pytest.mark.parametrize("m,k,n", [(700, 37, 900), (129, 16, 300), (260, 5, 385)], ids=str)
+def test_strides_that_only_the_general_kernel_takes(kdb, m, k, n, heads, bias):
+    """Both operands backwards (negative strides, which the pieces' loads do not address) in more than two small tiles a
+    CU: one batch level, two levels of heads, with and without the bias."""
+    rng = np.random.default_rng(m + heads)
+    batches = 12
+    a, b = rng.normal(size=(batches, m, k)).astype(np.float32), rng.normal(size=(batches, k, n)).astype(np.float32)
+    add = rng.normal(size=n).astype(np.float32) if bias else None
+    da, db, out = kdb.to_device(a), kdb.to_device(b), kdb.empty((batches, m, n), np.float32)
+    # the last element of each first matrix, from where rows and columns run backwards
+    pa, pb = ctypes.c_void_p(da.ptr + 4 * (m * k - 1)), ctypes.c_void_p(db.ptr + 4 * (k * n - 1))
+    outer = heads or 1
+    strides = kd.MatmulStrides((outer * m * k, -k, -1), (outer * k * n, -n, -1), (outer * m * n, n, 1))
+    args = (kd.F32, pa, pb, out.ptr, kd.MatmulSizes(batches, m, k, n), strides)
+    if heads:
+        kdb.call("matmul_strided_heads", *args, kd.MatmulHeads(heads, m * k, k * n, m * n))
+    elif bias:
+        kdb.call("matmul_strided_bias", *args, kdb.to_device(add).ptr)
+    else:
+        kdb.call("matmul_strided", *args)
+    check(out.numpy(), a[:, ::-1, ::-1], b[:, ::-1, ::-1], add)
 
 
 def test_split_batches_of_heads(kdb):
