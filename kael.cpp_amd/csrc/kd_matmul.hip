@@ -296,13 +296,14 @@ __global__ __launch_bounds__(WM * WN * 64, Occ) void pieces_kernel(const float* 
             }
         }
     };
-    // The end of a step in which the next stage was also split and stored: its VALU work between the
-    // MFMAs, six operations after each (999 x 768 x 3072: 34.4 us; four 37.5).
+    // The end of a step in which the next stage was also split and stored: its VALU work, 52 operations a unit,
+    // spread over the MFMAs (999 x 768 x 3072: 34 us; four after each 37.5).
+    constexpr int kProducts = IM * JN * 6 * (BK / 16);
     const auto mix = [&]() {
 #pragma unroll
-        for (int q = 0; q < IM * JN * 6 * (BK / 16); ++q) {
+        for (int q = 0; q < kProducts; ++q) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, (52 * kPer + kProducts - 1) / kProducts, 0);
         }
         __syncthreads();
     };
