@@ -38,12 +38,15 @@ import kd  # noqa: E402
 
 FP32_MFMA_PEAK_TFLOPS = 157.3   # MI355X dense FP32 matrix (AMD spec)
 FP64_MFMA_PEAK_TFLOPS = 78.6    # MI355X dense FP64 matrix (AMD spec)
+BF16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense BF16 matrix
+# what bounds the headline kernel: an f32 product is six bf16 products there
+PIECES_PEAK_TFLOPS = BF16_MFMA_PEAK_TFLOPS / 6
 HBM_PEAK_GBPS = 8000.0          # MI355X HBM3E
 # HBM bytes one 4096^3 launch of the headline kernel (pieces_kernel on 256 x 128 tiles) moves,
-# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (327 823 KiB and 65 536 KiB per dispatch), scaled
+# from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (327 830 KiB and 65 536 KiB per dispatch), scaled
 # by the factors a plain 256 MiB copy gives the same counters (x2.0 fetch, x1.0 write). The PMC
 # runs and commands are kept in profiles/.
-MATMUL_4096_TRAFFIC_BYTES = (2 * 327823 + 65536) * 1024
+MATMUL_4096_TRAFFIC_BYTES = (2 * 327830 + 65536) * 1024
 
 
 class Timer:
@@ -339,7 +342,8 @@ def bench_reference_device(backend, steps, warmup):
                                                             state.ctypes.data_as(ctypes.c_void_p)), "kd_dropout")
     sync_s = synced_call_s(backend, drop, iters)
     out["dropout_c4"] = {"elements": n, "synced_us": sync_s * 1e6, "synced_items_per_s": n / sync_s,
-                         "note": "one launch: mt19937_64 draws, compare, x * mask / keep, mask stored; "
+                         "note": "rounds of three launches (first words, jumps, chains): mt19937_64 draws, "
+                                 "compare, x * mask / keep, mask stored; "
                                  "the generator state copied in and back"}
     return out
 
@@ -773,6 +777,9 @@ def main() -> int:
                    "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP32_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
+                     # the kernel runs on the bf16 matrix cores, so this is the share of its own ceiling
+                     "peak_as_six_bf16_products": round(PIECES_PEAK_TFLOPS, 1),
+                     "frac_of_six_bf16_products": round(achieved / PIECES_PEAK_TFLOPS, 4),
                      "traffic": MATMUL_4096_TRAFFIC_BYTES if n == 4096 else None},
         "cpu_baseline": cpu,
         "extra": extra,

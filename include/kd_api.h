@@ -250,7 +250,7 @@ int kd_bernoulli(int dtype, void* out, int64_t count, double probability, uint64
 
 /* reference src/nn/functional.cpp:32-39 `dropout(input, p, training)` with keep = 1 - p: out[i] =
  * (in[i] * m[i]) / T(keep), m as kd_bernoulli(dtype, ..., keep) draws it and each op rounded to
- * the element type, in one launch; `mask` (may be NULL) receives m, which the backward pass
+ * the element type, in the pass that draws; `mask` (may be NULL) receives m, which the backward pass
  * needs. f32 or f64, contiguous `count` elements; keep in (0, 1]; out may equal in. */
 int kd_dropout(int dtype, void* out, void* mask, const void* in, int64_t count, double keep, uint64_t* state);
 
