@@ -1,7 +1,7 @@
 """Benchmark of the MI355X kael backend; prints ONE JSON line.
 
-Headline (BASELINE.json metric): f32 matmul TFLOP/s as a fraction of FP32 MFMA peak, on the
-north-star size 4096^3 (C = A.B, A and B contiguous row-major, uniform[-1,1]); a "step" is one
+Headline: f32 matmul TFLOP/s, as a fraction of FP32 MFMA peak and of six bf16 products, at
+4096^3 (C = A.B, A and B contiguous row-major, uniform[-1,1]); a "step" is one
 kd_matmul call over inputs already resident in HBM. Secondary figures in "extra": the C1 shape
 (512^3), the C2 elementwise/reduction ops in GB/s, the fused row kernels, the index and
 optimizer kernels at GPT-2-small scale, a C3 and a C4 training step (replayed from the recorded
